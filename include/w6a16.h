@@ -46,12 +46,13 @@ typedef struct w6a16_args {
     int64_t scales_batch_stride;       /* elements */
     void *out;                         /* [B][M][N] bf16, fp16 or fp32 (out_dtype) */
     int64_t out_batch_stride, out_row_stride;      /* elements */
-    void *workspace;                   /* split_k > 1 or M > 32: w6a16_workspace_size bytes, 256-byte aligned */
+    void *workspace;                   /* split_k > 1 or M > 32: w6a16_workspace_size bytes (unless 0), 256-byte aligned */
     size_t workspace_bytes;
     int32_t B, M, N, K;                /* K % 64 == 0, N % 16 == 0; M <= 32: B * ceil(M / 16) <= 65535,
                                           M > 32: B <= 65535 */
     int32_t group_k;                   /* % 64 == 0, divides K */
-    int32_t split_k;                   /* 1 .. 256: K is cut into split_k ranges of 64-row chunks */
+    int32_t split_k;                   /* 1 .. 256: bounds how many workgroups may share a tile's K (it sizes the
+                                          workspace their partial tiles go through); see w6a16_matmul */
     int32_t out_dtype;                 /* W6A16_OUT_BF16, W6A16_OUT_F16 or W6A16_OUT_F32 */
     int32_t format;                    /* W6A16_FORMAT_PLANES or W6A16_FORMAT_PACKED */
     int32_t a_dtype;                   /* W6A16_IN_BF16 (0) or W6A16_IN_F16 */
@@ -60,16 +61,16 @@ typedef struct w6a16_args {
 /* sizeof(w6a16_args) as compiled into the library (bindings check their struct layout against it). */
 size_t w6a16_args_size(void);
 
-/* Bytes of workspace `w6a16_matmul` needs (0 for split_k == 1 and M <= 32, for W6A16_FORMAT_PACKED with M > 256 (the
- * large-M kernel), and for M <= 32 with split_k 2..8 where the
- * in-workgroup split-K kernel runs: always for W6A16_FORMAT_PACKED, and for the planes when B * ceil(M / 16) *
- * ceil(N / 128) reaches the device's CU count; that kernel sums its split_k partial tiles in LDS): a fixed 1 MiB region of u32 arrival
- * counters (one per output tile; a call with more than 262144 tiles is refused with WKV7_ERR_SHAPE), then fp32
- * partial tiles (split_k > 1), then, for M > 32, the per-row sums of A that a small first launch computes and the
- * GEMM kernel reads.  The split that completes a tile last reduces it inside the kernel.  Contract: the counter
- * region (the first 1 MiB) must be zero before the workspace's first use; every completed call leaves it zero again
- * and never writes partials into it, so one workspace serves any number of calls of any shapes issued one after
- * another (stream order).  Calls that can run at the same time (different streams) need different workspaces. */
+/* Bytes of workspace `w6a16_matmul` needs: 0 for split_k == 1 and M <= 32, for W6A16_FORMAT_PACKED with M > 256 (the
+ * large-M kernel), and for M <= 32 with split_k 2..8 always for W6A16_FORMAT_PACKED and for the planes when
+ * B * ceil(M / 16) * ceil(N / 128) reaches the device's CU count; otherwise a fixed 1 MiB region of u32 arrival counters
+ * (a call whose B * ceil(M / rows) * ceil(N / 128), rows 16 up to M = 32, 32 up to 64, 64 above, exceeds 262144 with
+ * split_k > 1 is refused with WKV7_ERR_SHAPE), then room for split_k fp32 partial tiles (split_k > 1), then, for M > 32, a
+ * float per row and chain of two 64-row chunks.  The kernel uses the counters and as many partial tiles as it splits K
+ * over workgroups, the workgroup that completes a tile last sums it.  Contract: the counter region (the first 1 MiB)
+ * must be zero before the workspace's first use; every completed call leaves it zero again and never writes partials
+ * into it, so one workspace serves any number of calls of any shapes issued one after another (stream order).  Calls
+ * that can run at the same time (different streams) need different workspaces. */
 int w6a16_workspace_size(const w6a16_args *args, size_t *bytes);
 
 /* Split-K for a shape: the smallest power of two (<= 64, every range keeping at least one 64-row chunk) that gives
@@ -77,13 +78,15 @@ int w6a16_workspace_size(const w6a16_args *args, size_t *bytes);
  * within two workgroups per CU.  Replaces the split-K rule of plan_int6 (rwkv_next/kernels/int6_gemm.py:239-250). */
 int w6a16_plan_split(int32_t B, int32_t M, int32_t N, int32_t K);
 
-/* split_k for the packed layout (W6A16_FORMAT_PACKED), whose in-workgroup kernel prefers a shallower split where it
- * runs half strips; otherwise equal to w6a16_plan_split.  No counterpart in the reference (its weights come only as
- * planes); for callers that pass packed weights.  Results depend on split_k: a packed call gives the planes' bits
- * only at the same split_k. */
+/* split_k for the packed layout (W6A16_FORMAT_PACKED): 4 instead of 8 where B * ceil(M / 16) * ceil(N / 128) stays below
+ * the CU count and a range keeps 8 chunks; otherwise equal to w6a16_plan_split.  No counterpart in the reference (its
+ * weights come only as planes); for callers that pass packed weights.  Results may depend on split_k: a packed call is
+ * sure to give the planes' bits only at the same split_k. */
 int w6a16_plan_split_packed(int32_t B, int32_t M, int32_t N, int32_t K);
 
 /* C = A @ dequant(W) on `stream` (hipStream_t).  Replaces `_impl` + `_w6a16` (int6_gemm.py:253-287, 156-215).
+ * The summation order (which wavefronts share K, and in how many parts) follows from B, M, N, K and split_k, the same for
+ * both formats; equal calls give equal bits.
  * W6A16_FORMAT_PACKED with M > 256 runs the large-M kernel: A times the weight dequantised to A's type (s q rounded
  * once, the values w6a16_dequantize writes), fp32 accumulation, no workspace; split_k is not used there. */
 int w6a16_matmul(const w6a16_args *args, void *stream);

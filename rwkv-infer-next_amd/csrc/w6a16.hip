@@ -8,27 +8,18 @@
 //                       | (u[.. + j + 48] >> 4) << 6                                                 j < 16
 // C[b][m][n] = sum_k A[b][m][k] s[k / group_k][n] q[k][n] with fp32 accumulation (int6_gemm.py:156-215).
 //
-// Narrow kernel (M <= 32, the decode GEMV): a workgroup of four wavefronts covers four adjacent 128-column strips
-// (512 columns: neighbouring strips share DRAM pages, which the four wavefronts read at about the same time) for one
-// range of 64-row chunks (split-K over chunk ranges) and one 16-row tile of A.  Each wavefront computes a 16 (M) x
-// 128 (N) tile:
-//   * the chunk's 48 plane rows x 128 columns (6 KB) are loaded coalesced (16 bytes per lane, 8 lanes per row), with
-//     the next chunk's loads in flight, and written to the wave's own LDS buffer (no workgroup barrier: a wave's LDS
-//     operations execute in order);
-//   * ds_read_b64_tr_b8 hands each lane 8 consecutive plane rows of one column -- within each 16-lane group, lane
-//     L receives byte L & 7 of the 8-byte reads of lanes (L & 15) / 8 + 2 e, so lane s of group q reading
-//     row base + s / 2, columns 8 (s & 1) .. gives lane (i, q) rows base + e of column i -- which is exactly the
-//     B operand of v_mfma_f32_16x16x32_bf16 (8 consecutive k of one column).  One read of the lo plane covers both
-//     32-row halves of the chunk (low and high nibbles), one read of the hi plane supplies the top 2 bits;
-//   * the 6-bit code u becomes a bf16 operand without conversion instructions: 0x4300 | u is the bf16 of 128 + u,
-//     exact, assembled for two values with one v_perm_b32 against a register of 0x43 bytes.  One extra MFMA pair
-//     per chunk against a constant B of -160 removes the bias (128 + u - 160 = q) exactly;
-//   * each chunk's fp32 tile is scaled by s (fp16) and accumulated.
-// Split-K partials are reduced inside the kernel: every split stores its tile (fp32) and the workgroup increments its
-// tiles' arrival counters after one agent-scope release; the split that arrives last sums the partials in split
-// order (a fixed order: the result does not depend on which split arrives last), stores the result and resets the
-// counter to zero.  The wide kernel (M > 32) is described where it is defined.
-// Rows m >= M and columns n >= N are clamped on load (they only feed outputs that are not stored).
+// Tile kernel (decode-sized M; every M on the planes): a workgroup of W wavefronts computes 16 MT rows x 16 NT columns,
+// the wavefronts taking the 64-row chunks of K in turn, each on its own:
+//   * weights are loaded straight into registers in the order the matrix instruction takes them (packed layout) or four
+//     columns of eight rows a lane (planes) and become B operands of v_mfma_f32_16x16x32 without conversion
+//     instructions: 0x4300 | u is the bf16 of 128 + u, exact, assembled for two values with one v_perm_b32.  One MFMA
+//     pair per chunk and M tile against a constant B of -160 removes the bias (128 + u - 160 = q) exactly;
+//   * the chunk's rows of A are loaded coalesced (128 bytes a row) and turned into A operands through the wavefront's own
+//     LDS buffer;
+//   * each chunk's fp32 tile is scaled by s (fp16) and accumulated; the wavefronts' tiles are summed through LDS, and
+//     the tiles of several workgroups, where K is split over them, through the workspace, both in a fixed order.
+// Large-M kernel (packed weights): described where it is defined.
+// Rows m >= M read zeros and columns n >= N are clamped on load (they only feed outputs that are not stored).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -45,16 +36,9 @@ namespace {
 typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
 typedef float f4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u4 __attribute__((ext_vector_type(4)));
-typedef int v2i __attribute__((ext_vector_type(2)));
-typedef __attribute__((address_space(3))) v2i lds_v2i;
 
-constexpr int kTileN = 128;          // columns per wavefront
-constexpr int kTiles = kTileN / 16;  // 16x16 MFMA tiles per wavefront and M tile
-constexpr int kStrips = 4;           // adjacent 128-column strips per workgroup
-constexpr int kPitch = 136;          // LDS row pitch in bytes (128 + 8: the 8 rows of one transposing read differ in bank)
-constexpr int kRows = 48;            // plane rows per chunk: 32 lo + 16 hi
-constexpr int kScaleOff = kRows * kPitch;    // the chunk's 128 fp16 scales follow the plane rows
-constexpr int kBuf = kScaleOff + 2 * kTileN;
+constexpr int kTileN = 128;          // columns per strip of the packed layout
+constexpr int kTiles = kTileN / 16;  // 16-column tiles per strip
 constexpr int kCounterAlign = 256;   // bytes: workspace alignment
 // The arrival counters occupy a fixed region at the start of the workspace, the partials follow it.  Calls with
 // different tile counts can share one workspace: the partials of one call never overlap the counters of another,
@@ -70,11 +54,14 @@ struct Args {
     int64_t ss_b;
     void* out;
     int64_t so_b, so_m;
-    uint32_t* cnt;  // split_k > 1: arrival counters, one per (batch, M group, column strip); zero between calls
-    float* part;    // split_k > 1: partial tiles [tile][split][16 MT rows][128 columns]
-    float* rsum;    // wide kernel: row-sum bias per chain of 64 CG k, [batch][chain][mpad]
-    int32_t B, M, N, K, group_k, split_k, out_dtype, m_groups, n_strips, chunks_per_split;
-    int32_t mpad, chain_k, nchains, chains_per_split;  // wide kernel
+    uint32_t* cnt;  // K split over workgroups: arrival counters, one per tile; zero between calls
+    float* part;    // K split over workgroups: partial tiles [tile][split][rows][16 NT columns]
+    int32_t B, M, N, K, group_k, out_dtype, n_strips;
+    // tile kernel: M groups of 16 MT rows, wavefronts that share K, chunks of the longest share, scale groups, log2 of
+    // the workgroups (per M group) of an XCD unit
+    int32_t m_groups, parts, per_part, groups, unit_shift;
+    uint32_t gmul, gone;  // chunk c's scale group is (c gmul >> 32) + c gone
+    uint32_t mgmul;       // x / m_groups is x mgmul >> 31
     int32_t out_vec;  // large-M kernel: the output takes 8-byte (16-byte for fp32) stores of 4 adjacent columns
 };
 
@@ -83,8 +70,6 @@ __device__ __forceinline__ float h2f(uint16_t h) { return (float)__builtin_bit_c
 __device__ __forceinline__ f4 mfma(bf8 a, bf8 b, f4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
 
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
-typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
 
 // Activation element types.  The 6-bit code u becomes an exact MFMA operand 2^e + u with no conversion instruction
 // (the code byte beside a constant high byte), and one MFMA pair per chunk against the constant -(2^e + 32) takes the
@@ -94,23 +79,13 @@ typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
 struct ActBF16 {
     static constexpr uint32_t kCodeHi = 0x43434343u;
     static constexpr uint32_t kBias = 0xC320C320u;  // (-160, -160)
-    static constexpr uint32_t kOnes = 0x3F803F80u;  // (1, 1)
-    static constexpr float kOffset = 160.f;
     __device__ static f4 mma(u4 a, u4 b, f4 c) { return mfma(__builtin_bit_cast(bf8, a), __builtin_bit_cast(bf8, b), c); }
-    __device__ static float dot2(uint32_t a, uint32_t b, float c) {
-        return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf2, a), __builtin_bit_cast(bf2, b), c, false);
-    }
 };
 struct ActF16 {
     static constexpr uint32_t kCodeHi = 0x64646464u;
     static constexpr uint32_t kBias = 0xE420E420u;  // (-1056, -1056)
-    static constexpr uint32_t kOnes = 0x3C003C00u;  // (1, 1)
-    static constexpr float kOffset = 1056.f;
     __device__ static f4 mma(u4 a, u4 b, f4 c) {
         return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, a), __builtin_bit_cast(h8, b), c, 0, 0, 0);
-    }
-    __device__ static float dot2(uint32_t a, uint32_t b, float c) {
-        return __builtin_amdgcn_fdot2(__builtin_bit_cast(h2, a), __builtin_bit_cast(h2, b), c, false);
     }
 };
 
@@ -174,210 +149,6 @@ __device__ __forceinline__ float2 coherent_load2(const float* p) {
     return __builtin_bit_cast(float2, u);
 }
 
-// One chunk's operands, held in registers between its load and its use.
-template <int MT>
-struct Stage {
-    u4 plane[6];   // plane rows 8 k + lane / 8 of the chunk (0..31 lo, 32..47 hi), 16 columns each
-    u4 a[MT][2];   // A[m0 + 16 mt + i][chunk * 64 + 32 h + 8 q .. + 7]
-    uint32_t sc;   // scales of columns n0 + 2 lane, n0 + 2 lane + 1 for the chunk's group
-};
-
-// Loads never branch: a column or row outside the matrix is clamped to one inside it.  Output columns depend only
-// on their own weight columns and scales, output rows only on their own A rows, so the clamped values land in
-// outputs that are never stored.
-template <int MT>
-__device__ __forceinline__ void load_stage(const Args& p, int b, int m0, int n0, int c, Stage<MT>& s) {
-    const int lane = threadIdx.x & 63;
-    const int seg = lane & 7, rr = lane >> 3;
-    const int n = min(n0 + 16 * seg, p.N - 16);
-    const uint8_t* const lo = p.lo + (int64_t)b * p.sl_b + ((int64_t)c * 32 + rr) * p.N + n;
-    const uint8_t* const hi = p.hi + (int64_t)b * p.sh_b + ((int64_t)c * 16 + rr) * p.N + n;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) s.plane[k] = *reinterpret_cast<const u4*>(lo + (int64_t)(8 * k) * p.N);
-#pragma unroll
-    for (int k = 0; k < 2; ++k) s.plane[4 + k] = *reinterpret_cast<const u4*>(hi + (int64_t)(8 * k) * p.N);
-    const int i = lane & 15, q = lane >> 4;
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-        const int m = min(m0 + 16 * mt + i, p.M - 1);
-        const uint16_t* const arow = p.a + (int64_t)b * p.sa_b + (int64_t)m * p.sa_m + (int64_t)c * 64 + 8 * q;
-        s.a[mt][0] = *reinterpret_cast<const u4*>(arow);
-        s.a[mt][1] = *reinterpret_cast<const u4*>(arow + 32);
-    }
-    const int g = (c * 64) / p.group_k;
-    const int col = min(n0 + 2 * lane, p.N - 2);
-    s.sc = *reinterpret_cast<const uint32_t*>(p.sc + (int64_t)b * p.ss_b + (int64_t)g * p.N + col);
-}
-
-// Contract one chunk into acc: stage it in the wave's LDS buffer, read it back transposed, dequantise, MFMA.
-template <class A, int MT>
-__device__ __forceinline__ void process_stage(const Stage<MT>& s, uint8_t* buf, f4 (&acc)[MT][kTiles]) {
-    const int lane = threadIdx.x & 63, q = lane >> 4, i = lane & 15;
-    const int seg = lane & 7, rr = lane >> 3;
-    wave_lds_sync();  // the previous chunk's reads of buf are issued before these writes
-#pragma unroll
-    for (int k = 0; k < 6; ++k) {
-        uint8_t* dst = buf + (8 * k + rr) * kPitch + 16 * seg;
-        *reinterpret_cast<uint2*>(dst) = uint2{s.plane[k][0], s.plane[k][1]};
-        *reinterpret_cast<uint2*>(dst + 8) = uint2{s.plane[k][2], s.plane[k][3]};
-    }
-    *reinterpret_cast<uint32_t*>(buf + kScaleOff + 4 * lane) = s.sc;
-    wave_lds_sync();
-    const u4 bias = u4{A::kBias, A::kBias, A::kBias, A::kBias};  // -(2^e + 32)
-    f4 corr[MT];
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-        corr[mt] = A::mma(s.a[mt][0], bias, f4{0.f, 0.f, 0.f, 0.f});
-        corr[mt] = A::mma(s.a[mt][1], bias, corr[mt]);
-    }
-    const int sel = 2 * (q >> 1);  // hi-plane field of rows 8 q .. (first half); the second half's is 4 bits up
-    const int r = lane & 15;
-    const int off = (r >> 1) * kPitch + 8 * (r & 1);
-    // every transposing read of the chunk is issued before the first use (one LDS latency per chunk)
-    v2i lo_t[kTiles], hi_t[kTiles];
-#pragma unroll
-    for (int t = 0; t < kTiles; ++t) {
-        lo_t[t] = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i*)(buf + (8 * q) * kPitch + off + 16 * t));
-        hi_t[t] = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i*)(buf + (32 + 8 * (q & 1)) * kPitch + off + 16 * t));
-    }
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int t = 0; t < kTiles; ++t) {
-        const v2i lov = lo_t[t], hiv = hi_t[t];
-        const float sv = h2f(*reinterpret_cast<const uint16_t*>(buf + kScaleOff + 2 * (16 * t + i)));
-        // lov: lo-plane rows 8 q + e of column i (e = 0..7, one byte each); hiv: hi-plane rows 8 (q & 1) + e
-        uint32_t o0[4], o1[4];
-#pragma unroll
-        for (int d = 0; d < 2; ++d) {
-            const uint32_t L = (uint32_t)lov[d], Hs = (uint32_t)hiv[d] >> sel;
-            const uint32_t u0 = (L & 0x0F0F0F0Fu) | ((Hs & 0x03030303u) << 4);          // rows 8 q + e
-            const uint32_t u1 = ((L >> 4) & 0x0F0F0F0Fu) | (Hs & 0x30303030u);          // rows 32 + 8 q + e
-            codes_to_op<A>(u0, o0[2 * d], o0[2 * d + 1]);
-            codes_to_op<A>(u1, o1[2 * d], o1[2 * d + 1]);
-        }
-        const u4 w0 = u4{o0[0], o0[1], o0[2], o0[3]};
-        const u4 w1 = u4{o1[0], o1[1], o1[2], o1[3]};
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt) {
-            f4 tc = A::mma(s.a[mt][0], w0, corr[mt]);
-            tc = A::mma(s.a[mt][1], w1, tc);
-#pragma unroll
-            for (int v = 0; v < 4; ++v) acc[mt][t][v] += tc[v] * sv;
-        }
-    }
-}
-
-template <int MT, bool F16>
-__device__ __forceinline__ void store_tile_as(const Args& p, int b, int m0, int n0, const f4 (&acc)[MT][kTiles]) {
-    const int lane = threadIdx.x & 63, i = lane & 15, q = lane >> 4;
-    // lane (i, q) holds C[m0 + 16 mt + 4 q + v][n0 + 16 t + i]
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-        for (int t = 0; t < kTiles; ++t) {
-            const int n = n0 + 16 * t + i;
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int m = m0 + 16 * mt + 4 * q + v;
-                if (n >= p.N || m >= p.M) continue;
-                put_out<F16>(p, (int64_t)b * p.so_b + (int64_t)m * p.so_m + n, acc[mt][t][v]);
-            }
-        }
-}
-template <int MT>
-__device__ __forceinline__ void store_tile(const Args& p, int b, int m0, int n0, const f4 (&acc)[MT][kTiles]) {
-    if (p.out_dtype == W6A16_OUT_F16)
-        store_tile_as<MT, true>(p, b, m0, n0, acc);
-    else
-        store_tile_as<MT, false>(p, b, m0, n0, acc);
-}
-
-// Split-K reduction of rows r0 .. r0 + R - 1 (those below `rows`) of a tile whose partials lie at `part`: lane l sums
-// columns 2 l, 2 l + 1 split by split in order 0, 1, ... and stores the result.  The loads of R rows x 8 splits are
-// issued together (each batch waits about one memory latency); rows past `rows` and splits past split_k re-read
-// valid entries whose values are not used.
-template <int R, bool F16>
-__device__ __forceinline__ void reduce_rows(const Args& p, const float* part, int tile_floats, int r0, int rows,
-                                            int b, int m0, int n0) {
-    const int lane = threadIdx.x & 63;
-    const int n = n0 + 2 * lane;
-    const float* src[R];
-#pragma unroll
-    for (int j = 0; j < R; ++j) src[j] = part + min(r0 + j, rows - 1) * kTileN + 2 * lane;
-    float2 s[R];
-#pragma unroll
-    for (int j = 0; j < R; ++j) s[j] = float2{0.f, 0.f};
-    for (int sp = 0; sp < p.split_k; sp += 8) {
-        float2 x[R][8];
-#pragma unroll
-        for (int j = 0; j < R; ++j)
-#pragma unroll
-            for (int k = 0; k < 8; ++k)
-                x[j][k] = coherent_load2(src[j] + (int64_t)min(sp + k, p.split_k - 1) * tile_floats);
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            if (sp + k >= p.split_k) break;
-#pragma unroll
-            for (int j = 0; j < R; ++j) {
-                s[j].x += x[j][k].x;
-                s[j].y += x[j][k].y;
-            }
-        }
-    }
-    const int64_t ob = (int64_t)b * p.so_b;
-#pragma unroll
-    for (int j = 0; j < R; ++j) {
-        if (r0 + j >= rows || n >= p.N) continue;
-        const int64_t o = ob + (int64_t)(m0 + r0 + j) * p.so_m + n;
-        put_out<F16>(p, o, s[j].x);
-        put_out<F16>(p, o + 1, s[j].y);
-    }
-}
-
-// Split-K: this split's partial tile of `tile`, row-major [16 MT rows][128 columns] fp32 per (tile, split); rows >= M
-// are not written.
-template <int MT>
-__device__ __forceinline__ void publish_partials(const Args& p, int64_t tile, int split, int m0,
-                                                 const f4 (&acc)[MT][kTiles]) {
-    const int lane = threadIdx.x & 63, q = lane >> 4;
-    constexpr int kTileFloats = 16 * MT * kTileN;
-    const int rows = min(16 * MT, p.M - m0);  // valid rows of this tile
-    float* const mine = p.part + (tile * p.split_k + split) * kTileFloats + (lane & 15);
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-        for (int t = 0; t < kTiles; ++t)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int r = 16 * mt + 4 * q + v;
-                if (r < rows) coherent_store(mine + r * kTileN + 16 * t, acc[mt][t][v]);
-            }
-}
-
-// Split-K, in the split that completed `tile`: sum the partials in split order (a fixed order: the result does not
-// depend on which split arrived last), store the result, reset the tile's counter.
-template <int MT>
-__device__ __forceinline__ void reduce_tile(const Args& p, int64_t tile, int b, int m0, int n0) {
-    const int lane = threadIdx.x & 63;
-    constexpr int kTileFloats = 16 * MT * kTileN;
-    const float* const part = p.part + tile * p.split_k * kTileFloats;
-    const int rows = min(16 * MT, p.M - m0);
-    const bool f16 = p.out_dtype == W6A16_OUT_F16;
-    if (rows == 1) {
-        if (f16)
-            reduce_rows<1, true>(p, part, kTileFloats, 0, 1, b, m0, n0);
-        else
-            reduce_rows<1, false>(p, part, kTileFloats, 0, 1, b, m0, n0);
-    } else {
-        for (int r0 = 0; r0 < rows; r0 += 4)
-            if (f16)
-                reduce_rows<4, true>(p, part, kTileFloats, r0, rows, b, m0, n0);
-            else
-                reduce_rows<4, false>(p, part, kTileFloats, r0, rows, b, m0, n0);
-    }
-    if (lane == 0) __hip_atomic_store(p.cnt + tile, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
 // ---------------------------------------------------------------------------------------------------------------
 // Packed layout: the same 6 bits per weight and fp16 scales, re-laid out once (w6a16_pack) so that each wavefront's
 // 64-row chunk of a 128-column strip is one contiguous 6 KB block already in MFMA operand order.  Block (b, strip,
@@ -392,434 +163,11 @@ __device__ __forceinline__ void reduce_tile(const Args& p, int64_t tile, int b, 
 // lane (i, q) reads its eight columns' scales as one 16-byte load.  Columns past N hold zero codes and scales.
 constexpr int kPackBytes = 6144;
 
-template <int MT>
-struct PStage {
-    u4 w[6];       // the lane's 24-dword record
-    u4 a[MT][2];   // A[m0 + 16 mt + i][chunk * 64 + 32 h + 8 q .. + 7]
-    u4 sc;         // scales of columns n0 + 16 t + i, t = 0..7 (fp16)
-};
-
-template <int MT>
-__device__ __forceinline__ void load_pstage(const Args& p, int b, int m0, int strip, int c, PStage<MT>& s) {
-    const int lane = threadIdx.x & 63, i = lane & 15, q = lane >> 4;
-    const int nchunks = p.K / 64;
-    const uint8_t* const blk =
-        p.lo + (int64_t)b * p.sl_b + ((int64_t)strip * nchunks + c) * kPackBytes + 16 * lane;
-#pragma unroll
-    for (int k = 0; k < 6; ++k) s.w[k] = *reinterpret_cast<const u4*>(blk + 1024 * k);
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-        const int m = min(m0 + 16 * mt + i, p.M - 1);
-        const uint16_t* const arow = p.a + (int64_t)b * p.sa_b + (int64_t)m * p.sa_m + (int64_t)c * 64 + 8 * q;
-        s.a[mt][0] = *reinterpret_cast<const u4*>(arow);
-        s.a[mt][1] = *reinterpret_cast<const u4*>(arow + 32);
-    }
-    const int g = (c * 64) / p.group_k, groups = p.K / p.group_k;
-    s.sc = *reinterpret_cast<const u4*>(p.sc + (int64_t)b * p.ss_b + ((int64_t)strip * groups + g) * kTileN + 8 * i);
-}
-
-template <class A, int MT>
-__device__ __forceinline__ void process_pstage(const PStage<MT>& s, f4 (&acc)[MT][kTiles]) {
-    const u4 bias = u4{A::kBias, A::kBias, A::kBias, A::kBias};  // -(2^e + 32)
-    f4 corr[MT];
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-        corr[mt] = A::mma(s.a[mt][0], bias, f4{0.f, 0.f, 0.f, 0.f});
-        corr[mt] = A::mma(s.a[mt][1], bias, corr[mt]);
-    }
-#pragma unroll
-    for (int t = 0; t < kTiles; ++t) {
-        const uint32_t L0 = s.w[t >> 1][2 * (t & 1)], L1 = s.w[t >> 1][2 * (t & 1) + 1];
-        const uint32_t Hd = s.w[4 + (t >> 2)][t & 3];
-        const uint32_t u0a = (L0 & 0x0F0F0F0Fu) | ((Hd & 0x03030303u) << 4);         // rows 8 q + 0..3
-        const uint32_t u0b = (L1 & 0x0F0F0F0Fu) | (Hd & 0x30303030u);                // rows 8 q + 4..7
-        const uint32_t u1a = ((L0 >> 4) & 0x0F0F0F0Fu) | ((Hd & 0x0C0C0C0Cu) << 2);  // rows 32 + 8 q + 0..3
-        const uint32_t u1b = ((L1 >> 4) & 0x0F0F0F0Fu) | ((Hd >> 2) & 0x30303030u);  // rows 32 + 8 q + 4..7
-        uint32_t o0[4], o1[4];
-        codes_to_op<A>(u0a, o0[0], o0[1]);
-        codes_to_op<A>(u0b, o0[2], o0[3]);
-        codes_to_op<A>(u1a, o1[0], o1[1]);
-        codes_to_op<A>(u1b, o1[2], o1[3]);
-        const u4 w0 = u4{o0[0], o0[1], o0[2], o0[3]};
-        const u4 w1 = u4{o1[0], o1[1], o1[2], o1[3]};
-        const float sv = h2f((uint16_t)(s.sc[t >> 1] >> (16 * (t & 1))));
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt) {
-            f4 tc = A::mma(s.a[mt][0], w0, corr[mt]);
-            tc = A::mma(s.a[mt][1], w1, tc);
-#pragma unroll
-            for (int v = 0; v < 4; ++v) acc[mt][t][v] += tc[v] * sv;
-        }
-    }
-}
-
-// Narrow kernel (M <= 32), both weight formats: a workgroup of four wavefronts, one per 128-column strip.
-template <class A, int MT, int D, bool PACKED>
-__global__ __launch_bounds__(64 * kStrips) void w6a16_kernel(const Args p) {
-    constexpr int kStage = PACKED ? 16 : kStrips * kBuf;  // planes: each wavefront's staging buffer
-    __shared__ __attribute__((aligned(16))) uint8_t lds[kStage];
-    const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int sw = wv;
-    const int strip = blockIdx.x * kStrips + sw;
-    const bool live = strip < p.n_strips;
-    const int n0 = strip * kTileN;
-    const int split = blockIdx.y;
-    const int b = blockIdx.z / p.m_groups, mg = blockIdx.z % p.m_groups;
-    const int m0 = mg * 16 * MT;
-    const int nchunks = p.K / 64;
-    const int c0 = split * p.chunks_per_split, c1 = min(nchunks, c0 + p.chunks_per_split);
-    uint8_t* const buf = lds + (PACKED ? 0 : wv * kBuf);
-
-    f4 acc[MT][kTiles];
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-        for (int t = 0; t < kTiles; ++t) acc[mt][t] = f4{0.f, 0.f, 0.f, 0.f};
-
-    if (live && c0 < c1) {
-        // D chunks in flight.  Chunks past the range re-load the last one (a cache hit), so every load is
-        // unconditional.  Packed: whole groups of D chunks run unconditionally (a use of a stage under a condition
-        // let the compiler sink that stage's loads to the use, leaving no load in flight) and a scheduling barrier
-        // keeps each stage's loads where they are issued; the remainder (fewer than D chunks, already loaded)
-        // follows.
-        typedef typename std::conditional<PACKED, PStage<MT>, Stage<MT>>::type S;
-        S st[D];
-        auto load = [&](int c, S& x) {
-            if constexpr (PACKED) load_pstage<MT>(p, b, m0, strip, c, x);
-            else load_stage<MT>(p, b, m0, n0, c, x);
-        };
-        auto work = [&](const S& x) {
-            if constexpr (PACKED) process_pstage<A, MT>(x, acc);
-            else process_stage<A, MT>(x, buf, acc);
-        };
-#pragma unroll
-        for (int j = 0; j < D; ++j) load(min(c0 + j, c1 - 1), st[j]);
-        if constexpr (PACKED) {
-            const int full = c0 + (c1 - c0) / D * D;
-            for (int c = c0; c < full; c += D) {
-#pragma unroll
-                for (int j = 0; j < D; ++j) {
-                    work(st[j]);
-                    load(min(c + j + D, c1 - 1), st[j]);
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-            }
-#pragma unroll
-            for (int j = 0; j + 1 < D; ++j)
-                if (full + j < c1) work(st[j]);
-        } else {
-            // the planes' stages are consumed by LDS stores: here the compiler keeps the loads in place on its own
-            // (measured 1 us faster per call than the form above)
-            for (int c = c0; c < c1; c += D) {
-#pragma unroll
-                for (int j = 0; j < D; ++j) {
-                    if (c + j < c1) work(st[j]);
-                    load(min(c + j + D, c1 - 1), st[j]);
-                }
-            }
-        }
-    }
-
-    const bool owner = live;  // this wavefront finishes its strip's tile
-    if (p.split_k == 1) {  // uniform over the grid
-        if (owner) store_tile<MT>(p, b, m0, n0, acc);
-        return;
-    }
-    // Split-K hand-off, one agent-scope release per workgroup.  An agent-scope release fence writes back the XCD's L2
-    // (a walk whose cost grows with the number of releases, not with the dirty data): issued by every wavefront it
-    // cost 6 us per call at M = 1 and 42 us at M = 128.  Here every wavefront stores its strip's partials and waits
-    // for them; the workgroup barrier orders those stores before wavefront 0's release fence, which then counts all
-    // of the workgroup's strips in with relaxed atomic increments; if a strip completed, wavefront 0's acquire fence
-    // follows, and the second barrier orders it before the reducing wavefronts' reads.
-    const int64_t tile0 = ((int64_t)b * p.m_groups + mg) * p.n_strips;
-    if (owner) publish_partials<MT>(p, tile0 + strip, split, m0, acc);
-    __builtin_amdgcn_s_waitcnt(0);  // this wavefront's partial stores have completed
-    __shared__ uint32_t completed[kStrips];
-    __syncthreads();
-    if (wv == 0) {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-        bool done = false;
-        if (lane < kStrips) {
-            const int st = blockIdx.x * kStrips + lane;
-            if (st < p.n_strips)
-                done = __hip_atomic_fetch_add(p.cnt + tile0 + st, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
-                       (uint32_t)p.split_k - 1;
-            completed[lane] = done ? 1u : 0u;
-        }
-        if (__builtin_amdgcn_ballot_w64(done)) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-    }
-    __syncthreads();
-    if (owner && completed[sw]) reduce_tile<MT>(p, tile0 + strip, b, m0, n0);
-}
-
-// Half a strip of the packed layout (tiles 4 h .. 4 h + 3 of the 128-column strip, one 16-row tile of A): load
-// instructions 2 h, 2 h + 1 (the low bits) and 4 + h (the top bits) of the chunk's 6 KB block, scale dwords 2 h and
-// 2 h + 1.  Tile t of the half computes exactly what process_pstage computes for tile 4 h + t.
-struct PHalf {
-    u4 w[3];
-    u4 a[2];
-    uint2 sc;
-};
-
-__device__ __forceinline__ void load_phalf(const Args& p, int b, int m0, int strip, int h, int c, PHalf& s) {
-    const int lane = threadIdx.x & 63, i = lane & 15, q = lane >> 4;
-    const int nchunks = p.K / 64;
-    const uint8_t* const blk =
-        p.lo + (int64_t)b * p.sl_b + ((int64_t)strip * nchunks + c) * kPackBytes + 16 * lane;
-    s.w[0] = *reinterpret_cast<const u4*>(blk + 1024 * (2 * h));
-    s.w[1] = *reinterpret_cast<const u4*>(blk + 1024 * (2 * h + 1));
-    s.w[2] = *reinterpret_cast<const u4*>(blk + 1024 * (4 + h));
-    const int m = min(m0 + i, p.M - 1);
-    const uint16_t* const arow = p.a + (int64_t)b * p.sa_b + (int64_t)m * p.sa_m + (int64_t)c * 64 + 8 * q;
-    s.a[0] = *reinterpret_cast<const u4*>(arow);
-    s.a[1] = *reinterpret_cast<const u4*>(arow + 32);
-    const int g = (c * 64) / p.group_k, groups = p.K / p.group_k;
-    s.sc = *reinterpret_cast<const uint2*>(p.sc + (int64_t)b * p.ss_b + ((int64_t)strip * groups + g) * kTileN + 8 * i +
-                                           4 * h);
-}
-
-template <class A>
-__device__ __forceinline__ void process_phalf(const PHalf& s, f4 (&acc)[1][4]) {
-    const u4 bias = u4{A::kBias, A::kBias, A::kBias, A::kBias};  // -(2^e + 32)
-    f4 corr = A::mma(s.a[0], bias, f4{0.f, 0.f, 0.f, 0.f});
-    corr = A::mma(s.a[1], bias, corr);
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-        const uint32_t L0 = s.w[t >> 1][2 * (t & 1)], L1 = s.w[t >> 1][2 * (t & 1) + 1];
-        const uint32_t Hd = s.w[2][t];
-        const uint32_t u0a = (L0 & 0x0F0F0F0Fu) | ((Hd & 0x03030303u) << 4);
-        const uint32_t u0b = (L1 & 0x0F0F0F0Fu) | (Hd & 0x30303030u);
-        const uint32_t u1a = ((L0 >> 4) & 0x0F0F0F0Fu) | ((Hd & 0x0C0C0C0Cu) << 2);
-        const uint32_t u1b = ((L1 >> 4) & 0x0F0F0F0Fu) | ((Hd >> 2) & 0x30303030u);
-        uint32_t o0[4], o1[4];
-        codes_to_op<A>(u0a, o0[0], o0[1]);
-        codes_to_op<A>(u0b, o0[2], o0[3]);
-        codes_to_op<A>(u1a, o1[0], o1[1]);
-        codes_to_op<A>(u1b, o1[2], o1[3]);
-        const u4 w0 = u4{o0[0], o0[1], o0[2], o0[3]};
-        const u4 w1 = u4{o1[0], o1[1], o1[2], o1[3]};
-        const float sv = h2f((uint16_t)((t >> 1 ? s.sc.y : s.sc.x) >> (16 * (t & 1))));
-        f4 tc = A::mma(s.a[0], w0, corr);
-        tc = A::mma(s.a[1], w1, tc);
-#pragma unroll
-        for (int v = 0; v < 4; ++v) acc[0][t][v] += tc[v] * sv;
-    }
-}
-
-// In-workgroup split-K (M <= 32, 2 <= split_k <= kGemvMaxSplit): the split_k ranges of one 128-column strip run as
-// the wavefronts of one workgroup -- wavefront w takes exactly the chunks split w of w6a16_kernel takes -- and their
-// partial tiles are summed through LDS in split order 0, 1, ..., the same fp32 sums as w6a16_kernel's hand-off
-// (bit-identical results) with no cross-workgroup hand-off, counter or workspace traffic.  One workgroup per strip
-// and 16-row M group, or (NT = 4, packed layout) per half strip, which doubles the workgroups where strips are fewer
-// than CUs.
-constexpr int kGemvMaxSplit = 8;
-constexpr int kGemvPart = kGemvMaxSplit * 16 * kTileN * 4;  // fp32 partial tiles [split][16 rows][128 columns]
-constexpr int kGemvLds = kGemvMaxSplit * kBuf > kGemvPart ? kGemvMaxSplit * kBuf : kGemvPart;
-
-// The gemv epilogue: output element (r, col) of the tile is the sum of the ks wavefront partials in `part`.
-template <int NC, bool F16>
-__device__ __forceinline__ void gemv_sum_store(const Args& p, const float* part, int rows, int ks, int b, int m0,
-                                               int n0) {
-    for (int e = threadIdx.x; e < rows * NC; e += blockDim.x) {
-        const int r = e / NC, col = e % NC, n = n0 + col;
-        float sum = 0.f;
-        for (int w = 0; w < ks; ++w) sum += part[(w * 16 + r) * NC + col];
-        if (n >= p.N) continue;
-        put_out<F16>(p, (int64_t)b * p.so_b + (int64_t)(m0 + r) * p.so_m + n, sum);
-    }
-}
-
-template <class A, int D, bool PACKED, int NT>
-__global__ __launch_bounds__(64 * kGemvMaxSplit) void w6a16_gemv_kernel(const Args p) {
-    static_assert(NT == kTiles || (NT == 4 && PACKED), "half strips: packed layout only");
-    constexpr int MT = 1, NC = 16 * NT;  // NC: columns per workgroup
-    __shared__ __attribute__((aligned(16))) uint8_t lds[kGemvLds];
-    const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int strip = blockIdx.x / (kTiles / NT), h = blockIdx.x % (kTiles / NT);
-    const int n0 = strip * kTileN + h * NC;
-    const int b = blockIdx.z / p.m_groups, mg = blockIdx.z % p.m_groups;
-    const int m0 = mg * 16;
-    const int nchunks = p.K / 64;
-    const int c0 = wv * p.chunks_per_split, c1 = min(nchunks, c0 + p.chunks_per_split);
-    uint8_t* const buf = lds + (PACKED ? 0 : wv * kBuf);
-
-    f4 acc[MT][NT];
-#pragma unroll
-    for (int t = 0; t < NT; ++t) acc[0][t] = f4{0.f, 0.f, 0.f, 0.f};
-
-    if (c0 < c1) {  // the loop of w6a16_kernel, for this wavefront's range
-        typedef typename std::conditional<PACKED, typename std::conditional<NT == 4, PHalf, PStage<MT>>::type,
-                                          Stage<MT>>::type S;
-        S st[D];
-        auto load = [&](int c, S& x) {
-            if constexpr (PACKED && NT == 4) load_phalf(p, b, m0, strip, h, c, x);
-            else if constexpr (PACKED) load_pstage<MT>(p, b, m0, strip, c, x);
-            else load_stage<MT>(p, b, m0, n0, c, x);
-        };
-        auto work = [&](const S& x) {
-            if constexpr (PACKED && NT == 4) process_phalf<A>(x, acc);
-            else if constexpr (PACKED) process_pstage<A, MT>(x, acc);
-            else process_stage<A, MT>(x, buf, acc);
-        };
-#pragma unroll
-        for (int j = 0; j < D; ++j) load(min(c0 + j, c1 - 1), st[j]);
-        if constexpr (PACKED) {
-            const int full = c0 + (c1 - c0) / D * D;
-            for (int c = c0; c < full; c += D) {
-#pragma unroll
-                for (int j = 0; j < D; ++j) {
-                    work(st[j]);
-                    load(min(c + j + D, c1 - 1), st[j]);
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-            }
-#pragma unroll
-            for (int j = 0; j + 1 < D; ++j)
-                if (full + j < c1) work(st[j]);
-        } else {
-            for (int c = c0; c < c1; c += D) {
-#pragma unroll
-                for (int j = 0; j < D; ++j) {
-                    if (c + j < c1) work(st[j]);
-                    load(min(c + j + D, c1 - 1), st[j]);
-                }
-            }
-        }
-    }
-    __syncthreads();  // the staging buffers are dead: the partial tiles reuse the LDS
-    float* const part = reinterpret_cast<float*>(lds);
-    {
-        const int i = lane & 15, q = lane >> 4;  // lane (i, q) holds rows 4 q + v of column 16 t + i
-#pragma unroll
-        for (int t = 0; t < NT; ++t)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) part[(wv * 16 + 4 * q + v) * NC + 16 * t + i] = acc[0][t][v];
-    }
-    __syncthreads();
-    const int rows = min(16, p.M - m0), ks = p.split_k;
-    if (p.out_dtype == W6A16_OUT_F16)
-        gemv_sum_store<NC, true>(p, part, rows, ks, b, m0, n0);
-    else
-        gemv_sum_store<NC, false>(p, part, rows, ks, b, m0, n0);
-}
-
-// ---------------------------------------------------------------------------------------------------------------
-// Wide kernel (M > 32).  A workgroup of 4 KP wavefronts covers one 128-column strip for 16 MTW rows of A: wavefront
-// w owns column tiles 2 (w & 3) and 2 (w & 3) + 1 for all the workgroup's rows, over K part w >> 2 (the workgroup's
-// chunk range cut into KP contiguous parts, summed through LDS at the end).  Each dequantised weight operand serves
-// MTW M tiles, each A operand two column tiles.  The M groups of one strip are 8 blocks apart in dispatch order (the
-// same XCD, one after the other), so the weight bytes come from HBM once per strip and hit that XCD's L2 for the
-// other groups.
-//   * A's chunk of every part ([16 MTW rows][64 k] bf16) is staged in LDS, double-buffered, one workgroup barrier
-//     per step.  16-byte piece j of row r sits at slot 8 r + (j ^ ((r >> 1) & 7)): the 16 lanes of an MFMA operand
-//     read (rows r0 .. r0 + 15, one j) touch all 64 banks once, and so do the writes.
-//   * Chains: the products of CG consecutive chunks (CG = 2 when the quantisation group holds two chunks, else 1)
-//     accumulate in one MFMA chain whose accumulator starts at the chain's bias -160 sum_k A[m][k] (the row sums of
-//     w6a16_rowsum_kernel, computed once per call instead of once per strip), then are scaled once: acc += s * chain.
-//     (Measured against row sums taken by the staging threads with per-chunk scaling, which saves that launch: M = 64
-//     1 us faster, M = 128 3 us and M = 256 18 us slower per call -- the per-step VALU work decides at four M tiles.)
-//   * Packed weights are loaded straight into registers (16 + 8 bytes per lane and chunk: the lane's records of its
-//     two tiles), D steps ahead; planes are staged in LDS with A (48 rows x 128 columns) and read back transposed as
-//     in the narrow kernel.
-// Split-K (when used): one partial tile per (tile, split) in the accumulators' register layout, one release per
-// workgroup; the last split adds the others to its own registers in split order.
-constexpr int kCachePolicySC1 = 16;  // buffer instructions' cache-policy bit sc1: device-scope write-through
-constexpr int kPlaneBytes = kBuf;    // planes: the chunk's 48 plane rows and 128 scales, as in the narrow kernel
-
-template <int MTW>
-constexpr int part_a_bytes() { return 16 * MTW * 128; }
-
-// One K part's share of an LDS stage: A slots, the chain's row sums (16 MTW fp32), then (planes) the plane rows.
-template <int MTW, bool PACKED>
-constexpr int part_bytes() { return part_a_bytes<MTW>() + 16 * MTW * 4 + (PACKED ? 0 : kPlaneBytes); }
-
-__device__ __forceinline__ int a_slot(int r, int j) { return 8 * r + (j ^ ((r >> 1) & 7)); }
-
 using wkv7::unroll;  // f(integral_constant<0>), .., f(integral_constant<N - 1>)
 
-// (1, 1) as an activation pair held in a register (an empty asm keeps the compiler from folding the pair into an
-// inline constant, which the packed dot product would read differently).
-template <class A>
-__device__ __forceinline__ uint32_t ones_x2() {
-    uint32_t bits = A::kOnes;
-    asm("" : "+v"(bits));
-    return bits;
-}
-
-template <class A>
-__device__ __forceinline__ float sum8(const u4 v, uint32_t one) {
-    float x = 0.f;
-#pragma unroll
-    for (int d = 0; d < 4; ++d) {
-        // the element is copied out first: bit-casting a vector element in place (v[d]) compiled to a read of
-        // element 0 for every d
-        const uint32_t word = v[d];
-        x = A::dot2(word, one, x);
-    }
-    return x;
-}
-
-template <int CTRL>
-__device__ __forceinline__ float dpp_add(float x) {  // x + x of the lane DPP control CTRL selects (all lanes active)
-    return x + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xF, 0xF, false));
-}
-
-// Row sums of A per chain of 64 CG k: rsum[b][chain][m] = -(2^e + 32) sum A[b][m][chain 64 CG .. + 64 CG - 1], zero for
-// rows M <= m < mpad.  One wavefront per (row, 512-element segment of K; 8 bf16 per lane, coalesced); the 8 CG lanes
-// of a chain add their sums with DPP in a fixed order.
-template <class A>
-__global__ __launch_bounds__(256) void w6a16_rowsum_kernel(const Args p) {
-    const int lane = threadIdx.x & 63;
-    const int m = blockIdx.x * 4 + (threadIdx.x >> 6), k = blockIdx.y * 512 + 8 * lane, b = blockIdx.z;
-    if (m >= p.mpad) return;  // uniform over the wavefront
-    const int lanes_per_chain = 8 * p.chain_k / 64;  // 8 or 16
-    const uint16_t* const row = p.a + (int64_t)b * p.sa_b + (int64_t)min(m, p.M - 1) * p.sa_m;
-    // K is a multiple of 64 CG: a chain's lanes are all inside K or all past it
-    float x = (m < p.M && k < p.K) ? sum8<A>(*reinterpret_cast<const u4*>(row + k), ones_x2<A>()) : 0.f;
-    x = dpp_add<0xB1>(x);   // lanes ^ 1
-    x = dpp_add<0x4E>(x);   // lanes ^ 2: each lane holds its quad's sum
-    x = dpp_add<0x141>(x);  // half-row mirror: lane 7 - l of the 8-lane group, in the other quad
-    if (lanes_per_chain == 16) x = dpp_add<0x140>(x);  // row mirror: lane 15 - l, in the other half
-    if ((lane & (lanes_per_chain - 1)) == 0 && k < p.K)
-        p.rsum[((int64_t)b * p.nchains + k / p.chain_k) * p.mpad + m] = -A::kOffset * x;
-}
-
-// The chunk schedule of one workgroup: its split's range of chains, cut into KP contiguous parts.
-struct Sched {
-    int cg, c_s, per, n_s, nchunks;  // chunks per chain, first chunk of the split, chunks per part, split's chunks
-    __device__ __forceinline__ int part_n(int kq) const { return max(0, min(per, n_s - kq * per)); }
-    // chunk of part kq at step s, clamped into the part and the matrix (steps past a part's end re-load its last
-    // chunk; a part with no chunk loads a valid one)
-    __device__ __forceinline__ int chunk(int kq, int s) const {
-        return min(c_s + kq * per + max(0, min(s, part_n(kq) - 1)), nchunks - 1);
-    }
-};
-
-// What one thread loads per step into the LDS stage: MTW / 2 pieces of A, four row sums (threads 0 .. 4 MTW - 1
-// of each part's 256) and (planes) 16 bytes of a lo-plane row, 16 bytes of a hi-plane row (threads 0..127 of each
-// part's 256) or two scales (threads 128..191).
-template <int MTW, bool PACKED>
-struct WideLds {
-    u4 a[MTW / 2];
-    u4 rs;
-    u4 pl[2];
-    uint32_t sc;
-};
-
-// The packed weights of one chunk in one lane's registers: R[4 cp .. 4 cp + 3] (lo plane bytes of tiles 2 cp and
-// 2 cp + 1), R[16 + 2 cp], R[17 + 2 cp] (their top bits) and the two tiles' scales of column i.
-struct WideW {
-    u4 lo;
-    uint2 hd;
-    uint32_t sc;
-};
-
-// Buffer resources and per-lane offsets of the wide kernel's loads, fixed for the whole call: inside the loop only
-// the chunk-dependent part changes, and it is the same for a whole wavefront (its K part's chunk), so it goes into the
-// instructions' scalar offset and the loop's address arithmetic runs on the scalar unit.
-// A raw buffer over [base, base + bytes) (capped at 2 GB; the validation keeps every range the kernel addresses below
-// it).  The base and size are passed through readfirstlane so that the descriptor is provably wave-uniform: a
-// descriptor the compiler cannot prove uniform is used through a per-lane loop.
+// A raw buffer over [base, base + bytes) (capped at 2 GB).  The base and size are passed through readfirstlane so that
+// the descriptor is provably wave-uniform: a descriptor the compiler cannot prove uniform is used through a per-lane
+// loop.
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(uint64_t base, int64_t bytes) {
     const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)base);
     const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(base >> 32));
@@ -831,393 +179,437 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(uint64_t base, int64_t by
 // A wave-uniform scalar offset (held in an SGPR, as buffer instructions need it).
 __device__ __forceinline__ int soff(int x) { return __builtin_amdgcn_readfirstlane(x); }
 
-template <int MTW>
-struct WideSrc {
-    uint64_t a, rs, lo, hi, sc;                 // buffer bases (wave-uniform)
-    int64_t na, nrs, nlo, nhi, nsc;             // and sizes in bytes
-    uint32_t va[MTW / 2], vrs, vlo, vhi, vsc;  // per-lane byte offsets
-    int kq[MTW / 2], kq_t, kp;                 // wave-uniform K parts: of each A piece, of the row-sum / plane loads,
-                                               // of this wavefront
-};
-
-template <int MTW, int KP, bool PACKED>
-__device__ __forceinline__ void wide_src(const Args& p, int b, int m0, int strip, WideSrc<MTW>& x) {
-    const int tid = threadIdx.x, lane = tid & 63, t = tid & 255, i = lane & 15, cp = (tid >> 6) & 3;
-    const int n0 = strip * kTileN;
-    x.a = reinterpret_cast<uint64_t>(p.a + (int64_t)b * p.sa_b);
-    x.na = ((int64_t)(p.M - 1) * p.sa_m + p.K) * 2;
-#pragma unroll
-    for (int e = 0; e < MTW / 2; ++e) {
-        const int piece = tid + 256 * KP * e, w = piece % (128 * MTW);
-        x.kq[e] = __builtin_amdgcn_readfirstlane(piece / (128 * MTW));  // one K part per wavefront and e
-        const int m = min(m0 + (w >> 3), p.M - 1);
-        x.va[e] = (uint32_t)(((int64_t)m * p.sa_m + 8 * (w & 7)) * 2);
-    }
-    x.kq_t = __builtin_amdgcn_readfirstlane(tid >> 8);
-    x.kp = __builtin_amdgcn_readfirstlane(tid >> 8);
-    x.rs = reinterpret_cast<uint64_t>(p.rsum + (int64_t)b * p.nchains * p.mpad);
-    x.nrs = (int64_t)p.nchains * p.mpad * 4;
-    x.vrs = (m0 + 4 * min(t, 4 * MTW - 1)) * 4;
-    if constexpr (PACKED) {
-        const int nchunks = p.K / 64, groups = p.K / p.group_k;
-        x.lo = reinterpret_cast<uint64_t>(p.lo + (int64_t)b * p.sl_b + (int64_t)strip * nchunks * kPackBytes);
-        x.nlo = (int64_t)nchunks * kPackBytes;
-        x.vlo = 16 * lane + 1024 * cp;
-        x.vhi = 4096 + 1024 * (cp >> 1) + 8 * (cp & 1) + 16 * lane;
-        x.sc = reinterpret_cast<uint64_t>(p.sc + (int64_t)b * p.ss_b + (int64_t)strip * groups * kTileN);
-        x.nsc = (int64_t)groups * kTileN * 2;
-        x.vsc = (8 * i + 2 * cp) * 2;
-    } else {
-        const int row = t >> 3, n = min(n0 + 16 * (t & 7), p.N - 16);  // lo row 0..31; hi row (row & 15)
-        x.lo = reinterpret_cast<uint64_t>(p.lo + (int64_t)b * p.sl_b);
-        x.nlo = (int64_t)(p.K / 2) * p.N;
-        x.vlo = row * p.N + n;
-        x.hi = reinterpret_cast<uint64_t>(p.hi + (int64_t)b * p.sh_b);
-        x.nhi = (int64_t)(p.K / 4) * p.N;
-        x.vhi = (row & 15) * p.N + n;
-        x.sc = reinterpret_cast<uint64_t>(p.sc + (int64_t)b * p.ss_b);
-        x.nsc = (int64_t)(p.K / p.group_k) * p.N * 2;
-        x.vsc = min(n0 + 2 * (t & 63), p.N - 2) * 2;
-    }
-}
-
-template <int MTW, int KP, bool PACKED>
-__device__ __forceinline__ void wide_load_lds(const Args& p, const Sched& S, const WideSrc<MTW>& src, int s,
-                                              WideLds<MTW, PACKED>& x) {
-#pragma unroll
-    for (int e = 0; e < MTW / 2; ++e)
-        x.a[e] = __builtin_amdgcn_raw_buffer_load_b128(rsrc(src.a, src.na), src.va[e], soff(S.chunk(src.kq[e], s) * 128), 0);
-    const int c = soff(S.chunk(src.kq_t, s));
-    x.rs = __builtin_amdgcn_raw_buffer_load_b128(rsrc(src.rs, src.nrs), src.vrs, soff((c / S.cg) * p.mpad * 4), 0);
-    if constexpr (!PACKED) {
-        x.pl[0] = __builtin_amdgcn_raw_buffer_load_b128(rsrc(src.lo, src.nlo), src.vlo, soff(c * 32 * p.N), 0);
-        x.pl[1] = __builtin_amdgcn_raw_buffer_load_b128(rsrc(src.hi, src.nhi), src.vhi, soff(c * 16 * p.N), 0);
-        x.sc = __builtin_amdgcn_raw_buffer_load_b32(rsrc(src.sc, src.nsc), src.vsc, soff((c * 64 / p.group_k) * p.N * 2), 0);
-    }
-}
-
-template <int MTW, int KP, bool PACKED>
-__device__ __forceinline__ void wide_store_lds(const WideLds<MTW, PACKED>& x, uint8_t* st) {
-    constexpr int PB = part_bytes<MTW, PACKED>();
-    const int tid = threadIdx.x;
-#pragma unroll
-    for (int e = 0; e < MTW / 2; ++e) {
-        const int piece = tid + 256 * KP * e, kq = piece / (128 * MTW), w = piece % (128 * MTW);
-        *reinterpret_cast<u4*>(st + kq * PB + 16 * a_slot(w >> 3, w & 7)) = x.a[e];
-    }
-    const int kq = tid >> 8, t = tid & 255;
-    uint8_t* const ps = st + kq * PB;
-    if (t < 4 * MTW) *reinterpret_cast<u4*>(ps + part_a_bytes<MTW>() + 16 * t) = x.rs;
-    if constexpr (!PACKED) {
-        uint8_t* const pl = ps + part_a_bytes<MTW>() + 16 * MTW * 4;
-        uint8_t* dst = pl + (t >> 3) * kPitch + 16 * (t & 7);
-        *reinterpret_cast<uint2*>(dst) = uint2{x.pl[0][0], x.pl[0][1]};
-        *reinterpret_cast<uint2*>(dst + 8) = uint2{x.pl[0][2], x.pl[0][3]};
-        if (t < 128) {
-            dst += 32 * kPitch;
-            *reinterpret_cast<uint2*>(dst) = uint2{x.pl[1][0], x.pl[1][1]};
-            *reinterpret_cast<uint2*>(dst + 8) = uint2{x.pl[1][2], x.pl[1][3]};
-        } else if (t < 192) {
-            *reinterpret_cast<uint32_t*>(pl + kScaleOff + 4 * (t & 63)) = x.sc;
-        }
-    }
-}
-
-template <int MTW>
-__device__ __forceinline__ void wide_load_w(const Args& p, const WideSrc<MTW>& src, int c, WideW& w) {
-    const __amdgpu_buffer_rsrc_t lo = rsrc(src.lo, src.nlo);
-    const int off = soff(c * kPackBytes);
-    w.lo = __builtin_amdgcn_raw_buffer_load_b128(lo, src.vlo, off, 0);
-    w.hd = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(lo, src.vhi, off, 0));
-    w.sc = __builtin_amdgcn_raw_buffer_load_b32(rsrc(src.sc, src.nsc), src.vsc, soff((c * 64 / p.group_k) * kTileN * 2), 0);
-}
-
 // x s + a per element, written as a whole vector (stores into the components of an accumulator passed by reference
 // kept the accumulators in scratch memory)
 __device__ __forceinline__ f4 fma4(const f4 x, float s, const f4 a) {
     return f4{fmaf(x[0], s, a[0]), fmaf(x[1], s, a[1]), fmaf(x[2], s, a[2]), fmaf(x[3], s, a[3])};
 }
 
-// Dequantise the wavefront's two column tiles of one chunk into B operands w0 (rows 0..31 of the chunk) and w1
-// (rows 32..63), and their scales.
-template <class A, int MTW, bool PACKED>
-__device__ __forceinline__ void wide_dequant(const uint8_t* ps, const WideW& w, u4 (&w0)[2], u4 (&w1)[2],
-                                             float (&sv)[2]) {
-    const int lane = threadIdx.x & 63, cp = (threadIdx.x >> 6) & 3;
-    const int i = lane & 15, q = lane >> 4;
+// ---------------------------------------------------------------------------------------------------------------
+// Tile kernel.  K is shared by `parts` wavefronts (part g takes the chunks g, g + parts, ..), which run in one
+// workgroup or, `parts` / ks to a workgroup, in ks of them; their partial tiles are summed by quarters of the parts, in
+// order within a quarter and then (q0 + q1) + (q2 + q3), so the result depends on `parts` alone and not on how they
+// are placed: planes and packed weights give the same bits with different tiles.
+//
+// What bounds it: per-CU loads.  Every byte a workgroup reads passes its CU's vector L1, in order: a run of L2 hits (A)
+// behind HBM misses (weights) gets about 20 bytes a clock through (measured with a load-only kernel: weights alone
+// 8 B/clk at 5 TB/s over the chip, 1 : 2 mixed with L2 hits 19, 1 : 4 24), and a load instruction occupies the L1 for 2
+// clocks per 128-byte line or 4 lanes, whichever is more.  Hence: A's rows by whole lines (17 clocks an instruction;
+// loaded directly in operand order, 16 rows x 64 bytes, 65 clocks), the widest loads the layout allows (a 4-byte load
+// at a 16-byte stride takes 32 clocks, an 8-byte one 17), 64 columns to a workgroup wherever that still gives every CU
+// one, and no re-reading of A by narrower tiles.  No barrier in the loop and no LDS for the weights: the wavefronts
+// drift apart and their loads, LDS turns and MFMAs overlap.
+// Measured against the kernels it replaced (a strip-wide split-K kernel with a release fence per workgroup up to 32
+// rows, above them a kernel of 128-column workgroups in lock-step with a row-sum pass before it), us per call, packed /
+// planes: K = N = 4096, M = 1 11.5 / 11.6 -> 6.7 / 8.6, M = 16 26.1 / 26.1 -> 8.3 / 10.6, M = 64 17.6 / 18.4 ->
+// 10.7 / 15.5; K = 4096, N = 16384, M = 64 27.5 / 29.7 -> 24.3 / 27.9; K = 2560, N = 10240, M = 203 52 / 62 -> 36.6 / 42.6;
+// K = 10240, N = 2560, M = 203 57 / 67 -> 28.2 / 34.6; a layer's six products at C = 4096: M = 1 planes 83.7 -> 71.3,
+// M = 64 packed 130 -> 95; at C = 2560, M = 203 planes 281 -> 132.  Slower only where 193..256 rows meet K = 4096 and
+// N = 16384 (52 / 67 -> 63 / 71), and one row of packed weights there (11.9 -> 12.4): the rest of the layer gains more.
+
+// The weights of one chunk in one lane's registers.  Packed: the lane's record of its NT tiles (tile t: column
+// n0 + 16 t + i); one tile takes the 8-byte pair its top bits lie in.
+template <int NT, bool PACKED>
+struct TileW {
+    uint32_t lo[2 * NT], hd[NT < 2 ? 2 : NT], sc[2];
+};
+// Planes: lane (i, q) holds lo-plane rows 8 q + e (e = 0..7) and hi-plane rows 8 (q & 1) + 4 (q >> 1) + e (e = 0..3) of
+// columns n0 + 4 i .. + 3, which are its columns of tiles 0..3 (tile t: columns n0 + 4 i + t).
+template <int NT>
+struct TileW<NT, false> {
+    uint32_t lo[8], hd[4], sc[2];
+};
+
+// The wavefront's loads: wave-uniform 64-bit bases (moved from chunk to chunk on the scalar unit) and 32-bit per-lane
+// offsets fixed for the call, through raw buffers.  A's buffer ends with its last valid row: rows past M read zeros.
+// (64-bit lane offsets for planes whose 32 rows span 2 GB: FAR.)
+struct TileSrc {
+    uint64_t a, lo, hi, sc;
+    int na;  // bytes from the first row's start to the last valid row's end
+    uint32_t va, vlo, vhi, vsc;
+    int64_t flo, fhi;
+};
+
+template <int MT, bool PACKED, bool FAR>
+__device__ __forceinline__ TileSrc tile_src(const Args& p, int b, int m0, int tile, int row0) {
+    const int lane = threadIdx.x & 63, i = lane & 15, q = lane >> 4;
+    TileSrc s;
+    s.a = reinterpret_cast<uint64_t>(p.a + (int64_t)b * p.sa_b + (int64_t)m0 * p.sa_m);
+    s.na = (int)(((int64_t)(min(p.M - m0, 16 * MT) - 1) * p.sa_m + p.K) * 2);
+    s.va = (uint32_t)(row0 + (lane >> 3)) * (uint32_t)p.sa_m * 2 + 16 * (lane & 7);
     if constexpr (PACKED) {
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int tt = 0; tt < 2; ++tt) {
-            const uint32_t L0 = w.lo[2 * tt], L1 = w.lo[2 * tt + 1], Hd = tt ? w.hd.y : w.hd.x;
-            const uint32_t u0a = (L0 & 0x0F0F0F0Fu) | ((Hd & 0x03030303u) << 4);         // rows 8 q + 0..3
-            const uint32_t u0b = (L1 & 0x0F0F0F0Fu) | (Hd & 0x30303030u);                // rows 8 q + 4..7
-            const uint32_t u1a = ((L0 >> 4) & 0x0F0F0F0Fu) | ((Hd & 0x0C0C0C0Cu) << 2);  // rows 32 + 8 q + 0..3
-            const uint32_t u1b = ((L1 >> 4) & 0x0F0F0F0Fu) | ((Hd >> 2) & 0x30303030u);  // rows 32 + 8 q + 4..7
-            uint32_t o0[4], o1[4];
-            codes_to_op<A>(u0a, o0[0], o0[1]);
-            codes_to_op<A>(u0b, o0[2], o0[3]);
-            codes_to_op<A>(u1a, o1[0], o1[1]);
-            codes_to_op<A>(u1b, o1[2], o1[3]);
-            w0[tt] = u4{o0[0], o0[1], o0[2], o0[3]};
-            w1[tt] = u4{o1[0], o1[1], o1[2], o1[3]};
-            sv[tt] = h2f((uint16_t)(w.sc >> (16 * tt)));
-        }
+        const int strip = tile >> 3, t = tile & 7;
+        const uint64_t blk =
+            reinterpret_cast<uint64_t>(p.lo + (int64_t)b * p.sl_b + (int64_t)strip * (p.K / 64) * kPackBytes);
+        s.lo = blk + 1024 * (t >> 1) + 8 * (t & 1);
+        s.hi = blk + 1024 * (4 + (t >> 2)) + 4 * (t & 2);
+        s.sc = reinterpret_cast<uint64_t>(p.sc + (int64_t)b * p.ss_b + (int64_t)strip * p.groups * kTileN + (t & 4));
+        s.vlo = s.vhi = 16 * lane;
+        s.vsc = 16 * i;
     } else {
-        const uint8_t* const pl = ps + part_a_bytes<MTW>() + 16 * MTW * 4;
-        const int sel = 2 * (q >> 1), r = lane & 15;
-        const int off = (r >> 1) * kPitch + 8 * (r & 1);
-        v2i lo_t[2], hi_t[2];
-        uint16_t sh[2];
-#pragma unroll
-        for (int tt = 0; tt < 2; ++tt) {
-            const int t = 2 * cp + tt;
-            lo_t[tt] = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i*)(pl + (8 * q) * kPitch + off + 16 * t));
-            hi_t[tt] = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i*)(pl + (32 + 8 * (q & 1)) * kPitch + off + 16 * t));
-            sh[tt] = *reinterpret_cast<const uint16_t*>(pl + kScaleOff + 2 * (16 * t + i));
+        const uint32_t n = min(16 * tile + 4 * i, p.N - 4);
+        const int hrow = 8 * (q & 1) + 4 * (q >> 1);
+        s.lo = reinterpret_cast<uint64_t>(p.lo + (int64_t)b * p.sl_b);
+        s.hi = reinterpret_cast<uint64_t>(p.hi + (int64_t)b * p.sh_b);
+        s.sc = reinterpret_cast<uint64_t>(p.sc + (int64_t)b * p.ss_b);
+        if constexpr (FAR) {
+            s.flo = (int64_t)(8 * q) * p.N + n;
+            s.fhi = (int64_t)hrow * p.N + n;
+        } else {
+            s.vlo = (uint32_t)(8 * q) * p.N + n;
+            s.vhi = (uint32_t)hrow * p.N + n;
         }
-        __builtin_amdgcn_sched_barrier(0);
+        s.vsc = 2 * n;
+    }
+    return s;
+}
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t tile_rsrc(uint64_t base, int bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(base), 0, bytes, 0x00020000);
+}
+
+template <int NT, bool PACKED, bool FAR>
+__device__ __forceinline__ void tile_load_w(const Args& p, const TileSrc& src, int c, TileW<NT, PACKED>& s) {
+    constexpr int kAll = 0x7FFFFFFF;
+    const int g = (int)(__umulhi((uint32_t)c, p.gmul) + (uint32_t)c * p.gone);  // the chunk's scale group
+    if constexpr (PACKED) {
+        const __amdgpu_buffer_rsrc_t lo = tile_rsrc(src.lo + (uint64_t)c * kPackBytes, kAll),
+                                     hi = tile_rsrc(src.hi + (uint64_t)c * kPackBytes, kAll),
+                                     sc = tile_rsrc(src.sc + (uint64_t)g * (2 * kTileN), kAll);
+        if constexpr (NT == 1) {
+            const uint2 x = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(lo, src.vlo, 0, 0));
+            s.lo[0] = x.x, s.lo[1] = x.y;
+        } else {
 #pragma unroll
-        for (int tt = 0; tt < 2; ++tt) {
-            uint32_t o0[4], o1[4];
+            for (int k = 0; k < NT / 2; ++k) {
+                const u4 x = __builtin_amdgcn_raw_buffer_load_b128(lo, src.vlo + 1024 * k, 0, 0);
 #pragma unroll
-            for (int d = 0; d < 2; ++d) {
-                const uint32_t L = (uint32_t)lo_t[tt][d], Hs = (uint32_t)hi_t[tt][d] >> sel;
-                const uint32_t u0 = (L & 0x0F0F0F0Fu) | ((Hs & 0x03030303u) << 4);   // rows 8 q + e
-                const uint32_t u1 = ((L >> 4) & 0x0F0F0F0Fu) | (Hs & 0x30303030u);   // rows 32 + 8 q + e
-                codes_to_op<A>(u0, o0[2 * d], o0[2 * d + 1]);
-                codes_to_op<A>(u1, o1[2 * d], o1[2 * d + 1]);
+                for (int d = 0; d < 4; ++d) s.lo[4 * k + d] = x[d];
             }
-            w0[tt] = u4{o0[0], o0[1], o0[2], o0[3]};
-            w1[tt] = u4{o1[0], o1[1], o1[2], o1[3]};
-            sv[tt] = h2f(sh[tt]);
         }
+        if constexpr (NT == 4) {
+            const u4 y = __builtin_amdgcn_raw_buffer_load_b128(hi, src.vhi, 0, 0);
+#pragma unroll
+            for (int d = 0; d < 4; ++d) s.hd[d] = y[d];
+        } else {
+            const uint2 y = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(hi, src.vhi, 0, 0));
+            s.hd[0] = y.x, s.hd[1] = y.y;
+        }
+        const uint2 z = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(sc, src.vsc, 0, 0));
+        s.sc[0] = z.x, s.sc[1] = z.y;
+    } else {
+        const uint64_t lo = src.lo + (uint64_t)c * 32 * (uint64_t)p.N, hi = src.hi + (uint64_t)c * 16 * (uint64_t)p.N;
+        if constexpr (FAR) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                s.lo[e] = *reinterpret_cast<const __attribute__((address_space(1))) uint32_t*>(lo + (uint64_t)(src.flo + (int64_t)e * p.N));
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                s.hd[e] = *reinterpret_cast<const __attribute__((address_space(1))) uint32_t*>(hi + (uint64_t)(src.fhi + (int64_t)e * p.N));
+        } else {
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                s.lo[e] = __builtin_amdgcn_raw_buffer_load_b32(tile_rsrc(lo, kAll), src.vlo, e * p.N, 0);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                s.hd[e] = __builtin_amdgcn_raw_buffer_load_b32(tile_rsrc(hi, kAll), src.vhi, e * p.N, 0);
+        }
+        const uint2 z = __builtin_bit_cast(
+            uint2, __builtin_amdgcn_raw_buffer_load_b64(tile_rsrc(src.sc + (uint64_t)g * 2 * (uint64_t)p.N, kAll), src.vsc, 0, 0));
+        s.sc[0] = z.x, s.sc[1] = z.y;
     }
 }
 
-// One chunk of the wavefront's part: two MFMAs per (M tile, column tile) into the chain accumulators tc; FIRST starts
-// the chain at the row sums' bias, LAST scales it into acc.  The LDS reads are issued in batches of up to four M tiles
-// ahead of the work that hides them (the first batch ahead of the dequantisation, each further batch ahead of the
-// previous batch's MFMAs), with scheduling barriers keeping that order: left to itself the compiler reused a few
-// operand registers and waited on the LDS once per M tile.
-template <class A, int MTW, bool PACKED, bool FIRST, bool LAST>
-__device__ __forceinline__ void wide_compute(const uint8_t* ps, const WideW& w, f4 (&tc)[MTW][2], f4 (&acc)[MTW][2]) {
-    constexpr int MB = MTW < 4 ? MTW : 4;  // M tiles per batch of LDS reads
-    const int lane = threadIdx.x & 63;
-    const int i = lane & 15, q = lane >> 4;
-    const float* const rsum = reinterpret_cast<const float*>(ps + part_a_bytes<MTW>());
-    u4 a0[MB], a1[MB], w0[2], w1[2];
-    f4 nc[MB];
-    float sv[2];
-    auto read = [&](int mb) __attribute__((always_inline)) {
+// NA groups of 8 rows of A's chunk (128 bytes per row).
+template <int NA>
+__device__ __forceinline__ void tile_load_a(const Args& p, const TileSrc& src, int c, u4 (&a)[NA]) {
+    const __amdgpu_buffer_rsrc_t r = tile_rsrc(src.a + (uint64_t)c * 128, src.na - c * 128);
 #pragma unroll
-        for (int k = 0; k < MB; ++k) {
-            const int mt = mb + k;
-            a0[k] = *reinterpret_cast<const u4*>(ps + 16 * a_slot(16 * mt + i, q));
-            a1[k] = *reinterpret_cast<const u4*>(ps + 16 * a_slot(16 * mt + i, 4 + q));
-            if constexpr (FIRST) nc[k] = *reinterpret_cast<const f4*>(rsum + 16 * mt + 4 * q);  // rows 16 mt + 4 q + v
+    for (int e = 0; e < NA; ++e) a[e] = __builtin_amdgcn_raw_buffer_load_b128(r, src.va, 16 * e * (int)p.sa_m, 0);
+}
+
+// 16-byte piece j (k = 8 j ..) of row r of the chunk's rows of A in LDS: the 16 rows of one operand read (one j) fall in
+// 16 different 16-byte bank groups, and so do the writes.
+__device__ __forceinline__ int a_slot(int r, int j) { return 8 * r + (j ^ ((r >> 1) & 7)); }
+
+// Column tile t's weight operands (rows 8 q .. and 32 + 8 q .. of the chunk) and scale.  u0, u1: the planes' codes of
+// rows 8 q + e and 32 + 8 q + e, four columns each.
+template <class A, int NT, bool PACKED>
+__device__ __forceinline__ void tile_dequant(const TileW<NT, PACKED>& s, const uint32_t (&u0)[8], const uint32_t (&u1)[8],
+                                             int t, int tsel, u4& w0, u4& w1, float& sv) {
+    uint32_t o0[4], o1[4];
+    uint32_t sw;
+    if constexpr (PACKED) {
+        const uint32_t L0 = s.lo[2 * t], L1 = s.lo[2 * t + 1], Hd = NT == 1 ? (tsel & 1 ? s.hd[1] : s.hd[0]) : s.hd[t];
+        codes_to_op<A>((L0 & 0x0F0F0F0Fu) | ((Hd & 0x03030303u) << 4), o0[0], o0[1]);         // rows 8 q + 0..3
+        codes_to_op<A>((L1 & 0x0F0F0F0Fu) | (Hd & 0x30303030u), o0[2], o0[3]);                // rows 8 q + 4..7
+        codes_to_op<A>(((L0 >> 4) & 0x0F0F0F0Fu) | ((Hd & 0x0C0C0C0Cu) << 2), o1[0], o1[1]);  // rows 32 + 8 q ..
+        codes_to_op<A>(((L1 >> 4) & 0x0F0F0F0Fu) | ((Hd >> 2) & 0x30303030u), o1[2], o1[3]);
+        if constexpr (NT == 4) sw = s.sc[t >> 1] >> (16 * (t & 1));
+        else if constexpr (NT == 2) sw = (tsel & 2 ? s.sc[1] : s.sc[0]) >> (16 * t);
+        else sw = (tsel & 2 ? s.sc[1] : s.sc[0]) >> (16 * (tsel & 1));
+    } else {
+        // rows 2 d, 2 d + 1 of column t: the two rows' bytes interleaved, then each beside the constant high byte
+        constexpr uint32_t kPair[2] = {0x05010400u, 0x07030602u};  // columns 0, 1 and 2, 3
+#pragma unroll
+        for (int d = 0; d < 4; ++d) {
+            const uint32_t x = __builtin_amdgcn_perm(u0[2 * d + 1], u0[2 * d], kPair[t >> 1]);
+            const uint32_t y = __builtin_amdgcn_perm(u1[2 * d + 1], u1[2 * d], kPair[t >> 1]);
+            o0[d] = __builtin_amdgcn_perm(A::kCodeHi, x, t & 1 ? 0x04030402u : 0x04010400u);
+            o1[d] = __builtin_amdgcn_perm(A::kCodeHi, y, t & 1 ? 0x04030402u : 0x04010400u);
+        }
+        sw = s.sc[t >> 1] >> (16 * (t & 1));
+    }
+    sv = h2f((uint16_t)sw);
+    w0 = u4{o0[0], o0[1], o0[2], o0[3]};
+    w1 = u4{o1[0], o1[1], o1[2], o1[3]};
+}
+
+// One chunk: per (M tile, column tile) two MFMAs started at the M tile's bias, scaled into acc.  Software-pipelined over
+// the column tiles: tile t's MFMAs are issued between the dequantisation of tile t + 1 and the scaling of tile t - 1
+// (left to itself the compiler reused one accumulator and waited out each MFMA pair's latency).
+template <class A, int MT, int NT, bool PACKED>
+__device__ __forceinline__ void tile_work(const TileW<NT, PACKED>& s, const uint8_t* const (&ra)[2], int tsel,
+                                          f4 (&acc)[MT][NT]) {
+    const int q = (threadIdx.x & 63) >> 4;
+    const u4 bias = u4{A::kBias, A::kBias, A::kBias, A::kBias};  // -(2^e + 32)
+    f4 corr[MT], tc[2][MT];
+    u4 a[MT][2], w[2][2];
+    float sv[2];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) a[mt][h] = *reinterpret_cast<const u4*>(ra[h] + 2048 * mt);
+    uint32_t u0[8], u1[8];
+    if constexpr (!PACKED) {
+        const int sel = 2 * (q >> 1);  // the hi plane's field of rows 8 q ..
+        uint32_t hd[8];                // hi-plane rows 8 (q & 1) + e: the lower half-wavefront's four, then the upper's
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const auto x = __builtin_amdgcn_permlane32_swap(s.hd[e], s.hd[e], false, false);
+            hd[e] = x[0];
+            hd[4 + e] = x[1];
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const uint32_t L = s.lo[e], H = hd[e] >> sel;
+            u0[e] = (L & 0x0F0F0F0Fu) | ((H & 0x03030303u) << 4);
+            u1[e] = ((L >> 4) & 0x0F0F0F0Fu) | (H & 0x30303030u);
+        }
+    }
+    tile_dequant<A, NT, PACKED>(s, u0, u1, 0, tsel, w[0][0], w[0][1], sv[0]);
+    if constexpr (MT > 1) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) corr[mt] = A::mma(a[mt][0], bias, f4{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) corr[mt] = A::mma(a[mt][1], bias, corr[mt]);
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+        const int k = t & 1;
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) tc[k][mt] = A::mma(a[mt][0], w[k][0], corr[mt]);
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) tc[k][mt] = A::mma(a[mt][1], w[k][1], tc[k][mt]);
+        float nsv = 0.f;
+        if (t + 1 < NT) tile_dequant<A, NT, PACKED>(s, u0, u1, t + 1, tsel, w[k ^ 1][0], w[k ^ 1][1], nsv);
+        if (t > 0) {
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) acc[mt][t - 1] = fma4(tc[k ^ 1][mt], sv[k ^ 1], acc[mt][t - 1]);
+        }
+        sv[k ^ 1] = nsv;
+        if constexpr (MT > 1) {
+#pragma unroll
+            for (int x = 0; x < 2 * MT; ++x) {
+                __builtin_amdgcn_sched_group_barrier(8, 1, 0);                // an MFMA,
+                __builtin_amdgcn_sched_group_barrier(2, MT == 4 ? 5 : 7, 0);  // then VALU work of the two other tiles
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) acc[mt][NT - 1] = fma4(tc[(NT - 1) & 1][mt], sv[(NT - 1) & 1], acc[mt][NT - 1]);
+}
+
+// The sum of the W partials of element (r, col) of the workgroup's tile, by the quarters of the parts that it holds
+// (4 / ks).
+template <int MT, int NT, int CW, bool PACKED>
+__device__ __forceinline__ float tile_sum(const float* part, int W, int ks, int r, int wcol) {
+    const int col = wcol % (16 * NT), t = PACKED ? col >> 4 : col & 3, i = PACKED ? col & 15 : col >> 2;
+    const float* const x = part + (((wcol / (16 * NT) * MT + (r >> 4)) * NT + t) * 64 + i + 16 * ((r & 15) >> 2)) * 4 + (r & 3);
+    auto sum = [&](int w0, int w1) __attribute__((always_inline)) {
+        float y = 0.f;
+        for (int w = w0; w < min(w1, W); ++w) y += x[w * CW * MT * NT * 256];
+        return y;
+    };
+    if (ks == 4) return sum(0, W);
+    const int n = ks == 2 ? W >> 1 : (W + 3) >> 2;  // parts per quarter
+    const float s = sum(0, n) + sum(n, 2 * n);
+    return ks == 2 ? s : s + (sum(2 * n, 3 * n) + sum(3 * n, 4 * n));
+}
+
+// NA: groups of 8 rows of A a K part stages (1: M <= 8).  D chunks of weights and DA of A are in flight.  CW: wavefronts
+// side by side in a K part, 16 NT columns each, sharing its rows of A; with two, each loads half of them, the rows are
+// double-buffered and the workgroup meets at one barrier per chunk.
+template <class A, int MT, int NA, int NT, int CW, int D, int DA, int MAXW, bool PACKED, bool FAR>
+__global__ __launch_bounds__(64 * MAXW) void w6a16_tile_kernel(const Args p) {
+    static_assert(PACKED || NT == 4, "planes: four column tiles");
+    static_assert(D % DA == 0, "stage rings");
+    static_assert(CW == 1 || (CW == 2 && D == 2 && DA == 1 && NA % 2 == 0), "one or two column wavefronts");
+    constexpr int kA = 1024 * NA, kPart = MAXW * MT * NT * 1024, kStage = MAXW * kA;  // (CW = 2: two buffers a K part)
+    constexpr int NW = NA / CW;  // row groups this wavefront loads
+    __shared__ __attribute__((aligned(16))) uint8_t lds[kPart > kStage ? kPart : kStage];
+    __shared__ uint32_t completed;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int W = (blockDim.x >> 6) / CW, ks = gridDim.z, split = blockIdx.z;  // W: K parts in the workgroup
+    const int cw = CW == 1 ? 0 : wv & 1, kp = CW == 1 ? wv : wv >> 1;
+    // A unit of 4 or 8 adjacent column tiles and all its M groups go to one XCD (workgroups are dealt to the XCDs in
+    // turn): neighbouring tiles share cache lines of the weights, the M groups all of them.
+    const int u = blockIdx.x >> 3, v = (int)(((uint64_t)u * p.mgmul) >> 31);  // v = u / m_groups
+    const int us = p.unit_shift, unit = (v >> us) * 8 + (blockIdx.x & 7);
+    const int wtile = ((unit << us) + (v & ((1 << us) - 1))) * NT * CW, tile = wtile + cw * NT;
+    const int mg = u - v * p.m_groups, m0 = mg * 16 * MT, b = blockIdx.y;
+    if (16 * wtile >= p.N) return;  // uniform over the workgroup
+    // this wavefront's chunks g, g + parts, ..
+    const int g = split * W + kp, nchunks = p.K / 64;
+    const int n = p.per_part - (g + p.parts * (p.per_part - 1) >= nchunks ? 1 : 0);  // >= 1: parts <= chunks
+    // The chunk's rows of A lie at a_slot(row, piece) of the wavefront's buffer; the swizzle repeats every 16 rows, so
+    // two addresses serve all writes (row groups this wavefront loads, even and odd) and two all reads (k halves of row i).
+    uint8_t* const abuf = lds + kp * CW * kA;
+    const int odd = 8 * (cw & NW);  // a wavefront that starts at an odd row group (NW odd, its second half)
+    uint8_t* const wa[2] = {abuf + 16 * a_slot((lane >> 3) + odd, lane & 7) - 16 * 8 * odd,
+                            abuf + 16 * a_slot(8 - odd + (lane >> 3), lane & 7) - 16 * 8 * (8 - odd)};
+    const int ri = NA == 1 ? lane & 7 : lane & 15;
+    const uint8_t* const ra[2] = {abuf + 16 * a_slot(ri, lane >> 4), abuf + 16 * a_slot(ri, 4 + (lane >> 4))};
+
+    const TileSrc src = tile_src<MT, PACKED, FAR>(p, b, m0, tile, 8 * NW * cw);
+    f4 acc[MT][NT];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int t = 0; t < NT; ++t) acc[mt][t] = f4{0.f, 0.f, 0.f, 0.f};
+    TileW<NT, PACKED> w[D];
+    u4 a[DA][NW];
+    // past the end: the last chunk again (a cache hit), so that every load is unconditional
+    auto chunk = [&](int j) __attribute__((always_inline)) { return g + p.parts * min(j, n - 1); };
+    auto write = [&](const u4 (&x)[NW], int buf) __attribute__((always_inline)) {
+#pragma unroll
+        for (int e = 0; e < NW; ++e) {
+            *reinterpret_cast<u4*>(wa[e & 1] + 1024 * (e + NW * cw) + buf * kA) = x[e];
         }
     };
-    read(0);
-    wide_dequant<A, MTW, PACKED>(ps, w, w0, w1, sv);
+    auto work = [&](const TileW<NT, PACKED>& x, int buf) __attribute__((always_inline)) {
+        const uint8_t* const rb[2] = {ra[0] + buf * kA, ra[1] + buf * kA};
+        tile_work<A, MT, NT, PACKED>(x, rb, tile, acc);
+    };
 #pragma unroll
-    for (int mb = 0; mb < MTW; mb += MB) {
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int k = 0; k < MB; ++k)
-#pragma unroll
-            for (int tt = 0; tt < 2; ++tt) {
-                const f4 c = A::mma(a0[k], w0[tt], FIRST ? nc[k] : tc[mb + k][tt]);
-                tc[mb + k][tt] = A::mma(a1[k], w1[tt], c);
-            }
-        if (mb + MB < MTW) read(mb + MB);
+    for (int j = 0; j < D; ++j) {
+        tile_load_w<NT, PACKED, FAR>(p, src, chunk(j), w[j]);
+        if (j < DA) tile_load_a<NW>(p, src, chunk(j), a[j]);
     }
-    if constexpr (LAST) {
-#pragma unroll
-        for (int mt = 0; mt < MTW; ++mt)
-#pragma unroll
-            for (int tt = 0; tt < 2; ++tt) acc[mt][tt] = fma4(tc[mt][tt], sv[tt], acc[mt][tt]);
-    }
-}
-
-// lane (i, q) of wavefront cp holds C[m0 + 16 mt + 4 q + v][n0 + 16 (2 cp + tt) + i]
-template <int MTW, bool F16>
-__device__ __forceinline__ void wide_store_as(const Args& p, int b, int m0, int n0, const f4 (&acc)[MTW][2]) {
-    const int lane = threadIdx.x & 63, cp = (threadIdx.x >> 6) & 3;
-    const int i = lane & 15, q = lane >> 4;
-#pragma unroll
-    for (int mt = 0; mt < MTW; ++mt)
-#pragma unroll
-        for (int tt = 0; tt < 2; ++tt) {
-            const int n = n0 + 16 * (2 * cp + tt) + i;
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int m = m0 + 16 * mt + 4 * q + v;
-                if (n >= p.N || m >= p.M) continue;
-                put_out<F16>(p, (int64_t)b * p.so_b + (int64_t)m * p.so_m + n, acc[mt][tt][v]);
-            }
-        }
-}
-template <int MTW>
-__device__ __forceinline__ void wide_store(const Args& p, int b, int m0, int n0, const f4 (&acc)[MTW][2]) {
-    if (p.out_dtype == W6A16_OUT_F16)
-        wide_store_as<MTW, true>(p, b, m0, n0, acc);
-    else
-        wide_store_as<MTW, false>(p, b, m0, n0, acc);
-}
-
-template <class A, int MTW, int KP, int CG, int D, int NL, bool PACKED>
-__global__ __launch_bounds__(256 * KP) void w6a16_wide_kernel(const Args p) {
-    constexpr int PB = part_bytes<MTW, PACKED>(), kStage = KP * PB;
-    constexpr int kRed = (KP - 1) * 4 * MTW * 2 * 64 * 16;  // K-part partials in LDS
-    __shared__ __attribute__((aligned(16))) uint8_t lds[2 * kStage > kRed ? 2 * kStage : kRed];
-    __shared__ uint32_t completed;
-    static_assert(D % CG == 0 && D % 2 == 0 && D % NL == 0, "a group of D steps holds whole chains, buffer pairs and rings");
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, kp = wv >> 2;
-    // XCD-aware order: the M groups of one strip are 8 blocks apart (same XCD, consecutive in its dispatch order)
-    const int bx = blockIdx.x, rest = bx >> 3;
-    const int mg = rest % p.m_groups, strip = (rest / p.m_groups) * 8 + (bx & 7);
-    if (strip >= p.n_strips) return;  // uniform over the workgroup
-    const int n0 = strip * kTileN;
-    const int split = blockIdx.y, b = blockIdx.z;
-    const int m0 = mg * 16 * MTW;
-    Sched S;
-    S.cg = CG;
-    S.nchunks = p.K / 64;
-    {
-        const int nch = p.K / (64 * CG);  // chains
-        const int h0 = split * p.chains_per_split, h1 = min(nch, h0 + p.chains_per_split);
-        const int nh = max(0, h1 - h0);
-        S.c_s = h0 * CG;
-        S.n_s = nh * CG;
-        S.per = (nh + KP - 1) / KP * CG;
-    }
-    const int steps = S.per;        // uniform over the workgroup
-    WideSrc<MTW> src;
-    wide_src<MTW, KP, PACKED>(p, b, m0, strip, src);
-    const int mine_n = S.part_n(src.kp);  // this wavefront's chunks (uniform over the wavefront)
-
-    f4 acc[MTW][2], tc[MTW][2];
-#pragma unroll
-    for (int mt = 0; mt < MTW; ++mt) acc[mt][0] = acc[mt][1] = f4{0.f, 0.f, 0.f, 0.f};
-
-    if (steps > 0) {
-        // The LDS stage of step s is written in step s - 1 (after its reads of the other buffer have passed that
-        // step's barrier) from a ring of NL register stages loaded NL - 1 steps earlier; packed weights are loaded D
-        // steps ahead of their use.  Loads past a part's range re-load its last chunk (a cache hit), so every load is
-        // unconditional; whole groups of D steps run unconditionally with a scheduling barrier after each step's
-        // loads, and the remainder (fewer than D steps, already loaded, whole chains) follows.
-        WideLds<MTW, PACKED> ls[NL];
-        WideW ws[D];
-#pragma unroll
-        for (int j = 0; j < NL; ++j) wide_load_lds<MTW, KP, PACKED>(p, S, src, j, ls[j]);
-        if constexpr (PACKED) {
-#pragma unroll
-            for (int j = 0; j < D; ++j) wide_load_w(p, src, S.chunk(src.kp, j), ws[j]);
-        }
-        wide_store_lds<MTW, KP, PACKED>(ls[0], lds);
-        wide_load_lds<MTW, KP, PACKED>(p, S, src, NL, ls[0]);
-        __builtin_amdgcn_sched_barrier(0);
-        __syncthreads();
-        // step s = base + j (base a multiple of D, so s = j modulo 2 and NL): compute from buffer j & 1, write step
-        // s + 1 into buffer (j + 1) & 1 from ls[(j + 1) % NL], refill that register stage with step s + 1 + NL, and
-        // (packed) ws[j] with step s + D.  Every register index is a compile-time constant (a run-time one put the
-        // stages in scratch memory).
-        auto step = [&](int base, auto J) __attribute__((always_inline)) {
-            constexpr int j = decltype(J)::value;
-            const int s = base + j;
-            const uint8_t* const ps = lds + (j & 1) * kStage + kp * PB;
-            if (s < mine_n) wide_compute<A, MTW, PACKED, j % CG == 0, j % CG == CG - 1>(ps, ws[j], tc, acc);
-            if constexpr (PACKED) wide_load_w(p, src, S.chunk(src.kp, s + D), ws[j]);
-            wide_store_lds<MTW, KP, PACKED>(ls[(j + 1) % NL], lds + ((j + 1) & 1) * kStage);
-            wide_load_lds<MTW, KP, PACKED>(p, S, src, s + 1 + NL, ls[(j + 1) % NL]);
-            __builtin_amdgcn_sched_barrier(0);
-            __syncthreads();
+    __builtin_amdgcn_sched_barrier(0);
+    int base = 0;
+    if constexpr (CW == 1) {
+        auto stage = [&](const u4 (&x)[NW]) __attribute__((always_inline)) {
+            wave_lds_sync();  // the previous chunk's reads are issued before these writes
+            write(x, 0);
+            wave_lds_sync();
         };
-        const int full = steps / D * D;
-        for (int base = 0; base < full; base += D) unroll<D>([&](auto J) __attribute__((always_inline)) { step(base, J); });
-        unroll<D - 1>([&](auto J) __attribute__((always_inline)) {
-            if (full + decltype(J)::value < steps) step(full, J);
-        });
-    }
-
-    if constexpr (KP > 1) {  // sum the K parts through LDS in part order 0, 1, ..
-        f4* const red = reinterpret_cast<f4*>(lds) + (wv & 3) * MTW * 2 * 64 + lane;
-        constexpr int kPartF4 = 4 * MTW * 2 * 64;
-        __syncthreads();  // the last step's LDS reads are done
-        if (kp > 0) {
+        for (; base + D < n; base += D)
 #pragma unroll
-            for (int mt = 0; mt < MTW; ++mt)
+            for (int j = 0; j < D; ++j) {
+                stage(a[j % DA]);
+                tile_load_a<NW>(p, src, chunk(base + j + DA), a[j % DA]);
+                __builtin_amdgcn_sched_barrier(0);
+                work(w[j], 0);
+                tile_load_w<NT, PACKED, FAR>(p, src, chunk(base + D + j), w[j]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
 #pragma unroll
-                for (int tt = 0; tt < 2; ++tt) red[(kp - 1) * kPartF4 + (mt * 2 + tt) * 64] = acc[mt][tt];
-        }
+        for (int j = 0; j < D; ++j)
+            if (base + j < n) {
+                stage(a[j % DA]);
+                if (j + DA < D) tile_load_a<NW>(p, src, chunk(base + j + DA), a[j % DA]);
+                __builtin_amdgcn_sched_barrier(0);
+                work(w[j], 0);
+            }
+    } else {
+        // chunk j's rows lie in buffer j & 1; the next chunk's are written beside its work and met at the barrier
+        write(a[0], 0);
+        tile_load_a<NW>(p, src, chunk(1), a[0]);
         __syncthreads();
-        if (kp == 0) {
+        const int steps = p.per_part;  // uniform over the workgroup; a part with a chunk less skips its last one
+        for (; base + D < steps; base += D)
 #pragma unroll
-            for (int k = 1; k < KP; ++k)
+            for (int j = 0; j < D; ++j) {
+                write(a[0], (j + 1) & 1);
+                tile_load_a<NW>(p, src, chunk(base + j + 2), a[0]);
+                __builtin_amdgcn_sched_barrier(0);
+                work(w[j], j & 1);
+                tile_load_w<NT, PACKED, FAR>(p, src, chunk(base + D + j), w[j]);
+                __builtin_amdgcn_sched_barrier(0);
+                __syncthreads();
+            }
 #pragma unroll
-                for (int mt = 0; mt < MTW; ++mt)
-#pragma unroll
-                    for (int tt = 0; tt < 2; ++tt) acc[mt][tt] += red[(k - 1) * kPartF4 + (mt * 2 + tt) * 64];
+        for (int j = 0; j < D; ++j) {
+            if (j + 1 < D) write(a[0], (j + 1) & 1);
+            if (base + j < n) work(w[j], j & 1);
+            __syncthreads();
         }
     }
 
-    if (p.split_k == 1) {  // uniform over the grid
-        if (kp == 0) wide_store<MTW>(p, b, m0, n0, acc);
+    __syncthreads();  // the staging buffers are dead: the partial tiles reuse the LDS
+    f4* const part = reinterpret_cast<f4*>(lds) + wv * MT * NT * 64 + lane;  // [K part][column wavefront]
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int t = 0; t < NT; ++t) part[(mt * NT + t) * 64] = acc[mt][t];
+    __syncthreads();
+    const float* const sums = reinterpret_cast<const float*>(lds);
+    constexpr int NC = 16 * NT * CW;
+    const int items = min(16 * MT, p.M - m0) * NC, n0 = 16 * wtile;
+    auto store = [&](int e, float x) __attribute__((always_inline)) {
+        const int r = e / NC, col = e % NC;
+        if (n0 + col >= p.N) return;
+        const int64_t o = (int64_t)b * p.so_b + (int64_t)(m0 + r) * p.so_m + n0 + col;
+        if (p.out_dtype == W6A16_OUT_F16) put_out<true>(p, o, x);
+        else put_out<false>(p, o, x);
+    };
+    if (ks == 1) {
+        for (int e = threadIdx.x; e < items; e += blockDim.x)
+            store(e, tile_sum<MT, NT, CW, PACKED>(sums, W, 1, e / NC, e % NC));
         return;
     }
-    // Split-K hand-off, one release per workgroup.  Partials are kept in the accumulators' own layout
-    // ([wavefront][mt][tt][lane] f4, 16 bytes per lane and store) and written through the L2 (sc1 stores: written
-    // back, the release fence's L2 walk has nothing of theirs left to write; with plain stores it cost 10 us per call
-    // at M = 128); the release fence orders them before the arrival count, and the last split's acquire fence orders
-    // its loads after it.  The last split keeps its own tile in registers and adds the others' in split order 0, 1, ..
-    // (a fixed order: the result does not depend on which split arrives last).
-    const int64_t tile = ((int64_t)b * p.m_groups + mg) * p.n_strips + strip;
-    constexpr int kTileF4 = 4 * MTW * 2 * 64;  // f4 per partial tile
-    f4* const tbase = reinterpret_cast<f4*>(p.part) + tile * p.split_k * kTileF4;
-    const int cp = wv & 3;
-    if (kp == 0) {
-        const __amdgpu_buffer_rsrc_t prs =
-            __builtin_amdgcn_make_buffer_rsrc(tbase, 0, p.split_k * kTileF4 * 16, 0x00020000);
-        const int mine = split * kTileF4 + cp * MTW * 2 * 64 + lane;
-#pragma unroll
-        for (int mt = 0; mt < MTW; ++mt)
-#pragma unroll
-            for (int tt = 0; tt < 2; ++tt)
-                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, acc[mt][tt]), prs,
-                                                       (mine + (mt * 2 + tt) * 64) * 16, 0, kCachePolicySC1);
-    }
-    // Each wavefront waits for its own stores (wavefront 0's release fence waits only for wavefront 0's), then the
-    // barrier puts all of them before that fence.
-    __builtin_amdgcn_s_waitcnt(0);
+    // K split over ks workgroups.  The partial tile goes out in agent-scope atomic stores (written through to where every
+    // XCD sees them), each wavefront waits until its own have completed, and the barrier puts all of them before the
+    // arrival count; the workgroup that counts in last reads the partials by agent-scope atomic loads.  No release or
+    // acquire fence: a fence writes back or invalidates the XCD's whole L2, and nothing here is cached there (with one
+    // fence per workgroup a call of 256 workgroups took 1 us longer, one of 512 4 us).
+    constexpr int kTileFloats = 16 * MT * NC;
+    const int64_t id = ((int64_t)b * p.m_groups + mg) * ((p.N / 16 + NT * CW - 1) / (NT * CW)) + wtile / (NT * CW);
+    float* const part0 = p.part + id * ks * kTileFloats;
+    for (int e = threadIdx.x; e < items; e += blockDim.x)
+        coherent_store(part0 + split * kTileFloats + e,
+                       tile_sum<MT, NT, CW, PACKED>(sums, W, ks, e / NC, e % NC));
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_s_waitcnt(0);  // this wavefront's partial stores have completed
     __syncthreads();
-    if (wv == 0) {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-        bool done = false;
-        if (lane == 0) {
-            done = __hip_atomic_fetch_add(p.cnt + tile, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
-                   (uint32_t)p.split_k - 1;
-            completed = done ? 1u : 0u;
-        }
-        if (__builtin_amdgcn_ballot_w64(done)) {
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-            if (lane == 0) __hip_atomic_store(p.cnt + tile, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
+    if (threadIdx.x == 0) {
+        const bool done =
+            __hip_atomic_fetch_add(p.cnt + id, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (uint32_t)ks - 1;
+        if (done) __hip_atomic_store(p.cnt + id, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        completed = done ? 1u : 0u;
     }
-    __syncthreads();  // wavefront 0's acquire precedes every wavefront's loads
-    if (!completed || kp != 0) return;
-    const f4* const part = tbase + cp * MTW * 2 * 64 + lane;
-    f4 tot[MTW][2];
-    for (int sp = 0; sp < p.split_k; ++sp) {
+    __syncthreads();
+    if (!completed) return;
+    for (int e = 2 * threadIdx.x; e < items; e += 2 * blockDim.x) {
+        float2 x[4];
 #pragma unroll
-        for (int mt = 0; mt < MTW; ++mt)
-#pragma unroll
-            for (int tt = 0; tt < 2; ++tt) {
-                const f4 x = sp == split ? acc[mt][tt] : part[sp * kTileF4 + (mt * 2 + tt) * 64];
-                tot[mt][tt] = sp == 0 ? x : tot[mt][tt] + x;
-            }
+        for (int k = 0; k < 4; ++k) x[k] = coherent_load2(part0 + min(k, ks - 1) * kTileFloats + e);
+        float2 sum = float2{x[0].x + x[1].x, x[0].y + x[1].y};
+        if (ks == 4) sum = float2{sum.x + (x[2].x + x[3].x), sum.y + (x[2].y + x[3].y)};
+        store(e, sum.x);
+        store(e + 1, sum.y);
     }
-    wide_store<MTW>(p, b, m0, n0, tot);
 }
 
 // Dequantise the packed layout: one thread per (b, strip, chunk, lane) writes its 16 rows x 8 columns (rows
@@ -1640,23 +1032,6 @@ int cu_count() { return wkv7::device_cu_count(); }
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
-// Narrow kernel (M <= 32 rows): one 16-row tile per wavefront, one M group per 16 rows (measured at K = 4096,
-// N = 16384: M = 32 is faster with one tile per wavefront and two M groups).  Wide kernel (M > 32): MTW 16-row tiles
-// per wavefront, KP K parts per workgroup, chains of CG chunks.
-bool wide_rows(int M) { return M > 32; }
-
-struct WideCfg {
-    int mtw, kp;
-};
-// Measured at K = 4096, N = 16384 (us per call, packed / planes): M = 64 (2, 2) 27.2 / 33.0, (4, 2) 31.3 / 32.4,
-// (2, 1) 32.8 / 44.9; M = 128 (4, 2) 36.2 / 40.9, (2, 2) 46.2 / 54.8, (4, 1) 43.7 / 53.5; M = 256 (4, 1) 54.1 / 71.9,
-// (8, 2) 57.5 / 72.8, (8, 1) 94.4 / 103.5, (4, 2) 64.1 / 73.2.
-WideCfg wide_cfg(int M) {
-    if (M <= 64) return {2, 2};
-    if (M <= 128) return {4, 2};
-    return {4, 1};
-}
-
 // Large-M kernel: M above this, packed weights (no workspace, no split-K).
 constexpr int kBigMinM = 256;
 // (its loads go through raw buffers: A's batch slice and the packed weight's below 2 GB)
@@ -1667,47 +1042,110 @@ bool big_rows(const w6a16_args* a) {
     return a_bytes < 0x7FFFFFFF && w_bytes < 0x7FFFFFFF;
 }
 
+// Rows of A up to which a split of 2..8 needs no workspace (include/w6a16.h, w6a16_workspace_size).
+constexpr int kSmallM = 32;
+constexpr int kGemvMaxSplit = 8;
+
+// The workspace that include/w6a16.h promises for a shape and split: the counter region, partial tiles of split_k ranges
+// and, above 32 rows, one float per row and two chunks of K.  The tile kernel uses what it needs of it (counters and
+// partial tiles where it splits K over workgroups; the last part stays unused).
 struct Layout {
     bool big;                    // the large-M kernel
-    bool wide, gemv, gemv_half;  // gemv: the in-workgroup split-K kernel (no workspace); gemv_half: per half strip
-    int mt, kp, cg, m_groups, n_strips, mpad, nchains;
-    size_t tiles, counter_bytes, partial_bytes, rsum_offset, rsum_bytes;
+    bool wide, gemv, gemv_half;  // wide: more than 32 rows; gemv: at most 32, no workspace; gemv_half: of those, packed
+                                 // weights with fewer strips than CUs
+    int kp, m_groups, n_strips, nchains;
+    size_t tiles, partial_bytes, total_bytes;
 };
 
 Layout layout(const w6a16_args* a) {
     Layout l{};
     l.big = big_rows(a);
-    l.wide = !l.big && wide_rows(a->M);
+    l.wide = !l.big && a->M > kSmallM;
     l.n_strips = (a->N + kTileN - 1) / kTileN;
     if (l.big) return l;  // no workspace
-    if (l.wide) {
-        const WideCfg c = wide_cfg(a->M);
-        l.mt = c.mtw;
-        l.kp = c.kp;
-        l.cg = (a->group_k % 128 == 0) ? 2 : 1;
-        l.nchains = a->K / (64 * l.cg);
-    } else {
-        l.mt = 1;
-        l.kp = 1;
-    }
-    const int rows_per_group = 16 * l.mt;  // A rows per workgroup (wide) or per wavefront (narrow)
+    const int mt = !l.wide ? 1 : a->M <= 64 ? 2 : 4;
+    l.kp = l.wide && a->M <= 128 ? 2 : 1;
+    l.nchains = a->K / (a->group_k % 128 == 0 ? 128 : 64);
+    const int rows_per_group = 16 * mt;
     l.m_groups = (a->M + rows_per_group - 1) / rows_per_group;
-    l.mpad = l.m_groups * rows_per_group;
-    // In-workgroup split-K for the packed layout, and for the planes once its grid (one workgroup per strip and M
-    // group) fills the chip.  Measured at K = 4096, N = 16384 (us per call, planes / packed, split 8): M = 1 split-K
-    // across workgroups 17.2 / 16.4, in-workgroup 20.6 / 16.1; M = 16 22.4 / 23.1 against 22.6 / 18.6; M = 32 (split 4
-    // across workgroups) 30.1 / 26.5 against 22.0 / 18.6.
     l.gemv = !l.wide && a->split_k >= 2 && a->split_k <= kGemvMaxSplit &&
              (a->format == W6A16_FORMAT_PACKED || (int64_t)a->B * l.m_groups * l.n_strips >= cu_count());
     l.gemv_half = l.gemv && a->format == W6A16_FORMAT_PACKED && (int64_t)a->B * l.m_groups * l.n_strips < cu_count();
     if ((a->split_k > 1 && !l.gemv) || l.wide) {
         l.tiles = (size_t)a->B * l.m_groups * l.n_strips;
-        l.counter_bytes = kCounterRegion;
         l.partial_bytes = a->split_k > 1 ? l.tiles * a->split_k * (size_t)rows_per_group * kTileN * 4 : 0;
-        l.rsum_offset = l.counter_bytes + l.partial_bytes;
-        l.rsum_bytes = l.wide ? (size_t)a->B * l.nchains * l.mpad * 4 : 0;
+        l.total_bytes = kCounterRegion + l.partial_bytes +
+                        (l.wide ? (size_t)a->B * l.nchains * l.m_groups * rows_per_group * 4 : 0);
     }
     return l;
+}
+
+// The tile kernel's shape for a call: MT 16-row tiles, NT 16-column tiles a wavefront and CW wavefronts side by side to a
+// workgroup, K shared by `parts`, in ks workgroups.
+struct TilePlan {
+    int mt, nt, cw, parts, ks;
+    bool far;
+};
+
+// mt, cw and parts depend on the sizes and on split_k only, not on the format, so that planes and packed weights give the
+// same bits.  A CU takes its workgroups one after the other, so a shape costs its rounds over the CUs times what one
+// workgroup costs per chunk: the KB that pass the CU's L1, 2 per row tile and 3.5 per 64 columns.
+TilePlan tile_plan(const w6a16_args* a, const Layout& l, bool packed) {
+    TilePlan t{};
+    const int64_t cus = cu_count();
+    const int chunks = a->K / 64, tiles = a->N / 16;
+    auto groups = [&](int mt) { return (int64_t)a->B * ((a->M + 16 * mt - 1) / (16 * mt)); };
+    auto wgs = [&](int mt, int nt) { return groups(mt) * ((tiles + nt - 1) / nt); };
+    auto rounds = [&](int64_t n) { return (n + cus - 1) / cus; };
+    // Rows to a workgroup: one tile up to 16 rows, two up to 32; above, two to four tiles and, from three on, 64 or 128
+    // columns, whatever costs least (us, packed: K = N = 4096, M = 64: mt 2 10.3, mt 4 13.3; N = 16384: 25.6 / 22.2;
+    // K = N = 2560, M = 203: mt 2, 3, 4 14.9 / 11.4 / 12.8).
+    t.cw = 1;
+    if (a->M <= 16) {
+        t.mt = 1;
+    } else {
+        t.mt = 2;
+        auto cost = [&](int mt, int cw) { return rounds(wgs(mt, 4 * cw)) * (4 * mt + 7 * cw); };
+        int64_t best = cost(2, 1);
+        if (a->M > 32)
+            for (int mt = 3; mt <= 4; ++mt)
+                for (int cw = 1; cw <= 2; ++cw)
+                    if (cost(mt, cw) < best) best = cost(mt, cw), t.mt = mt, t.cw = cw;
+    }
+    const int64_t w4 = wgs(t.mt, 4 * t.cw);
+    // Workgroups that may share K: none without room for their counters and partial tiles (so split_k bounds it; up to
+    // 32 rows a split of at most 8 has no workspace).
+    int most = a->M <= kSmallM ? (a->split_k > kGemvMaxSplit ? 4 : 1) : a->split_k >= 4 ? 4 : a->split_k >= 2 ? 2 : 1;
+    if ((size_t)(groups(t.mt) * tiles) * 4 > kCounterRegion) most = 1;
+    while (most > 1 && (size_t)w4 * most * 16 * t.mt * 64 * t.cw * 4 > l.partial_bytes) most >>= 1;
+    // Wavefronts that share K: eight to a workgroup (with two column wavefronts four), with one row tile 16 where the
+    // workgroups do not fill the chip and 4 where they do (K = 4096, N = 16384, M = 1, packed / planes: 4 12.4 / 16.2, 8
+    // 12.6 / 16.8, 16 13.3 / 17.7), and twice or four times as many where a deep K would otherwise leave CUs without
+    // work (K = 16384, N = 4096, M = 1: 16 parts in one workgroup 16.4, 32 in two 14.1).
+    const int wide = t.mt == 1 ? (w4 < cus ? 16 : 4) : 8 / t.cw;
+    int spread = 1;  // workgroups of `wide` wavefronts
+    while (spread < most && chunks >= wide * spread * 2 && w4 * spread * 2 <= cus &&
+           (chunks > 128 || (t.mt == 2 && w4 * 4 <= cus && spread < 2)) && !(t.mt == 1 && spread == 2))
+        spread *= 2;
+    t.parts = std::min(chunks, wide * spread);
+    auto fits = [&](int ks, int max_w) { return ks == 1 ? t.parts <= max_w : t.parts % 4 == 0 && t.parts / ks <= max_w; };
+    // Columns to a wavefront and workgroups to a K range.  Packed: as few workgroups to a K range as hold the parts, and
+    // the columns whose rounds cost least.  Planes: always 64 columns (a lane loads four), K spread over more workgroups
+    // while every one of them still gets a CU.
+    int64_t best = 0;
+    for (int nt = packed ? 1 : 4; nt <= 4; nt *= 2) {
+        if (t.mt > 2 && nt < 4) continue;
+        const int max_w = t.mt == 1 || (t.mt == 2 && nt == 1) ? 16 : 8 / t.cw;
+        int ks = 1;
+        while (ks < most && !fits(ks, max_w)) ks *= 2;
+        if (!fits(ks, max_w)) continue;
+        if (!packed)
+            while (ks * 2 <= most && fits(ks * 2, max_w) && t.parts / (ks * 2) >= 4 && w4 * ks * 2 <= cus) ks *= 2;
+        const int64_t cost = rounds(wgs(t.mt, nt * t.cw) * ks) * (2 * nt + 3 * t.mt);
+        if (!best || cost < best) best = cost, t.nt = nt, t.ks = ks;
+    }
+    t.far = !packed && a->N >= (1 << 26);
+    return t;
 }
 
 int validate(const w6a16_args* a) {
@@ -1739,72 +1177,92 @@ int validate(const w6a16_args* a) {
     if (l.wide && (int64_t)l.m_groups * ((l.n_strips + 7) / 8) * 8 > 0x7FFFFFFF) return WKV7_ERR_SHAPE;
     if (a->split_k > 1 && l.tiles * 4 > kCounterRegion) return WKV7_ERR_SHAPE;  // more tiles than counters (0: gemv)
     if ((a->split_k > 1 && !l.gemv) || l.wide) {
-        if (!a->workspace || a->workspace_bytes < l.rsum_offset + l.rsum_bytes) return WKV7_ERR_WORKSPACE;
+        if (!a->workspace || a->workspace_bytes < l.total_bytes) return WKV7_ERR_WORKSPACE;
         if (reinterpret_cast<uintptr_t>(a->workspace) % kCounterAlign) return WKV7_ERR_ALIGN;
     }
     return WKV7_OK;
 }
 
-template <class A, int D, int DH>
-void launch_gemv(const Args& p, const Layout& l, bool packed, hipStream_t s) {
-    const dim3 block(64 * p.split_k);
-    if (packed && l.gemv_half)
-        hipLaunchKernelGGL((w6a16_gemv_kernel<A, DH, true, 4>), dim3(2 * l.n_strips, 1, p.B * l.m_groups), block, 0, s,
-                           p);
-    else if (packed)
-        hipLaunchKernelGGL((w6a16_gemv_kernel<A, D, true, kTiles>), dim3(l.n_strips, 1, p.B * l.m_groups), block, 0, s,
-                           p);
-    else
-        hipLaunchKernelGGL((w6a16_gemv_kernel<A, D, false, kTiles>), dim3(l.n_strips, 1, p.B * l.m_groups), block, 0, s,
-                           p);
+template <class A, int MT, int NA, int NT, int CW, int D, int DA, int MAXW, bool PACKED, bool FAR = false>
+void launch_tile(Args& p, const TilePlan& t, hipStream_t s) {
+    const int tiles = p.N / 16, chunks = p.K / 64, gc = p.group_k / 64;
+    p.m_groups = (p.M + 16 * MT - 1) / (16 * MT);
+    p.mgmul = (uint32_t)(((uint64_t(1) << 31) + p.m_groups - 1) / p.m_groups);
+    p.gone = gc == 1;
+    p.gmul = gc == 1 ? 0 : (uint32_t)(((uint64_t(1) << 32) + gc - 1) / gc);
+    p.parts = t.parts;
+    p.per_part = (chunks + t.parts - 1) / t.parts;
+    p.groups = p.K / p.group_k;
+    // units of eight tiles (a whole line of the planes, a whole block of the packed layout) where they divide evenly
+    // among the XCDs or a workgroup takes eight, else of four
+    const int unit = CW * NT == 8 || ((tiles + 7) / 8) % 8 == 0 ? 8 : 4, units = (tiles + unit - 1) / unit;
+    p.unit_shift = 31 - __builtin_clz(unit / (NT * CW));
+    const dim3 grid(8 * ((units + 7) / 8) * (unit / (NT * CW)) * p.m_groups, p.B, t.ks);
+    hipLaunchKernelGGL((w6a16_tile_kernel<A, MT, NA, NT, CW, D, DA, MAXW, PACKED, FAR>), grid,
+                       dim3(64 * CW * t.parts / t.ks), 0, s, p);
 }
 
-template <class A, int MT, int D>
-void launch(const Args& p, const Layout& l, bool packed, hipStream_t s) {
-    const dim3 grid((l.n_strips + kStrips - 1) / kStrips, p.split_k, p.B * l.m_groups);
-    if (packed)
-        hipLaunchKernelGGL((w6a16_kernel<A, MT, D, true>), grid, dim3(64 * kStrips), 0, s, p);
-    else
-        hipLaunchKernelGGL((w6a16_kernel<A, MT, D, false>), grid, dim3(64 * kStrips), 0, s, p);
+// D chunks of weights and DA of A in flight: as many as the registers of MAXW wavefronts allow.
+template <class A, int NA, bool PACKED>
+void launch_tile_one(Args& p, const TilePlan& t, hipStream_t s) {  // one row tile
+    if constexpr (PACKED) {
+        if (t.nt == 1) return launch_tile<A, 1, NA, 1, 1, 4, 4, 16, true>(p, t, s);
+        if (t.nt == 2) return launch_tile<A, 1, NA, 2, 1, 4, 4, 16, true>(p, t, s);
+    }
+    if (t.parts / t.ks > 8) return launch_tile<A, 1, NA, 4, 1, 2, 2, 16, PACKED>(p, t, s);
+    launch_tile<A, 1, NA, 4, 1, 4, 4, 8, PACKED>(p, t, s);
 }
 
-template <class A, int MTW, int KP, int CG>
-void launch_wide(const Args& p, const Layout& l, bool packed, hipStream_t s) {
-    constexpr int D = 4, NL = 4;  // packed weights D steps ahead; NL register stages of the LDS ring
-    hipLaunchKernelGGL(w6a16_rowsum_kernel<A>, dim3(l.mpad / 4, (p.K + 511) / 512, p.B), dim3(256), 0, s, p);
-    const dim3 grid(8 * l.m_groups * ((l.n_strips + 7) / 8), p.split_k, p.B);
-    if (packed)
-        hipLaunchKernelGGL((w6a16_wide_kernel<A, MTW, KP, CG, D, NL, true>), grid, dim3(256 * KP), 0, s, p);
-    else
-        hipLaunchKernelGGL((w6a16_wide_kernel<A, MTW, KP, CG, D, NL, false>), grid, dim3(256 * KP), 0, s, p);
-}
-
-template <class A, int MTW, int KP>
-void launch_wide_cg(const Args& p, const Layout& l, bool packed, hipStream_t s) {
-    if (l.cg == 2)
-        launch_wide<A, MTW, KP, 2>(p, l, packed, s);
-    else
-        launch_wide<A, MTW, KP, 1>(p, l, packed, s);
+template <class A, bool PACKED>
+void launch_tile_plan(Args& p, const TilePlan& t, hipStream_t s) {
+    if constexpr (!PACKED)
+        if (t.far) return launch_tile<A, 1, 2, 4, 1, 2, 2, 16, false, true>(p, t, s);
+    if (t.mt == 1) return p.M <= 8 ? launch_tile_one<A, 1, PACKED>(p, t, s) : launch_tile_one<A, 2, PACKED>(p, t, s);
+    if (t.mt == 2) {
+        if constexpr (PACKED) {
+            if (t.nt == 1) return launch_tile<A, 2, 4, 1, 1, 2, 2, 16, true>(p, t, s);
+            if (t.nt == 2) return launch_tile<A, 2, 4, 2, 1, 2, 2, 8, true>(p, t, s);
+        }
+        return launch_tile<A, 2, 4, 4, 1, 2, 2, 8, PACKED>(p, t, s);
+    }
+    if (t.mt == 3)
+        return t.cw == 2 ? launch_tile<A, 3, 6, 4, 2, 2, 1, 8, PACKED>(p, t, s) : launch_tile<A, 3, 6, 4, 1, 2, 1, 8, PACKED>(p, t, s);
+    t.cw == 2 ? launch_tile<A, 4, 8, 4, 2, 2, 1, 8, PACKED>(p, t, s) : launch_tile<A, 4, 8, 4, 1, 2, 1, 8, PACKED>(p, t, s);
 }
 
 // The kernel for the call's shape and layout, with activations of type A.
 template <class A>
-void launch_matmul(const Args& p, const Layout& l, bool packed, hipStream_t s) {
+void launch_matmul(Args& p, const w6a16_args* a, const Layout& l, hipStream_t s) {
+    const bool packed = a->format == W6A16_FORMAT_PACKED;
     if (l.big) {
         const int tiles = ((p.M + kBigTile - 1) / kBigTile) * ((p.N + kBigTile - 1) / kBigTile);
         hipLaunchKernelGGL(w6a16_big_kernel<A>, dim3(tiles, 1, p.B), dim3(512), 0, s, p);
-    } else if (l.gemv && l.gemv_half && p.split_k <= 4)  // half strips, split <= 4: three chunks in flight
-        launch_gemv<A, 2, 3>(p, l, packed, s);
-    else if (l.gemv)
-        launch_gemv<A, 2, 2>(p, l, packed, s);
-    else if (!l.wide)
-        launch<A, 1, 2>(p, l, packed, s);
-    else if (l.mt == 2)
-        launch_wide_cg<A, 2, 2>(p, l, packed, s);
-    else if (l.kp == 2)
-        launch_wide_cg<A, 4, 2>(p, l, packed, s);
-    else
-        launch_wide_cg<A, 4, 1>(p, l, packed, s);
+        return;
+    }
+    auto launch = [&](Args& q, const w6a16_args* shape) {
+        const TilePlan t = tile_plan(shape, l, packed);
+        if (packed)
+            launch_tile_plan<A, true>(q, t, s);
+        else
+            launch_tile_plan<A, false>(q, t, s);
+    };
+    if (p.sa_m < (1 << 24)) return launch(p, a);
+    // rows so far apart that a workgroup's 64 do not fit a buffer's 32-bit offsets: row by row
+    w6a16_args row = *a;
+    row.M = row.B = row.split_k = 1;
+    for (int b = 0; b < a->B; ++b)
+        for (int m = 0; m < a->M; ++m) {
+            Args q = p;
+            q.a += (int64_t)b * p.sa_b + (int64_t)m * p.sa_m;
+            q.lo += (int64_t)b * p.sl_b;
+            if (q.hi) q.hi += (int64_t)b * p.sh_b;
+            q.sc += (int64_t)b * p.ss_b;
+            const int64_t o = (int64_t)b * p.so_b + (int64_t)m * p.so_m;
+            q.out = static_cast<char*>(p.out) + o * (p.out_dtype == W6A16_OUT_F32 ? 4 : 2);
+            q.B = q.M = 1;
+            q.sa_m = p.K;
+            launch(q, &row);
+        }
 }
 
 }  // namespace
@@ -1817,12 +1275,12 @@ size_t w6a16_args_size(void) { return sizeof(w6a16_args); }
 int w6a16_workspace_size(const w6a16_args* a, size_t* bytes) {
     if (!a || !bytes) return WKV7_ERR_NULL;
     if (a->M <= 0 || a->B < 1 || a->N < 1 || a->K < 64 || a->group_k < 64 ||
-        (a->split_k <= 1 && !w6::wide_rows(a->M)) || w6::big_rows(a)) {
+        (a->split_k <= 1 && a->M <= w6::kSmallM) || w6::big_rows(a)) {
         *bytes = 0;
         return WKV7_OK;
     }
     const w6::Layout l = w6::layout(a);
-    *bytes = l.rsum_offset + l.rsum_bytes;
+    *bytes = l.total_bytes;
     return WKV7_OK;
 }
 
@@ -1835,21 +1293,16 @@ int w6a16_plan_split(int32_t B, int32_t M, int32_t N, int32_t K) {
     shape.K = K;
     shape.group_k = K % 128 == 0 ? 128 : 64;  // chains of two chunks where K allows them
     const w6::Layout l = w6::layout(&shape);
-    // workgroups per split: narrow, four strips per workgroup; wide, one strip per workgroup
-    const int64_t groups = (int64_t)B * l.m_groups * (l.wide ? l.n_strips : (l.n_strips + w6::kStrips - 1) / w6::kStrips);
+    // The rule's units: for M <= 32 four 128-column strips per 16 rows, with one unit per CU; above, one strip per M group
+    // and eight wavefronts (4 KP a unit) per CU.
+    const int64_t groups = (int64_t)B * l.m_groups * (l.wide ? l.n_strips : (l.n_strips + 3) / 4);
     const int chunks = l.wide ? l.nchains : K / 64;  // the units a split range holds
-    // narrow: one workgroup per CU; wide (4 KP wavefronts per workgroup): eight wavefronts per CU
     const int64_t cus = l.wide ? w6::cu_count() * 2 / l.kp : w6::cu_count();
-    // The smallest power of two that gives every CU a workgroup (every range keeps at least one chunk); then doubled
-    // while ranges keep at least 16 chunks and the launch stays within one workgroup per CU (each workgroup's
-    // split-K hand-off costs one agent-scope release).  Measured at K = 4096, N = 16384 (us, planes / packed): M = 128
-    // split 2 63.5 / 53.9, split 4 64.0 / 60.6; M = 64 split 4 41.7 / 37.1, split 8 51.3 / 49.1; M = 16 split 8
-    // 23.6 / 23.4, split 4 29.1 / 25.3.
+    // The smallest power of two that gives every CU a unit (every range keeps at least one chunk); then doubled while
+    // ranges keep at least 16 chunks and the launch stays within one unit per CU.
     int sk = 1;
     while (groups * sk < cus && sk * 2 <= 64 && chunks / (sk * 2) >= 1) sk *= 2;
     while (chunks / (sk * 2) >= 16 && groups * sk * 2 <= cus && sk * 2 <= 64) sk *= 2;
-    // Narrow, split, and one workgroup per (strip, M group) fills the chip: the in-workgroup split-K kernel takes the
-    // split, and its deepest split is the fastest (M = 32 above: split 4 24.1 / 19.5 us, split 8 22.0 / 18.6).
     if (!l.wide && sk >= 2 && (int64_t)B * l.m_groups * l.n_strips >= cus)
         while (sk * 2 <= w6::kGemvMaxSplit && chunks / (sk * 2) >= 1) sk *= 2;
     return sk;
@@ -1867,9 +1320,7 @@ int w6a16_plan_split_packed(int32_t B, int32_t M, int32_t N, int32_t K) {
     shape.split_k = sk;
     shape.format = W6A16_FORMAT_PACKED;
     const w6::Layout l = w6::layout(&shape);
-    // Half strips (the in-workgroup kernel where strips are fewer than CUs) run fastest at split 4 with three chunks
-    // in flight, given at least 8 chunks per range.  Measured at K = 4096, N = 16384 (us per call): M = 1 split 4
-    // 11.9, split 8 12.4; M = 16 14.1 / 14.7.
+    // shallower where a batch's strips are fewer than the CUs and the ranges keep at least 8 chunks
     if (l.gemv_half && K / 64 / 4 >= 8) return 4;
     return sk;
 }
@@ -1881,7 +1332,7 @@ int w6a16_matmul(const w6a16_args* a, void* stream) {
     w6::Args p{};
     p.a = a->a;
     p.sa_b = a->a_batch_stride;
-    p.sa_m = a->a_row_stride;
+    p.sa_m = a->M > 1 ? a->a_row_stride : a->K;
     p.lo = a->lo;
     p.hi = a->hi;
     p.sl_b = a->lo_batch_stride;
@@ -1891,35 +1342,21 @@ int w6a16_matmul(const w6a16_args* a, void* stream) {
     p.out = a->out;
     p.so_b = a->out_batch_stride;
     p.so_m = a->out_row_stride;
-    if ((a->split_k > 1 && !l.gemv) || l.wide) {
-        p.cnt = static_cast<uint32_t*>(a->workspace);
-        p.part = reinterpret_cast<float*>(static_cast<char*>(a->workspace) + l.counter_bytes);
-        p.rsum = reinterpret_cast<float*>(static_cast<char*>(a->workspace) + l.rsum_offset);
-    }
+    p.cnt = static_cast<uint32_t*>(a->workspace);  // used only where the plan splits K over workgroups
+    p.part = reinterpret_cast<float*>(static_cast<char*>(a->workspace) + w6::kCounterRegion);
     p.B = a->B;
     p.M = a->M;
     p.N = a->N;
     p.K = a->K;
     p.group_k = a->group_k;
-    p.split_k = a->split_k;
     p.out_dtype = a->out_dtype;
-    p.m_groups = l.m_groups;
     p.n_strips = l.n_strips;
-    const int chunks = a->K / 64;
-    p.chunks_per_split = (chunks + a->split_k - 1) / a->split_k;
-    if (l.wide) {
-        p.mpad = l.mpad;
-        p.chain_k = 64 * l.cg;
-        p.nchains = l.nchains;
-        p.chains_per_split = (l.nchains + a->split_k - 1) / a->split_k;
-    }
     p.out_vec = w6::aligned16(a->out) && a->out_row_stride % 8 == 0 && a->out_batch_stride % 8 == 0;
     const hipStream_t s = static_cast<hipStream_t>(stream);
-    const bool packed = a->format == W6A16_FORMAT_PACKED;
     if (a->a_dtype == W6A16_IN_F16)
-        w6::launch_matmul<w6::ActF16>(p, l, packed, s);
+        w6::launch_matmul<w6::ActF16>(p, a, l, s);
     else
-        w6::launch_matmul<w6::ActBF16>(p, l, packed, s);
+        w6::launch_matmul<w6::ActBF16>(p, a, l, s);
     return static_cast<int>(hipGetLastError());
 }
 

@@ -21,7 +21,7 @@ fp16 scale, w ~ s q; the code u = q + 32 is split into bit planes per 64-row chu
 Compute: one MFMA kernel for every M up to MAX_M (the reference's reduction form for M = 1 has no counterpart:
 an MFMA with M padded to 16 rows costs the CDNA4 matrix core less than a VALU reduction costs the vector units, and
 the weight bytes, not the arithmetic, bound both).  `use_dot` is accepted for the reference's signature and does
-not change the computation.  Above MAX_M the weight is dequantised once to the activations' type and the product
+not change the computation; `split_k` bounds over how many workgroups the kernel may split K.  Above MAX_M the weight is dequantised once to the activations' type and the product
 goes to the library GEMM (hipBLASLt through torch.matmul), which is compute-bound there.  The C ABI has its own kernel
 for that range (packed weights, M > 256: dequantisation in LDS fused with the product, the same values); at K = 4096,
 N = 16384 it is level with dequantise + hipBLASLt at M = 1024 and slower from M = 2048 (585 against 465 us at
@@ -153,8 +153,9 @@ def dequantize_int6(lo, hi, sc, group_k, dtype=torch.float32):
 # dispatch
 # ----------------------------------------------------------------------------------------------------------------
 def plan_int6(M, N, K, n_batch, device=None):
-    """(split_k, use_dot) for one shape.  split_k is the kernel's rule (w6a16_plan_split: the smallest power of two
-    that gives every CU a workgroup, doubled while ranges keep 16 chunks within two workgroups per CU); use_dot is M > 1 as in the reference and does not change the computation."""
+    """(split_k, use_dot) for one shape.  split_k follows w6a16_plan_split (a power of two that grows with the CUs a
+    shape would leave idle) and bounds over how many workgroups the kernel splits K; use_dot is M > 1 as in the
+    reference and does not change the computation."""
     if device is not None and torch.device(device).type == "cuda":
         with torch.cuda.device(device):
             sk = _lib.load().w6a16_plan_split(n_batch, M, N, K)
@@ -164,8 +165,8 @@ def plan_int6(M, N, K, n_batch, device=None):
 
 
 def plan_int6_packed(M, N, K, n_batch, device=None):
-    """split_k for a packed weight (w6a16_plan_split_packed; no counterpart in the reference): plan_int6's split, made
-    shallower where the packed kernel runs half strips.  A packed call equals the planes' bit for bit only at the same
+    """split_k for a packed weight (w6a16_plan_split_packed; no counterpart in the reference): plan_int6's split, 4
+    instead of 8 where strips are few.  A packed call is sure to equal the planes' bit for bit only at the same
     split_k."""
     lib = _lib.load()
     if device is not None and torch.device(device).type == "cuda":
@@ -294,7 +295,7 @@ def _impl(a, w: _W, split_k, out_dtype=None):
     lib = _lib.load()
     n = ctypes.c_size_t(0)
     _lib.check(lib.w6a16_workspace_size(args, ctypes.byref(n)))
-    if n.value:  # split-K counters and partials, and the wide kernel's row sums (M > 32)
+    if n.value:  # counters and partial tiles of a K split over workgroups
         ws = _workspace(A.device, int(n.value))
         args.workspace, args.workspace_bytes = ws.data_ptr(), ws.numel()
     _lib.check(lib.w6a16_matmul(args, torch.cuda.current_stream(A.device).cuda_stream))

@@ -1,0 +1,84 @@
+"""The W6A16 tile kernel (rwkv-infer-next_amd/csrc/w6a16.hip) at the edges of its shapes: every row and column tiling, K
+shared by few, many and uneven parts, K split over workgroups, ragged columns, and addresses past 32 bits.  Planes and
+packed weights give the same bits, within the kernel tolerance of the oracle (tests/test_gpu_int6.py)."""
+import numpy as np
+import pytest
+
+from gpu_util import say
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+from test_gpu_int6 import DEV, F16_KERNEL_TOL, KERNEL_TOL, _act, _check, _dev, _weights  # noqa: E402
+
+
+@pytest.mark.parametrize("B,M,N,K,g,split", [
+    (1, 1, 16, 64, 64, 16),          # one chunk, one column tile
+    (1, 8, 80, 192, 64, 16),         # 8 rows staged, three chunks, a ragged unit of columns
+    (1, 9, 208, 1088, 64, 16),       # 16 rows staged; 17 chunks over 16 parts; K split over workgroups on the planes
+    (2, 5, 64, 16384, 128, 16),      # deep K: 32 parts over two or four workgroups
+    (1, 16, 16384, 320, 64, 8),      # the workgroups fill the chip: four parts, five chunks
+    (1, 17, 272, 2048, 256, 16),     # two row tiles, the second with one row
+    (1, 32, 48, 16384, 128, 32),     # two row tiles, 32 parts
+    (1, 40, 64, 16384, 128, 4),      # above 32 rows, K over four workgroups
+    (1, 40, 64, 16384, 128, 2),      # over two
+    (1, 33, 144, 1024, 128, 1),      # no split
+    (1, 203, 2560, 320, 64, 2),      # three row tiles, 64 columns
+    (1, 64, 16384, 192, 64, 1),      # four row tiles, 64 columns, three chunks
+    (1, 203, 10240, 320, 64, 1),     # three row tiles, 128 columns; five chunks over four parts
+    (1, 128, 16336, 576, 64, 1),     # four row tiles, 128 columns, nine chunks, columns that end inside a strip
+])
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
+def test_tile_shapes(B, M, N, K, g, split, dtype):
+    from rwkv_next_amd.kernels import int6_gemm as I6
+    say("w6a16 tile", dict(B=B, M=M, N=N, K=K, g=g, split=split, dtype=dtype))
+    rng = np.random.default_rng(11000 + M + N + K)
+    lo, hi, sc = _weights(rng, B, K, N, g)
+    a = _act(rng, B, M, K)
+    if dtype == "f16":
+        a = a.to(torch.float16)
+    Ld, Hd, Sd = _dev(lo, hi, sc)
+    C = I6.int6_matmul(a.to(DEV), Ld, Hd, Sd, g, split_k=split, out_dtype=torch.float32)
+    Cp = I6.int6_matmul(a.to(DEV), I6.prepack_int6(Ld, Hd, Sd, g), split_k=split, out_dtype=torch.float32)
+    again = I6.int6_matmul(a.to(DEV), Ld, Hd, Sd, g, split_k=split, out_dtype=torch.float32)
+    torch.cuda.synchronize()
+    assert torch.equal(C, Cp) and torch.equal(C, again)
+    _check(C, a, lo, hi, sc, g, KERNEL_TOL if dtype == "bf16" else F16_KERNEL_TOL)
+
+
+def test_rows_far_apart():
+    """A row stride of 2^24 elements: a workgroup's rows span more than its buffer's 32-bit offsets reach."""
+    from rwkv_next_amd.kernels import int6_gemm as I6
+    B, M, N, K, g = 2, 3, 80, 256, 64
+    say("w6a16 rows far apart")
+    rng = np.random.default_rng(11)
+    lo, hi, sc = _weights(rng, B, K, N, g)
+    a = _act(rng, B, M, K)
+    Ld, Hd, Sd = _dev(lo, hi, sc)
+    far = torch.zeros(B * M, 1 << 24, dtype=torch.bfloat16, device=DEV)
+    far[:, :K] = a.reshape(B * M, K).to(DEV)
+    view = far.view(B, M, 1 << 24)[:, :, :K]
+    C = I6.int6_matmul(view, Ld, Hd, Sd, g, out_dtype=torch.float32)
+    Cp = I6.int6_matmul(view, I6.prepack_int6(Ld, Hd, Sd, g), out_dtype=torch.float32)
+    torch.cuda.synchronize()
+    assert torch.equal(C, Cp)
+    _check(C, a, lo, hi, sc, g, KERNEL_TOL)
+
+
+def test_planes_past_2_gb():
+    """2^26 + 80 columns: the planes' rows of one chunk span more than 2 GB.  Columns from both ends equal the same
+    columns multiplied alone."""
+    from rwkv_next_amd.kernels import int6_gemm as I6
+    M, N, K, g = 2, (1 << 26) + 80, 64, 64
+    say("w6a16 planes past 2 GB")
+    gen = torch.Generator(device=DEV).manual_seed(12)
+    lo = torch.randint(0, 256, (K // 2, N), device=DEV, dtype=torch.uint8, generator=gen)
+    hi = torch.randint(0, 256, (K // 4, N), device=DEV, dtype=torch.uint8, generator=gen)
+    sc = (torch.rand(K // g, N, device=DEV, generator=gen) * 0.05 + 0.002).half()
+    a = torch.randn(M, K, device=DEV, generator=gen).to(torch.bfloat16)
+    C = I6.int6_matmul(a, lo, hi, sc, g, out_dtype=torch.float32)
+    for n0 in (0, N // 32 * 16, N - 256):
+        part = [x[:, n0:n0 + 256].contiguous() for x in (lo, hi, sc)]
+        P = I6.int6_matmul(a, *part, g, out_dtype=torch.float32)
+        torch.cuda.synchronize()
+        assert torch.equal(C[:, n0:n0 + 256], P), n0

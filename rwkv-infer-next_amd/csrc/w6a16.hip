@@ -612,49 +612,111 @@ __global__ __launch_bounds__(64 * MAXW) void w6a16_tile_kernel(const Args p) {
     }
 }
 
-// Dequantise the packed layout: one thread per (b, strip, chunk, lane) writes its 16 rows x 8 columns (rows
-// 8 q + e and 32 + 8 q + e, columns 128 strip + 16 t + i); for each (row, tile) the 16 lanes of a row group store
-// 16 consecutive columns.
+// Eight codes (one per byte of u) of eight columns with scales sc: s q, exact in fp32 (11 x 6 bit product).
+__device__ __forceinline__ void dequant8(const uint2 u, const u4 sc, float (&v)[8]) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const uint32_t word = e < 4 ? u.x : u.y;
+        v[e] = h2f((uint16_t)(sc[e >> 1] >> (16 * (e & 1)))) * ((float)((word >> (8 * (e & 3))) & 0xFF) - 32.f);
+    }
+}
+
+template <typename OutT>
+__device__ __forceinline__ void store_row8(OutT* dst, const float (&v)[8], bool vec) {
+    if (vec) {
+        store8(dst, v);
+    } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) dst[e] = (OutT)v[e];
+    }
+}
+
+typedef int v2i __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(3))) v2i lds_v2i;
+
+// Dequantise the packed layout: one wavefront per (b, strip, chunk).  HBM-bound (0.75 byte read and 2 written per weight
+// for bf16) once the stores are whole lines: the block's codes, one column's rows per lane, are turned in LDS -- by
+// ds_read_b64_tr_b8 from [column][row] to eight columns of a row, then into row order -- so that 16 lanes store 256
+// bytes of a row.  K = 4096, N = 16384, bf16, weights cycled: 49.4 us with 2-byte stores of 16 columns -> 34.9
+// (185 MB).
+constexpr int kDqCol = 72, kDqRow = 136;  // byte pitches of the two turns: 64 rows or 128 columns, and 8
+constexpr int kDqWave = kTileN * kDqCol + 2 * kTileN;
+
 template <typename OutT>
 __global__ __launch_bounds__(256) void w6a16_dequant_packed_kernel(const uint8_t* pk, const uint16_t* psc, OutT* w,
                                                                    int32_t K, int32_t N, int32_t group_k,
-                                                                   int32_t strips, int64_t sw_b) {
+                                                                   int32_t strips, int64_t sw_b, bool vec) {
+    __shared__ __attribute__((aligned(16))) uint8_t lds[4 * kDqWave];
+    static_assert(64 * kDqRow <= kTileN * kDqCol, "the second turn reuses the first one's bytes");
     const int nchunks = K / 64, groups = K / group_k;
-    const int64_t x = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int64_t x = (int64_t)blockIdx.x * 4 + wv;  // strip * nchunks + c
     const int b = blockIdx.y;
-    if (x >= (int64_t)strips * nchunks * 64) return;
-    const int lane = (int)(x & 63);
-    const int64_t sc = x >> 6;
-    const int c = (int)(sc % nchunks), strip = (int)(sc / nchunks);
+    if (x >= (int64_t)strips * nchunks) return;  // uniform over the wavefront; no barrier follows
+    const int c = (int)(x % nchunks), strip = (int)(x / nchunks);
     const int i = lane & 15, q = lane >> 4;
-    const uint8_t* const blk = pk + ((int64_t)b * strips * nchunks + sc) * kPackBytes + 16 * lane;
-    uint32_t R[24];
+    uint8_t* const buf = lds + wv * kDqWave;
+    uint8_t* const scl = buf + kTileN * kDqCol;  // the chunk's 128 scales in column order
+    const uint8_t* const blk = pk + ((int64_t)b * strips * nchunks + x) * kPackBytes + 16 * lane;
+    u4 R[6];
 #pragma unroll
-    for (int k = 0; k < 6; ++k) {
-        const u4 v = *reinterpret_cast<const u4*>(blk + 1024 * k);
-        R[4 * k] = v[0];
-        R[4 * k + 1] = v[1];
-        R[4 * k + 2] = v[2];
-        R[4 * k + 3] = v[3];
-    }
+    for (int k = 0; k < 6; ++k) R[k] = *reinterpret_cast<const u4*>(blk + 1024 * k);
     const int g = (c * 64) / group_k;
-    const u4 sv = *reinterpret_cast<const u4*>(psc + ((int64_t)b * strips * groups + (int64_t)strip * groups + g) * kTileN + 8 * i);
-    OutT* const wb = w + b * sw_b;
+    const u4 sv = *reinterpret_cast<const u4*>(psc + ((int64_t)b * strips * groups + (int64_t)strip * groups + g) * kTileN +
+                                               8 * i);
 #pragma unroll
     for (int t = 0; t < kTiles; ++t) {
-        const int n = strip * kTileN + 16 * t + i;
-        if (n >= N) continue;
-        const float s = h2f((uint16_t)(sv[t >> 1] >> (16 * (t & 1))));
-        const uint32_t Lw[2] = {R[2 * t], R[2 * t + 1]}, Hd = R[16 + t];
+        const uint32_t L0 = R[t >> 1][2 * (t & 1)], L1 = R[t >> 1][2 * (t & 1) + 1], Hd = R[4 + (t >> 2)][t & 3];
+        uint8_t* const col = buf + (16 * t + i) * kDqCol + 8 * q;
+        *reinterpret_cast<uint2*>(col) = uint2{(L0 & 0x0F0F0F0Fu) | ((Hd & 0x03030303u) << 4),
+                                               (L1 & 0x0F0F0F0Fu) | (Hd & 0x30303030u)};
+        *reinterpret_cast<uint2*>(col + 32) = uint2{((L0 >> 4) & 0x0F0F0F0Fu) | ((Hd & 0x0C0C0C0Cu) << 2),
+                                                    ((L1 >> 4) & 0x0F0F0F0Fu) | ((Hd >> 2) & 0x30303030u)};
+        if (q == 0) *reinterpret_cast<uint16_t*>(scl + 2 * (16 * t + i)) = (uint16_t)(sv[t >> 1] >> (16 * (t & 1)));
+    }
+    wave_lds_sync();
+    // lane i of group q: row 16 k + i, columns 8 (4 m + q) .. + 7
+    v2i u[4][4];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const uint32_t lb = (Lw[e >> 2] >> (8 * (e & 3))) & 0xFF;
-            const uint32_t hb = (Hd >> (8 * (e & 3) + 4 * (e >> 2))) & 0xF;  // bits 0-1: row 8 q + e, 2-3: row 32 + ..
-            const int q0 = (int)((lb & 15) | ((hb & 3) << 4)) - 32;
-            const int q1 = (int)((lb >> 4) | ((hb >> 2) << 4)) - 32;
-            const int64_t r0 = (int64_t)c * 64 + 8 * q + e;
-            wb[r0 * N + n] = (OutT)(s * (float)q0);
-            wb[(r0 + 32) * N + n] = (OutT)(s * (float)q1);
+    for (int k = 0; k < 4; ++k)
+#pragma unroll
+        for (int m = 0; m < 4; ++m)
+            u[k][m] = __builtin_amdgcn_ds_read_tr8_b64_v2i32(
+                (lds_v2i*)(buf + (8 * (4 * m + q) + (i >> 1)) * kDqCol + 16 * k + 8 * (i & 1)));
+    wave_lds_sync();
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+#pragma unroll
+        for (int m = 0; m < 4; ++m) *reinterpret_cast<v2i*>(buf + (16 * k + i) * kDqRow + 8 * (4 * m + q)) = u[k][m];
+    wave_lds_sync();
+    // 16 bytes a lane: eight columns of four rows an instruction, in fp32 four columns of two
+    if constexpr (sizeof(OutT) == 2) {
+        const int n = strip * kTileN + 8 * i;
+        if (n >= N) return;
+        const u4 sc = *reinterpret_cast<const u4*>(scl + 16 * i);
+        OutT* const dst = w + b * sw_b + ((int64_t)c * 64 + q) * N + n;
+#pragma unroll
+        for (int y = 0; y < 16; ++y) {
+            float v[8];
+            dequant8(*reinterpret_cast<const uint2*>(buf + (4 * y + q) * kDqRow + 8 * i), sc, v);
+            store_row8(dst + (int64_t)(4 * y) * N, v, vec);
+        }
+    } else {
+        const int h = lane >> 5, k = lane & 31, n = strip * kTileN + 4 * k;
+        if (n >= N) return;
+        const uint2 sc = *reinterpret_cast<const uint2*>(scl + 8 * k);
+        OutT* const dst = w + b * sw_b + ((int64_t)c * 64 + h) * N + n;
+#pragma unroll
+        for (int y = 0; y < 32; ++y) {
+            float v[8];
+            const uint32_t u = *reinterpret_cast<const uint32_t*>(buf + (2 * y + h) * kDqRow + 4 * k);
+            dequant8(uint2{u, 0}, u4{sc.x, sc.y, 0, 0}, v);
+            OutT* const d = dst + (int64_t)(2 * y) * N;
+            if (vec)
+                *reinterpret_cast<f4*>(d) = f4{v[0], v[1], v[2], v[3]};
+            else
+#pragma unroll
+                for (int e = 0; e < 4; ++e) d[e] = v[e];
         }
     }
 }
@@ -728,41 +790,40 @@ __global__ __launch_bounds__(256) void w6a16_pack_scales_kernel(const uint16_t* 
     *reinterpret_cast<u4*>(out + ((int64_t)b * strips * groups + sg) * kTileN + 8 * i) = u4{o[0], o[1], o[2], o[3]};
 }
 
-// Dequantise: w[b][k][n] = s q as bf16 or fp32 (the large-M path hands the result to a library GEMM).  Grid
-// (ceil(N / 4096), K / 2, B): one thread per (lo row c * 32 + j, 16 columns); it writes rows c * 64 + j and
-// c * 64 + j + 32 of those columns.
+// Dequantise: w[b][k][n] = s q as bf16, fp16 or fp32 (the large-M path hands the result to a library GEMM).  Grid
+// (ceil(N / 2048), K / 16, B): one thread per (four hi rows, 8 columns); hi row j's four fields and lo rows j and j + 16
+// give rows j, j + 16, j + 32 and j + 48 of the chunk, stored as whole lines (a wavefront 1 KB of a row in bf16).
+// K = 4096, N = 16384, bf16, weights cycled: 52.3 us with two 16-byte stores at 32 bytes from lane to lane -> 32.4.
 template <typename OutT>
 __global__ __launch_bounds__(256) void w6a16_dequant_kernel(const uint8_t* lo, const uint8_t* hi, const uint16_t* sc,
                                                             OutT* w, int32_t K, int32_t N, int32_t group_k,
                                                             int64_t sl_b, int64_t sh_b, int64_t ss_b, int64_t sw_b) {
-    const int n = (blockIdx.x * 256 + threadIdx.x) * 16;
+    const int64_t n = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 8;
     if (n >= N) return;
-    const int lrow = blockIdx.y, b = blockIdx.z;
-    const int c = lrow >> 5, j = lrow & 31;
-    const u4 L = *reinterpret_cast<const u4*>(lo + b * sl_b + (int64_t)lrow * N + n);
-    const u4 H = *reinterpret_cast<const u4*>(hi + b * sh_b + ((int64_t)c * 16 + (j & 15)) * N + n);
-    const int sh0 = 2 * (j >> 4), sh1 = sh0 + 4;  // 2-bit fields of rows j and j + 32
-    const int r0 = c * 64 + j, r1 = r0 + 32;
-    const uint16_t* const s0 = sc + b * ss_b + (int64_t)(r0 / group_k) * N + n;
-    const uint16_t* const s1 = sc + b * ss_b + (int64_t)(r1 / group_k) * N + n;
-    OutT* const w0 = w + b * sw_b + (int64_t)r0 * N + n;
-    OutT* const w1 = w + b * sw_b + (int64_t)r1 * N + n;
+    const int c = blockIdx.y >> 2, j0 = 4 * (blockIdx.y & 3), b = blockIdx.z;
+    const uint8_t* const L = lo + b * sl_b + ((int64_t)c * 32 + j0) * N + n;
+    const uint8_t* const H = hi + b * sh_b + ((int64_t)c * 16 + j0) * N + n;
+    const u4 s = *reinterpret_cast<const u4*>(sc + b * ss_b + (int64_t)(c * 64 / group_k) * N + n);
+    OutT* const dst = w + b * sw_b + ((int64_t)c * 64 + j0) * N + n;
+    uint2 l[4][2], h[4];
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {  // columns n + 8 h .. + 7
-        const u4 sa = *reinterpret_cast<const u4*>(s0 + 8 * h), sb = *reinterpret_cast<const u4*>(s1 + 8 * h);
-        float va[8], vb[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const int col = 8 * h + e, wd = col >> 2, by = 8 * (col & 3);
-            const uint32_t l = (L[wd] >> by) & 0xFF, hh = (H[wd] >> by) & 0xFF;
-            const int q0 = (int)((l & 15) | (((hh >> sh0) & 3) << 4)) - 32;
-            const int q1 = (int)((l >> 4) | (((hh >> sh1) & 3) << 4)) - 32;
-            va[e] = h2f((uint16_t)(sa[e >> 1] >> (16 * (e & 1)))) * (float)q0;  // exact: 11 x 6 bit product
-            vb[e] = h2f((uint16_t)(sb[e >> 1] >> (16 * (e & 1)))) * (float)q1;
-        }
-        store8(w0 + 8 * h, va);
-        store8(w1 + 8 * h, vb);
+    for (int j = 0; j < 4; ++j) {
+        l[j][0] = *reinterpret_cast<const uint2*>(L + (int64_t)j * N);
+        l[j][1] = *reinterpret_cast<const uint2*>(L + (int64_t)(16 + j) * N);
+        h[j] = *reinterpret_cast<const uint2*>(H + (int64_t)j * N);
     }
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int f = 0; f < 4; ++f) {  // row j0 + j + 16 f: nibble f >> 1 of lo row j0 + j + 16 (f & 1), field f of the hi row
+            const uint2 x = l[j][f & 1];
+            const int nib = 4 * (f >> 1);
+            const uint2 u = uint2{((x.x >> nib) & 0x0F0F0F0Fu) | (((h[j].x >> (2 * f)) & 0x03030303u) << 4),
+                                  ((x.y >> nib) & 0x0F0F0F0Fu) | (((h[j].y >> (2 * f)) & 0x03030303u) << 4)};
+            float v[8];
+            dequant8(u, s, v);
+            store8(dst + (int64_t)(16 * f + j) * N, v);
+        }
 }
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -1369,19 +1430,19 @@ int w6a16_dequantize_packed(const void* packed, const uint16_t* packed_scales, v
     if (!w6::aligned16(packed) || !w6::aligned16(packed_scales)) return WKV7_ERR_ALIGN;
     if (B > 65535) return WKV7_ERR_SHAPE;
     const int strips = (N + w6::kTileN - 1) / w6::kTileN;
-    const int64_t nw = (int64_t)strips * (K / 64) * 64;
-    const dim3 grid((unsigned)((nw + 255) / 256), B);
+    const dim3 grid((unsigned)(((int64_t)strips * (K / 64) + 3) / 4), B);
+    const bool vec = w6::aligned16(w) && w_batch_stride % 8 == 0;  // fp32: 8 elements are two 16-byte stores
     const hipStream_t s = static_cast<hipStream_t>(stream);
     const uint8_t* pk = static_cast<const uint8_t*>(packed);
     if (out_dtype == W6A16_OUT_F32)
         hipLaunchKernelGGL(w6::w6a16_dequant_packed_kernel<float>, grid, dim3(256), 0, s, pk, packed_scales,
-                           static_cast<float*>(w), K, N, group_k, strips, w_batch_stride);
+                           static_cast<float*>(w), K, N, group_k, strips, w_batch_stride, vec);
     else if (out_dtype == W6A16_OUT_F16)
         hipLaunchKernelGGL(w6::w6a16_dequant_packed_kernel<_Float16>, grid, dim3(256), 0, s, pk, packed_scales,
-                           static_cast<_Float16*>(w), K, N, group_k, strips, w_batch_stride);
+                           static_cast<_Float16*>(w), K, N, group_k, strips, w_batch_stride, vec);
     else
         hipLaunchKernelGGL(w6::w6a16_dequant_packed_kernel<__bf16>, grid, dim3(256), 0, s, pk, packed_scales,
-                           static_cast<__bf16*>(w), K, N, group_k, strips, w_batch_stride);
+                           static_cast<__bf16*>(w), K, N, group_k, strips, w_batch_stride, vec);
     return static_cast<int>(hipGetLastError());
 }
 
@@ -1425,7 +1486,7 @@ int w6a16_dequantize(const uint8_t* lo, const uint8_t* hi, const uint16_t* scale
         lo_batch_stride % 16 || hi_batch_stride % 16 || scales_batch_stride % 8 || w_batch_stride % 8)
         return WKV7_ERR_ALIGN;
     if (K / 2 > 65535 || B > 65535) return WKV7_ERR_SHAPE;  // grid y and z
-    const dim3 grid((N / 16 + 255) / 256, K / 2, B);
+    const dim3 grid((N / 8 + 255) / 256, K / 16, B);
     const hipStream_t s = static_cast<hipStream_t>(stream);
     if (out_dtype == W6A16_OUT_F32)
         hipLaunchKernelGGL(w6::w6a16_dequant_kernel<float>, grid, dim3(256), 0, s, lo, hi, scales,

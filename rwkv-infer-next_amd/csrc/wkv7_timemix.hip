@@ -18,8 +18,13 @@
 // load per operand row), 8 lanes cover a head and a wavefront covers a group of 8 heads of one token.  Each
 // wavefront stays on one head group and strides over tokens, so the per-channel parameters are loaded once into
 // registers; the per-head sums are 8-lane butterflies.  All arithmetic is fp32 with one bf16 rounding per output
-// (the reference rounds after every torch op).
+// (the reference rounds after every torch op).  Decode-sized launches are bound by latency: with the work split, the
+// look-ahead and the sums below in their present form, 12 layers of one token with H = 12 (prologue, recurrence and
+// epilogue in one graph) went from 101 to 94 us, 8 layers of 23 tokens with H = 40 from 125 to 117, 4 of 64 with
+// H = 64 from 135.4 to 132.6; T = 4096, H = 64 from 107.6 to 106.3 (5.4 TB/s).
 #include <stdint.h>
+
+#include <algorithm>
 
 #include "wkv7.h"
 #include "wkv7_device.h"
@@ -28,7 +33,7 @@
 namespace wkv7 {
 namespace {
 
-constexpr int kWaves = 4;                 // wavefronts per workgroup
+constexpr int kWaves = 4;                 // wavefronts per workgroup (one where that leaves CUs without a workgroup)
 constexpr int kVec = 8;                   // channels per lane
 constexpr int kHeadLanes = HS / kVec;     // lanes per head (8)
 constexpr int kGroupHeads = 64 / kHeadLanes;  // heads per wavefront (8)
@@ -53,12 +58,14 @@ __device__ __forceinline__ void zero8(float (&x)[kVec]) {
     for (int j = 0; j < kVec; ++j) x[j] = 0.f;
 }
 
-// Sum over the 8 lanes of one head.
-__device__ __forceinline__ float head_sum(float x) {
-#pragma unroll
-    for (int m = 1; m < kHeadLanes; m <<= 1) x += __shfl_xor(x, m);
-    return x;
+template <int CTRL>
+__device__ __forceinline__ float dpp_add(float x) {  // x + x of the lane DPP control CTRL selects (all lanes active)
+    return x + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xF, 0xF, false));
 }
+
+// Sum over the 8 lanes of one head: lanes ^ 1, lanes ^ 2, then lane 7 - l, whose quad holds the other half's sum (the sums
+// of a three-step butterfly, without its round trips through the LDS crossbar).
+__device__ __forceinline__ float head_sum(float x) { return dpp_add<0x141>(dpp_add<0x4E>(dpp_add<0xB1>(x))); }
 
 // Transcendentals on the hardware's base-2 exp/log and reciprocal (about 1 ulp of fp32; every output is rounded
 // to bf16, 2^-9 relative).
@@ -74,30 +81,38 @@ __device__ __forceinline__ float softplus(float x) {
     return fmaxf(x, 0.f) + kLn2 * __builtin_amdgcn_logf(1.f + __builtin_amdgcn_exp2f(-fabsf(x) * kLog2e));
 }
 
-// Work split shared by both kernels: wavefront gw owns head group gw % groups and tokens gw / groups, + stride.
+// Work split shared by both kernels: wavefront gw owns head group gw % groups and tokens gw / groups, + stride.  The
+// division is a multiplication by a reciprocal from the host (three 64-bit divisions took a decode-sized launch
+// longer than its arithmetic).
+struct Split {
+    int groups;        // head groups of a token
+    uint32_t inv;      // gw / groups = gw inv >> 32
+    int per;           // tokens under way at a time
+};
+
 struct Lanes {
     int64_t t0, tstride;
     int c;        // first channel of this lane within a token row
     bool active;  // the wavefront has work and the lane's head exists
 };
 
-__device__ __forceinline__ Lanes lanes(int H) {
+__device__ __forceinline__ Lanes lanes(int H, int64_t tokens, const Split& s) {
     const int lane = threadIdx.x & 63;
-    const int groups = (H + kGroupHeads - 1) / kGroupHeads;
-    const int64_t gw = (int64_t)blockIdx.x * kWaves + (threadIdx.x >> 6);
-    const int64_t per = (int64_t)gridDim.x * kWaves / groups;  // >= 1 by the launch (grid_for)
+    const uint32_t gw = blockIdx.x * (blockDim.x >> 6) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int t0 = s.groups == 1 ? (int)gw : (int)__umulhi(gw, s.inv);
     Lanes l;
-    const int h = (int)(gw % groups) * kGroupHeads + lane / kHeadLanes;
-    l.t0 = gw / groups;
-    l.tstride = per;
+    const int h = ((int)gw - t0 * s.groups) * kGroupHeads + lane / kHeadLanes;
+    l.t0 = t0;
+    l.tstride = s.per;
     l.c = h * HS + (lane % kHeadLanes) * kVec;
-    l.active = h < H && l.t0 < per;  // waves past per * groups would repeat another wave's tokens
+    // waves past per * groups would repeat another wave's tokens, or pass the last token
+    l.active = h < H && t0 < s.per && t0 < tokens;
     return l;
 }
 
 // Token rows of one lane, raw (8 bf16 per operand).  Two of these alternate in the token loops below, so the
 // loads of the next token are in flight while the current one is computed; the row index is clamped to the last
-// token so that the look-ahead loads are unconditional and in bounds.
+// token so that the look-ahead loads are unconditional and in bounds.  A wavefront with one token (decode) looks not ahead.
 struct ProRows {
     u4 k, v, ow, oa, vf, ov;
 };
@@ -163,18 +178,19 @@ __device__ __forceinline__ void prologue_token(const wkv7_prologue_args& a, cons
 }
 
 template <bool MIX>
-__global__ __launch_bounds__(64 * kWaves) void timemix_prologue_kernel(const wkv7_prologue_args a) {
-    const Lanes l = lanes(a.H);
+__global__ __launch_bounds__(64 * kWaves) void timemix_prologue_kernel(const wkv7_prologue_args a, const Split s) {
+    const Lanes l = lanes(a.H, a.tokens, s);
     if (!l.active) return;
+    ProRows x0, x1;
+    int64_t t = l.t0;
+    load_rows<MIX>(a, t, l.c, x0);
     ProParams p;
     load8(a.b_w + l.c, p.bw);
     load8(a.b_a + l.c, p.ba);
     load8(a.kk_mul + l.c, p.km);
     load8(a.ka_mul + l.c, p.ka);
     if constexpr (MIX) load8(a.b_v + l.c, p.bv);
-    ProRows x0, x1;
-    int64_t t = l.t0;
-    load_rows<MIX>(a, t, l.c, x0);
+    if (l.tstride >= a.tokens) return prologue_token<MIX>(a, p, x0, t, l.c);
     while (t < a.tokens) {
         load_rows<MIX>(a, t + l.tstride, l.c, x1);
         prologue_token<MIX>(a, p, x0, t, l.c);
@@ -232,16 +248,17 @@ __device__ __forceinline__ void epilogue_token(const wkv7_epilogue_args& a, cons
     store8(a.out + t * a.out_stride + c, out);
 }
 
-__global__ __launch_bounds__(64 * kWaves) void timemix_epilogue_kernel(const wkv7_epilogue_args a) {
-    const Lanes l = lanes(a.H);
+__global__ __launch_bounds__(64 * kWaves) void timemix_epilogue_kernel(const wkv7_epilogue_args a, const Split s) {
+    const Lanes l = lanes(a.H, a.tokens, s);
     if (!l.active) return;
+    EpiRows x0, x1;
+    int64_t t = l.t0;
+    load_rows(a, t, l.c, x0);
     EpiParams p;
     load8(a.lnx_w + l.c, p.lw);
     load8(a.lnx_b + l.c, p.lb);
     load8(a.r_k + l.c, p.rk);  // r_k is [H][64]: the same offset as the channel
-    EpiRows x0, x1;
-    int64_t t = l.t0;
-    load_rows(a, t, l.c, x0);
+    if (l.tstride >= a.tokens) return epilogue_token(a, p, x0, t, l.c);
     while (t < a.tokens) {
         load_rows(a, t + l.tstride, l.c, x1);
         epilogue_token(a, p, x0, t, l.c);
@@ -253,17 +270,21 @@ __global__ __launch_bounds__(64 * kWaves) void timemix_epilogue_kernel(const wkv
     }
 }
 
-// Workgroups for `tokens` tokens of H heads: enough wavefronts in flight to stream HBM (8 workgroups per CU),
-// and at least one wavefront per head group.
-int grid_for(int64_t tokens, int H) {
-    const int cus = device_cu_count();
-    const int64_t groups = (H + kGroupHeads - 1) / kGroupHeads;
-    const int64_t need = (tokens * groups + kWaves - 1) / kWaves;
-    const int64_t cap = (int64_t)cus * 8;
-    const int64_t floor = (groups + kWaves - 1) / kWaves;
-    int64_t b = need < cap ? need : cap;
-    if (b < floor) b = floor;
-    return (int)b;
+// Launch for `tokens` tokens of H heads: enough wavefronts in flight to stream HBM (32 per CU), at least one per head
+// group; single-wavefront workgroups where workgroups of four would leave CUs idle.
+struct Launch {
+    dim3 grid, block;
+    Split split;
+};
+
+Launch launch_for(int64_t tokens, int H) {
+    const int64_t cus = device_cu_count(), groups = (H + kGroupHeads - 1) / kGroupHeads;
+    int64_t waves = std::max(groups, std::min(tokens * groups, cus * 8 * kWaves));
+    const int w = waves < cus * kWaves ? 1 : kWaves;
+    const int64_t wgs = (waves + w - 1) / w;
+    waves = wgs * w;
+    return {dim3((unsigned)wgs), dim3(64 * w),
+            {(int)groups, (uint32_t)(((uint64_t(1) << 32) + groups - 1) / groups), (int)(waves / groups)}};
 }
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
@@ -292,11 +313,12 @@ int wkv7_timemix_prologue(const wkv7_prologue_args* a, void* stream) {
     if (a->v_first && (!wkv7::aligned16(a->v_first) || !wkv7::aligned16(a->o_v) || !wkv7::aligned16(a->b_v)))
         return WKV7_ERR_ALIGN;
     if (a->in_stride % 8 || a->out_stride % 8) return WKV7_ERR_ALIGN;
-    const dim3 grid(wkv7::grid_for(a->tokens, a->H)), block(64 * wkv7::kWaves);
+    const wkv7::Launch l = wkv7::launch_for(a->tokens, a->H);
+    const hipStream_t s = static_cast<hipStream_t>(stream);
     if (a->v_first)
-        hipLaunchKernelGGL(wkv7::timemix_prologue_kernel<true>, grid, block, 0, static_cast<hipStream_t>(stream), *a);
+        hipLaunchKernelGGL(wkv7::timemix_prologue_kernel<true>, l.grid, l.block, 0, s, *a, l.split);
     else
-        hipLaunchKernelGGL(wkv7::timemix_prologue_kernel<false>, grid, block, 0, static_cast<hipStream_t>(stream), *a);
+        hipLaunchKernelGGL(wkv7::timemix_prologue_kernel<false>, l.grid, l.block, 0, s, *a, l.split);
     return static_cast<int>(hipGetLastError());
 }
 
@@ -313,8 +335,8 @@ int wkv7_timemix_epilogue(const wkv7_epilogue_args* a, void* stream) {
     for (const void* q : req)
         if (!wkv7::aligned16(q)) return WKV7_ERR_ALIGN;
     if (a->in_stride % 8 || a->out_stride % 8) return WKV7_ERR_ALIGN;
-    hipLaunchKernelGGL(wkv7::timemix_epilogue_kernel, dim3(wkv7::grid_for(a->tokens, a->H)),
-                       dim3(64 * wkv7::kWaves), 0, static_cast<hipStream_t>(stream), *a);
+    const wkv7::Launch l = wkv7::launch_for(a->tokens, a->H);
+    hipLaunchKernelGGL(wkv7::timemix_epilogue_kernel, l.grid, l.block, 0, static_cast<hipStream_t>(stream), *a, l.split);
     return static_cast<int>(hipGetLastError());
 }
 

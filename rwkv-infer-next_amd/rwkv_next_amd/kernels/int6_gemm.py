@@ -39,7 +39,7 @@ from typing import NamedTuple
 import torch
 
 from .. import _lib
-from ._workspace import stream_workspace
+from ._workspace import on_device, stream_handle, stream_workspace
 
 CHUNK = 64
 QMIN, QMAX = -32, 31
@@ -142,10 +142,10 @@ def dequantize_int6(lo, hi, sc, group_k, dtype=torch.float32):
     if dtype not in _OUT_CODES:
         raise TypeError(f"dequantize_int6 writes bfloat16, float16 or float32 (got {dtype})")
     w = torch.empty((Bq, K, N), dtype=dtype, device=L.device)
-    with torch.cuda.device(L.device):
+    with on_device(L.device):
         _lib.check(_lib.load().w6a16_dequantize(
             L.data_ptr(), H.data_ptr(), S.data_ptr(), w.data_ptr(), Bq, K, N, g, L.stride(0), H.stride(0),
-            S.stride(0), w.stride(0), _OUT_CODES[dtype], torch.cuda.current_stream(L.device).cuda_stream))
+            S.stride(0), w.stride(0), _OUT_CODES[dtype], stream_handle(L.device)))
     return w[0] if squeeze else w
 
 
@@ -198,10 +198,10 @@ def prepack_int6(lo, hi, s, group_k) -> Int6Packed:
     _lib.check(lib.w6a16_packed_size(Bq, K, N, g, ctypes.byref(wb), ctypes.byref(sb)))
     weight = torch.empty(int(wb.value), dtype=torch.uint8, device=L.device)
     scales = torch.empty(int(sb.value) // 2, dtype=torch.float16, device=L.device)
-    with torch.cuda.device(L.device):
+    with on_device(L.device):
         _lib.check(lib.w6a16_pack(L.data_ptr(), H.data_ptr(), S.data_ptr(), Bq, K, N, g, L.stride(0), H.stride(0),
                                   S.stride(0), weight.data_ptr(), scales.data_ptr(),
-                                  torch.cuda.current_stream(L.device).cuda_stream))
+                                  stream_handle(L.device)))
     return Int6Packed(weight.view(Bq, -1), scales.view(Bq, -1), 0 if lo.dim() == 2 else Bq, K, N, g)
 
 
@@ -212,10 +212,10 @@ def dequantize_int6_packed(pk: Int6Packed, dtype=torch.float32):
         raise TypeError(f"dequantize_int6_packed writes bfloat16, float16 or float32 (got {dtype})")
     Bq = pk.weight.shape[0]
     w = torch.empty((Bq, pk.K, pk.N), dtype=dtype, device=pk.weight.device)
-    with torch.cuda.device(w.device):
+    with on_device(w.device):
         _lib.check(_lib.load().w6a16_dequantize_packed(
             pk.weight.data_ptr(), pk.scales.data_ptr(), w.data_ptr(), Bq, pk.K, pk.N, pk.group_k, w.stride(0),
-            _OUT_CODES[dtype], torch.cuda.current_stream(w.device).cuda_stream))
+            _OUT_CODES[dtype], stream_handle(w.device)))
     return w if pk.batches else w[0]
 
 
@@ -298,7 +298,7 @@ def _impl(a, w: _W, split_k, out_dtype=None):
     if n.value:  # counters and partial tiles of a K split over workgroups
         ws = _workspace(A.device, int(n.value))
         args.workspace, args.workspace_bytes = ws.data_ptr(), ws.numel()
-    _lib.check(lib.w6a16_matmul(args, torch.cuda.current_stream(A.device).cuda_stream))
+    _lib.check(lib.w6a16_matmul(args, stream_handle(A.device)))
     return out if batched else out[0]
 
 
@@ -323,7 +323,7 @@ def int6_matmul(a, lo, hi=None, s=None, group_k=None, split_k=None, use_dot=None
     M = a.shape[-2]
     if split_k is None:
         split_k = plan_int6_packed(M, w.N, w.K, B, a.device) if packed else plan_int6(M, w.N, w.K, B, a.device)[0]
-    with torch.cuda.device(a.device):
+    with on_device(a.device):
         return _impl(a, w, split_k, out_dtype)
 
 
@@ -332,7 +332,7 @@ def int6_matmul_op(a: torch.Tensor, lo: torch.Tensor, hi: torch.Tensor, s: torch
                    use_dot: bool) -> torch.Tensor:
     """Functional op with the schema of the reference's rwkv_next::int6_matmul (int6_gemm.py:316-323); the plan
     (split_k, use_dot) comes from plan_int6, resolved by the caller."""
-    with torch.cuda.device(a.device):
+    with on_device(a.device):
         return _impl(a, _planes(lo, hi, s, group_k), split_k)
 
 
@@ -340,7 +340,7 @@ def int6_matmul_op(a: torch.Tensor, lo: torch.Tensor, hi: torch.Tensor, s: torch
 def int6_matmul_packed_op(a: torch.Tensor, weight: torch.Tensor, scales: torch.Tensor, batches: int, K: int, N: int,
                           group_k: int, split_k: int) -> torch.Tensor:
     """int6_matmul_op for a packed weight (the fields of an Int6Packed); no counterpart in the reference."""
-    with torch.cuda.device(a.device):
+    with on_device(a.device):
         return _impl(a, _packed(Int6Packed(weight, scales, batches, K, N, group_k)), split_k)
 
 

@@ -15,6 +15,7 @@ from __future__ import annotations
 import torch
 
 from .. import _lib
+from ._workspace import on_device, stream_handle
 
 HEAD_SIZE = 64
 
@@ -59,15 +60,11 @@ def timemix_prologue(r, k, v, o, v_first, b_w, b_a, b_v, kk_mul, ka_mul, H, N, f
     vf = None if first_layer else _rows(v_first, C, "v_first")
     prm = [_param(x, C, n) for x, n in ((b_w, "b_w"), (b_a, "b_a"), (b_v, "b_v"), (kk_mul, "kk_mul"), (ka_mul, "ka_mul"))]
     outs = [torch.empty(M, C, device=k.device, dtype=torch.bfloat16) for _ in range(5)]
-    a = _lib.PrologueArgs()
-    a.k, a.v = kk2.data_ptr(), vv2.data_ptr()
-    a.o_v, a.o_w, a.o_a = (t.data_ptr() for t in oo)
-    a.v_first = None if vf is None else vf.data_ptr()
-    a.b_w, a.b_a, a.b_v, a.kk_mul, a.ka_mul = (t.data_ptr() for t in prm)
-    a.w_out, a.k_out, a.v_out, a.a_out, a.b_out = (t.data_ptr() for t in outs)
-    a.tokens, a.in_stride, a.out_stride, a.H, a.head_size = M, C, C, H, N
-    with torch.cuda.device(k.device):
-        _lib.check(_lib.load().wkv7_timemix_prologue(a, torch.cuda.current_stream(k.device).cuda_stream))
+    a = _lib.PrologueArgs(kk2.data_ptr(), vv2.data_ptr(), *[t.data_ptr() for t in oo],
+                          None if vf is None else vf.data_ptr(), *[t.data_ptr() for t in prm],
+                          *[t.data_ptr() for t in outs], M, C, C, H, N)  # in the order of the fields
+    with on_device(k.device):
+        _lib.check(_lib.load().wkv7_timemix_prologue(a, stream_handle(k.device)))
     w, k2, v2, aa, bb = (t.view(shape) for t in outs)
     ins = (r, w, k2, v2, aa, bb)
     return ins, (v if first_layer else v_first)
@@ -86,10 +83,7 @@ def timemix_epilogue(y, r, k, v, g, lnx_w, lnx_b, r_k, H, N, eps):
             raise ValueError("epilogue inputs must have the same number of rows")
     lw, lb, rk = _param(lnx_w, C, "lnx_w"), _param(lnx_b, C, "lnx_b"), _param(r_k, C, "r_k")
     out = torch.empty(M, C, device=y.device, dtype=torch.bfloat16)
-    a = _lib.EpilogueArgs()
-    a.y, a.r, a.k, a.v, a.g = (t.data_ptr() for t in (yy, rr, kk, vv, gg))
-    a.lnx_w, a.lnx_b, a.r_k, a.out = lw.data_ptr(), lb.data_ptr(), rk.data_ptr(), out.data_ptr()
-    a.tokens, a.in_stride, a.out_stride, a.eps, a.H, a.head_size = M, C, C, float(eps), H, N
-    with torch.cuda.device(y.device):
-        _lib.check(_lib.load().wkv7_timemix_epilogue(a, torch.cuda.current_stream(y.device).cuda_stream))
+    a = _lib.EpilogueArgs(*[t.data_ptr() for t in (yy, rr, kk, vv, gg, lw, lb, rk, out)], M, C, C, float(eps), H, N)
+    with on_device(y.device):
+        _lib.check(_lib.load().wkv7_timemix_epilogue(a, stream_handle(y.device)))
     return out

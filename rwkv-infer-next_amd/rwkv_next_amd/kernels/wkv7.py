@@ -30,7 +30,7 @@ import torch
 from torch import Tensor
 
 from .. import _lib
-from ._workspace import stream_workspace
+from ._workspace import on_device, stream_handle, stream_workspace
 
 _WORKSPACES: dict = {}  # (device index, stream handle) -> [workspace, flags zeroed in stream order, capture id]
 
@@ -58,7 +58,7 @@ def _prep_operands(r, w, k, v, a, b, H, K):
             raise ValueError(f"operand {name} has shape {tuple(t.shape)}, expected {tuple(shape)}")
         if t.dtype != torch.bfloat16:
             raise TypeError(f"operand {name} must be bfloat16 (got {t.dtype})")
-        if t.device.type != "cuda":
+        if not t.is_cuda:
             raise ValueError(f"operand {name} must be on a GPU (got {t.device})")
     if r.dim() == 4:
         B, T = shape[0], shape[1]
@@ -90,36 +90,26 @@ def _launch(ops, *, H, K=HEAD_SIZE, num_seqs, T, total, o=None, h0=None, h0_idx=
             ht_idx=None, ht_rows=0, fresh=None, cu=None, n_keep=None, snap=None, algo=_lib.ALGO_AUTO, rec_max_len=-1,
             status=None):
     dev = ops[0].device
-    args = _lib.Wkv7Args()
-    for name, t in zip(OPERANDS, ops):
-        setattr(args, name, t.data_ptr())
-    args.in_tok_stride = H * K
-    args.o = _ptr(o)
-    args.o_tok_stride = H * K
-    args.h0, args.h0_idx, args.h0_rows = _ptr(h0), _ptr(h0_idx), h0_rows
-    args.ht, args.ht_idx, args.ht_rows = _ptr(ht), _ptr(ht_idx), ht_rows
-    args.fresh = _ptr(fresh)
-    args.cu_seqlens = _ptr(cu)
-    args.n_keep = _ptr(n_keep)
-    args.snapshots = _ptr(snap)
-    args.num_seqs, args.T, args.total_tokens = num_seqs, T, total
-    args.H, args.head_size, args.algo, args.rec_max_len = H, K, algo, rec_max_len
-    args.status = _ptr(status)
+    # positional, in the order of the structure's fields: setting them one by one costs a few microseconds a call
+    args = _lib.Wkv7Args(*[t.data_ptr() for t in ops], H * K, _ptr(o), H * K, _ptr(h0), _ptr(h0_idx), h0_rows,
+                         _ptr(ht), _ptr(ht_idx), ht_rows, _ptr(fresh), _ptr(cu), _ptr(n_keep), _ptr(snap), None, 0,
+                         num_seqs, T, total, H, K, algo, rec_max_len, _ptr(status))
     nbytes = _lib.workspace_size(args)
     ws = None
     if nbytes:
         # one workspace per (device, stream): its leading flag region starts zero and every call leaves it zero
         ws = stream_workspace(_WORKSPACES, dev, nbytes, _lib.WKV7_FLAG_REGION_BYTES)
         args.workspace, args.workspace_bytes = ws.data_ptr(), ws.numel()
-    with torch.cuda.device(dev):
-        _lib.run(args, torch.cuda.current_stream(dev).cuda_stream)
+    with on_device(dev):
+        _lib.run(args, stream_handle(dev))
     return ws
 
 
 def _index_tensor(x, dev, dtype, name):
     if x is None:
         return None
-    x = torch.as_tensor(x, device=dev)
+    if not isinstance(x, Tensor) or x.device != dev:
+        x = torch.as_tensor(x, device=dev)
     if x.dtype != dtype:
         x = x.to(dtype)
     return x.contiguous()
@@ -189,7 +179,7 @@ def wkv7(r, w, k, v, a, b, state, H, K, cu_seqlens=None, final=True, *, algo: in
     Mirrors rwkv_next/kernels/wkv7.py:126-138."""
     if cu_seqlens is None:
         if algo == _lib.ALGO_AUTO:
-            h0 = state.contiguous() if state is not None else r.new_empty(0, dtype=torch.float32)
+            h0 = state.contiguous() if state is not None else torch.empty(0, dtype=torch.float32, device=r.device)
             o, ht = wkv7_fwd(r, w, k, v, a, b, h0, H, K, final)
         else:
             o, ht = _fwd_impl(r, w, k, v, a, b, state, H, K, final, algo)
@@ -331,7 +321,10 @@ def wkv7_pool_(r, w, k, v, a, b, pool, slots, H, K, *, cu_seqlens=None, n_keep=N
     nk = _index_tensor(n_keep, dev, torch.int64, "n_keep")
     fr = None
     if fresh is not None:
-        fr = torch.as_tensor(fresh, device=dev)
+        # a bool tensor's bytes are 0 and 1 already: read as they are, not converted by a kernel
+        fr = fresh if isinstance(fresh, Tensor) and fresh.device == dev else torch.as_tensor(fresh, device=dev)
+        if fr.dtype == torch.bool:
+            fr = fr.view(torch.uint8)
         fr = (fr if fr.dtype == torch.uint8 else fr.to(torch.uint8)).contiguous()
     if snapshots is not None:
         if cu is not None and max_len < 1:
@@ -384,7 +377,7 @@ def check_distinct_slots(slots: torch.Tensor, num_slots: int) -> None:
 
 
 def _stream(dev):
-    return torch.cuda.current_stream(dev).cuda_stream
+    return stream_handle(dev)
 
 
 def restore_snapshots_(pool, slots, snapshots, n):
@@ -403,7 +396,7 @@ def restore_snapshots_(pool, slots, snapshots, n):
     nn = _index_tensor(n, dev, torch.int64, "n")
     if sl.numel() != N or nn.numel() != N:
         raise ValueError(f"slots and n must have {N} entries")
-    with torch.cuda.device(dev):
+    with on_device(dev):
         _lib.check(_lib.load().wkv7_snapshot_restore(pool.data_ptr(), pool.shape[0], H, sl.data_ptr(),
                                                      snapshots.data_ptr(), T, nn.data_ptr(), N, _stream(dev)))
     return pool

@@ -56,6 +56,7 @@ namespace {
 
 typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
 typedef short s4 __attribute__((ext_vector_type(4)));
+typedef short s8 __attribute__((ext_vector_type(8)));
 typedef uint32_t u2v __attribute__((ext_vector_type(2)));
 
 constexpr int SC = kSegChunk;          // 32 tokens per chunk
@@ -69,14 +70,20 @@ constexpr int kFlagSpinLimit = 1 << 20;  // segment hand-off waits (s_sleep 8 ea
 // factor 2^{c-m} kept apart): the state wavefronts apply
 //   U = W S + U0,   S <- Gamma S + diag(2^{c-m}) (Bp^T U + Kp^T V),   y^T = S^T R0^T + U^T rho^T + V^T sigma^T
 // per 16-column tile, which costs them about as many MFMAs as a dense A S + H would and saves the prep wavefront
-// forming A, H and O (its critical path; the state wavefronts have slack).  Bp and Kp go into the record as exact
-// transposes of the prep's own hi/lo splits, so the prep wavefront does not rescale and split them again.
+// forming A, H and O.  What bounds the rate is the issue of the two wavefronts a SIMD holds: time stamps of a
+// T = 4096, H = 64 call gave 16.4 k cycles of a 21.5 k period to a prep wavefront's chunk, the rest waiting for a slot
+// while a state wavefront, whose step takes 1.5 k cycles beside an idle partner, takes 6 to 7 k beside one that issues
+// without a pause (raising either side's priority only moves the wait).  So instructions are what counts: Bp, Kp and
+// V go into the record as the token rows the prep wavefront holds, and the transposes are LDS reads.  As identity
+// MFMAs and conversions on the prep wavefront they were 56 of its 246 MFMAs; without them T = 4096, H = 64 takes 113.5
+// instead of 117.5 us, T = 256, H = 12 (one unit a head) 23.5 instead of 24.8, five ragged rows of 8192 tokens, H = 64,
+// 199 instead of 207.
 constexpr int REC_W = 0;                       // W^T hi/lo as 16x16x32 A operands: [token tile][kb][hl][lane]
-constexpr int REC_B = REC_W + 8 * 1024;        // Bp hi/lo as 16x16x32 A operands: [k tile m][hl][lane]
+constexpr int REC_B = REC_W + 8 * 1024;        // Bp hi, then lo: token rows of 64 channels (n_off)
 constexpr int REC_K = REC_B + 8 * 1024;        // Kp hi/lo, same
 constexpr int REC_R = REC_K + 8 * 1024;        // R0^T hi as 16x16x32 B operands: [token tile][kb][lane]
 constexpr int REC_U = REC_R + 4 * 1024;        // U0, RL fp32: [column tile j][token tile][lane]
-constexpr int REC_V = REC_U + 8 * 1024;        // V (exact), RL tiles (0, j), (1, j) stacked: [column tile j][lane]
+constexpr int REC_V = REC_U + 8 * 1024;        // V (exact): token rows of 64 channels (n_off)
 constexpr int REC_RHO = REC_V + 4 * 1024;      // rho^T hi: tile (0,0) (low 8 bytes), then tiles (0,1), (1,1) stacked
 constexpr int REC_SIG = REC_RHO + 2 * 1024;    // sigma^T hi, same
 constexpr int REC_G = REC_SIG + 2 * 1024;      // Gamma = 2^c per channel, fp32 [64]
@@ -113,6 +120,26 @@ __device__ __forceinline__ s4 hi_t(f4 x) {
 __device__ __forceinline__ bf8 cat(s4 a, s4 b) {
     return __builtin_bit_cast(bf8, __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7));
 }
+
+// Token rows in LDS: 32 rows of 64 bf16 (128 bytes), the 16-byte pieces of row t permuted by t & 7 so that neither the
+// row-wise stores nor the transposing reads meet bank conflicts.
+// Where lane (i, q)'s N fragment of token tile 0, channel block 0 goes; tile 1 is 2048 bytes on, block 1 is at ^ 64.
+__device__ __forceinline__ int n_off(int lane) {
+    const int i = lane & 15, q = lane >> 4;
+    return i * 128 + ((q ^ (i & 7)) * 16);
+}
+// Where the lane's transposing read (ds_read_b64_tr_b16: each lane of a 16-lane group reads 4 consecutive values, lane
+// s receives value s & 3 of the reads of lanes s / 4 + 4 e) of token tile 0, channel tile 0 starts; channel tile m is at
+// ^ 32 m, token tile 1 is 2048 bytes on.  The lane then holds the RL tile: tokens 16 tau + 4 q + v of channel 16 m + i.
+__device__ __forceinline__ int tr_off(int lane) {
+    const int s = lane & 15, t = 4 * (lane >> 4) + (s >> 2);
+    return t * 128 + ((((s & 3) >> 1) ^ (t & 7)) * 16) + (s & 1) * 8;
+}
+typedef __attribute__((address_space(3))) s4 lds_s4;
+__device__ __forceinline__ s4 tr_read(const char* p) { return __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)(p)); }
+// RL tiles of token tiles 0 and 1 stacked: a 16x16x32 operand over the chunk's 32 tokens
+__device__ __forceinline__ bf8 tr_read2(const char* p) { return cat(tr_read(p), tr_read(p + 2048)); }
+
 __device__ __forceinline__ T8 cat(T4 a, T4 b) { return T8{cat(a.h, b.h), cat(a.l, b.l)}; }
 // RL(X^T Y) += ..., 16 contraction rows (small terms first)
 __device__ __forceinline__ f4 p16x3(T4 x, T4 y, f4 c) {
@@ -626,20 +653,7 @@ __device__ __forceinline__ void prep_chunk(const Raw& raw, int Lc, char* rec, fl
     }
     const T8 ttp = cat(tt01, tt11);  // rows s 0-31 of (T^T)'s token tile 1
 
-    // ---- 5. token-row RL tiles (token tile tau, channel tile j) through identity MFMAs (exact): V now, the others
-    //         on the fly below.
-    const bf8 I0 = isel(0, lane), I1 = isel(1, lane);
-    s4 rV[2][4];
-#pragma unroll
-    for (int tau = 0; tau < 2; ++tau)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) rV[tau][j] = hi_t(mma32(Vn[tau][j >> 1], (j & 1) ? I1 : I0, z4()));
-    auto rl = [&](const bf8 (&H8)[2][2], const bf8 (&L8)[2][2], int tau, int j) {
-        const bf8 I = (j & 1) ? I1 : I0;
-        return T4{hi_t(mma32(H8[tau][j >> 1], I, z4())), hi_t(mma32(L8[tau][j >> 1], I, z4()))};
-    };
-
-    // ---- 6. wait for the ring slot
+    // ---- 5. wait for the ring slot
     {
         bool ok = false;
         for (int it = 0; it < kSpinLimit; ++it) {
@@ -655,8 +669,30 @@ __device__ __forceinline__ void prep_chunk(const Raw& raw, int Lc, char* rec, fl
     }
     uint4* const R = reinterpret_cast<uint4*>(rec);
 
+    // ---- 6. the operands' token rows: Bp, Kp and V for the state wavefronts and, V, for the transposing reads below;
+    //         Ah for those too, in W's place until W is stored
+    {
+        const int no = n_off(lane);
+#pragma unroll
+        for (int tau = 0; tau < 2; ++tau)
+#pragma unroll
+            for (int kb = 0; kb < 2; ++kb) {
+                char* const d = rec + tau * 2048 + (no ^ (64 * kb));
+                *reinterpret_cast<uint4*>(d + REC_W) = as_u4(Ah[tau][kb]);
+                *reinterpret_cast<uint4*>(d + REC_W + 4096) = as_u4(Al[tau][kb]);
+                *reinterpret_cast<uint4*>(d + REC_V) = as_u4(Vn[tau][kb]);
+                *reinterpret_cast<uint4*>(d + REC_B) = as_u4(Bh[tau][kb]);
+                *reinterpret_cast<uint4*>(d + REC_B + 4096) = as_u4(Bl[tau][kb]);
+                *reinterpret_cast<uint4*>(d + REC_K) = as_u4(Kh[tau][kb]);
+                *reinterpret_cast<uint4*>(d + REC_K + 4096) = as_u4(Kl[tau][kb]);
+            }
+    }
+    wave_lds_sync();
+    const int to = tr_off(lane);
+    const bf8 I0 = isel(0, lane), I1 = isel(1, lane);
+
     // ---- 7. per channel tile j: W^T = diag(2^m) (T Ah)^T (RL tiles (j, token tile): the record's X = W S operand),
-    //         U0 = T (beta V) and V (RL tiles (token tile, j)), R0^T = diag(2^m) Rh^T (tiles (j, token tile)), all
+    //         U0 = T (beta V) (RL tiles (token tile, j)), R0^T = diag(2^m) Rh^T (tiles (j, token tile)), all
     //         stored
     f4 emr[4];  // 2^m of rows 16 j + 4 q + v, read in one batch ahead of the record stores
 #pragma unroll
@@ -669,7 +705,10 @@ __device__ __forceinline__ void prep_chunk(const Raw& raw, int Lc, char* rec, fl
         T4 Wtt[4][2];
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            const T4 a0 = rl(Ah, Al, 0, j), a1 = rl(Ah, Al, 1, j);
+            const char* const at = rec + REC_W + (to ^ (32 * j));
+            const T4 a0{tr_read(at), tr_read(at + 4096)}, a1{tr_read(at + 2048), tr_read(at + 4096 + 2048)};
+            const char* const vt = rec + REC_V + (to ^ (32 * j));
+            const s4 rV0 = tr_read(vt), rV1 = tr_read(vt + 2048);
             f4 w0 = p16x3(a0, tt00, z4()), w1 = p32x3(cat(a0, a1), ttp, z4());
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
@@ -678,8 +717,8 @@ __device__ __forceinline__ void prep_chunk(const Raw& raw, int Lc, char* rec, fl
             }
             Wtt[j][0] = split_t(w0);
             Wtt[j][1] = split_t(w1);
-            const T4 bv0 = split_t(p16x2(b00, rV[0][j], z4()));
-            const T4 bv1 = split_t(p32x2(bp, cat(rV[0][j], rV[1][j]), z4()));
+            const T4 bv0 = split_t(p16x2(b00, rV0, z4()));
+            const T4 bv1 = split_t(p32x2(bp, cat(rV0, rV1), z4()));
             const f4 u0f = p16x3(tt00, bv0, z4()), u1f = p32x3(ttp, cat(bv0, bv1), z4());
             const bf8 I = (j & 1) ? I1 : I0;
             f4 q0 = mma32(I, Rh[0][j >> 1], z4()), q1 = mma32(I, Rh[1][j >> 1], z4());
@@ -693,7 +732,6 @@ __device__ __forceinline__ void prep_chunk(const Raw& raw, int Lc, char* rec, fl
             reinterpret_cast<uint2*>(R + (REC_R / 16) + (1 * 2 + (j >> 1)) * 64 + lane)[j & 1] = __builtin_bit_cast(uint2, hi_t(q1));
             R[(REC_U / 16) + (j * 2 + 0) * 64 + lane] = __builtin_bit_cast(uint4, u0f);
             R[(REC_U / 16) + (j * 2 + 1) * 64 + lane] = __builtin_bit_cast(uint4, u1f);
-            R[(REC_V / 16) + j * 64 + lane] = as_u4(cat(rV[0][j], rV[1][j]));
         }
         // W^T pieces [token tile][kb][hl]: k tiles 2 kb, 2 kb + 1 stacked
 #pragma unroll
@@ -714,17 +752,6 @@ __device__ __forceinline__ void prep_chunk(const Raw& raw, int Lc, char* rec, fl
             reinterpret_cast<f4*>(rec + REC_G)[lane] = *reinterpret_cast<const f4*>(&fac[2][4 * lane]);
     }
 
-    // ---- 8. per k tile m: Bp and Kp as token-row RL tiles (the transposes of their hi and lo parts, each exact),
-    //         stored with the row factors 2^{c-m}
-#pragma unroll
-    for (int m = 0; m < 4; ++m) {
-        const T8 bpm = cat(rl(Bh, Bl, 0, m), rl(Bh, Bl, 1, m));
-        R[(REC_B / 16) + (m * 2 + 0) * 64 + lane] = as_u4(bpm.h);
-        R[(REC_B / 16) + (m * 2 + 1) * 64 + lane] = as_u4(bpm.l);
-        const T8 kpm = cat(rl(Kh, Kl, 0, m), rl(Kh, Kl, 1, m));
-        R[(REC_K / 16) + (m * 2 + 0) * 64 + lane] = as_u4(kpm.h);
-        R[(REC_K / 16) + (m * 2 + 1) * 64 + lane] = as_u4(kpm.l);
-    }
     if (lane < 16) reinterpret_cast<f4*>(rec + REC_F)[lane] = *reinterpret_cast<const f4*>(&fac[1][4 * lane]);
 }
 
@@ -849,7 +876,9 @@ __device__ __forceinline__ void run_unit(const Params& p, const Unit& U, int32_t
                 asm volatile("" ::: "memory");
             }
             const uint4* const R = reinterpret_cast<const uint4*>(sm.ring[slot]);
-            uint4 rw[2][2][2], rb[4][2], rk[4][2], rr[2][2], rho[2], sig[2], rv;
+            const int to = tr_off(lane);
+            uint4 rw[2][2][2], rr[2][2], rho[2], sig[2];
+            bf8 rb[4][2], rk[4][2], rv;
             f4 ru[2], gm[4], cf[4];
 #pragma unroll
             for (int tau = 0; tau < 2; ++tau)
@@ -861,8 +890,8 @@ __device__ __forceinline__ void run_unit(const Params& p, const Unit& U, int32_t
             for (int m = 0; m < 4; ++m) {
 #pragma unroll
                 for (int hl = 0; hl < 2; ++hl) {
-                    rb[m][hl] = R[(REC_B / 16) + (m * 2 + hl) * 64 + lane];
-                    rk[m][hl] = R[(REC_K / 16) + (m * 2 + hl) * 64 + lane];
+                    rb[m][hl] = tr_read2(sm.ring[slot] + REC_B + hl * 4096 + (to ^ (32 * m)));
+                    rk[m][hl] = tr_read2(sm.ring[slot] + REC_K + hl * 4096 + (to ^ (32 * m)));
                 }
                 gm[m] = reinterpret_cast<const f4*>(sm.ring[slot] + REC_G)[4 * m + q];  // 2^c of rows 16 m + 4 q + v
                 cf[m] = reinterpret_cast<const f4*>(sm.ring[slot] + REC_F)[4 * m + q];  // 2^{c-m}, same rows
@@ -875,7 +904,7 @@ __device__ __forceinline__ void run_unit(const Params& p, const Unit& U, int32_t
                 rho[tau] = R[(REC_RHO / 16) + tau * 64 + lane];
                 sig[tau] = R[(REC_SIG / 16) + tau * 64 + lane];
             }
-            rv = R[(REC_V / 16) + j * 64 + lane];
+            rv = tr_read2(sm.ring[slot] + REC_V + (to ^ (32 * j)));
             lds_wait_all();
             if (lane == 0) lds_store(&sm.done[slot][j], cl / NREC + 1);
 
@@ -899,8 +928,8 @@ __device__ __forceinline__ void run_unit(const Params& p, const Unit& U, int32_t
 #pragma unroll
                 for (int m = 0; m < 4; ++m) {
                     f4 x = z4();
-                    if (state) x = p32x2(T8{as_bf8(rk[m][0]), as_bf8(rk[m][1])}, as_bf8(rv), x);
-                    x = p32x3(T8{as_bf8(rb[m][0]), as_bf8(rb[m][1])}, xo, x);
+                    if (state) x = p32x2(T8{rk[m][0], rk[m][1]}, rv, x);
+                    x = p32x3(T8{rb[m][0], rb[m][1]}, xo, x);
 #pragma unroll
                     for (int v = 0; v < 4; ++v) M[m][v] = fmaf(cf[m][v], x[v], gm[m][v] * M[m][v]);
                 }
@@ -923,10 +952,10 @@ __device__ __forceinline__ void run_unit(const Params& p, const Unit& U, int32_t
             for (int tau = 0; tau < 2; ++tau) X[tau] += ru[tau];  // U = W S + U0
             f4 y[2] = {z4(), z4()};
             {  // V^T sigma^T
-                const bf8 vp = as_bf8(rv);
-                const s4 v0 = __builtin_bit_cast(s4, uint2{rv.x, rv.y});
+                const s8 v8 = __builtin_bit_cast(s8, rv);
+                const s4 v0 = __builtin_shufflevector(v8, v8, 0, 1, 2, 3);
                 y[0] = mma16(v0, __builtin_bit_cast(s4, uint2{sig[0].x, sig[0].y}), y[0]);
-                y[1] = mma32(vp, as_bf8(sig[1]), y[1]);
+                y[1] = mma32(rv, as_bf8(sig[1]), y[1]);
             }
             qmul(so, X, y);
             store_y(p, tok0, Lc, h, j, lane, y);

@@ -320,12 +320,13 @@ __device__ __forceinline__ void tile_load_w(const Args& p, const TileSrc& src, i
     }
 }
 
-// NA groups of 8 rows of A's chunk (128 bytes per row).
+// NA groups of 8 rows of A's chunk (128 bytes per row).  The rows' offsets are lane offsets: those are what a raw buffer's
+// bound covers by its definition, and it is the bound that keeps rows past M from being read.
 template <int NA>
 __device__ __forceinline__ void tile_load_a(const Args& p, const TileSrc& src, int c, u4 (&a)[NA]) {
     const __amdgpu_buffer_rsrc_t r = tile_rsrc(src.a + (uint64_t)c * 128, src.na - c * 128);
 #pragma unroll
-    for (int e = 0; e < NA; ++e) a[e] = __builtin_amdgcn_raw_buffer_load_b128(r, src.va, 16 * e * (int)p.sa_m, 0);
+    for (int e = 0; e < NA; ++e) a[e] = __builtin_amdgcn_raw_buffer_load_b128(r, src.va + 16 * e * (uint32_t)p.sa_m, 0, 0);
 }
 
 // 16-byte piece j (k = 8 j ..) of row r of the chunk's rows of A in LDS: the 16 rows of one operand read (one j) fall in

@@ -1193,7 +1193,9 @@ TilePlan tile_plan(const w6a16_args* a, const Layout& l, bool packed) {
     auto fits = [&](int ks, int max_w) { return ks == 1 ? t.parts <= max_w : t.parts % 4 == 0 && t.parts / ks <= max_w; };
     // Columns to a wavefront and workgroups to a K range.  Packed: as few workgroups to a K range as hold the parts, and
     // the columns whose rounds cost least.  Planes: always 64 columns (a lane loads four), K spread over more workgroups
-    // while every one of them still gets a CU.
+    // while every one of them still gets a CU and, from two row tiles on, a part has six chunks: their partial tiles then
+    // cost more than what a short loop gains (six products of C = 768, M = 33: 69 us spread, 53 not; C = 2560, five chunks
+    // a part, M = 48: 90.8 / 85.8; C = 4096, eight, M = 64: 133 / 141; one row tile, C = 2560, M = 1: 59.6 / 64.7).
     int64_t best = 0;
     for (int nt = packed ? 1 : 4; nt <= 4; nt *= 2) {
         if (t.mt > 2 && nt < 4) continue;
@@ -1202,7 +1204,9 @@ TilePlan tile_plan(const w6a16_args* a, const Layout& l, bool packed) {
         while (ks < most && !fits(ks, max_w)) ks *= 2;
         if (!fits(ks, max_w)) continue;
         if (!packed)
-            while (ks * 2 <= most && fits(ks * 2, max_w) && t.parts / (ks * 2) >= 4 && w4 * ks * 2 <= cus) ks *= 2;
+            while (ks * 2 <= most && fits(ks * 2, max_w) && t.parts / (ks * 2) >= 4 && w4 * ks * 2 <= cus &&
+                   (t.mt == 1 || chunks >= 6 * t.parts))
+                ks *= 2;
         const int64_t cost = rounds(wgs(t.mt, nt * t.cw) * ks) * (2 * nt + 3 * t.mt);
         if (!best || cost < best) best = cost, t.nt = nt, t.ks = ks;
     }

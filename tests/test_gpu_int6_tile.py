@@ -23,6 +23,9 @@ from test_gpu_int6 import DEV, F16_KERNEL_TOL, KERNEL_TOL, _act, _check, _dev, _
     (1, 40, 64, 16384, 128, 4),      # above 32 rows, K over four workgroups
     (1, 40, 64, 16384, 128, 2),      # over two
     (1, 33, 144, 1024, 128, 1),      # no split
+    (1, 40, 640, 3072, 128, 4),      # planes: three chunks a part, K over as few workgroups as hold the parts
+    (1, 40, 640, 6144, 128, 4),      # six chunks a part, over four
+    (1, 20, 640, 2560, 128, 16),     # up to 32 rows, five chunks a part
     (1, 203, 2560, 320, 64, 2),      # three row tiles, 64 columns
     (1, 64, 16384, 192, 64, 1),      # four row tiles, 64 columns, three chunks
     (1, 203, 10240, 320, 64, 1),     # three row tiles, 128 columns; five chunks over four parts

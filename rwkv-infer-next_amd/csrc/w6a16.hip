@@ -28,6 +28,7 @@
 #include <utility>
 
 #include "w6a16.h"
+#include "w6a16_grid.h"
 #include "wkv7_launch.h"
 
 namespace w6 {
@@ -57,11 +58,9 @@ struct Args {
     uint32_t* cnt;  // K split over workgroups: arrival counters, one per tile; zero between calls
     float* part;    // K split over workgroups: partial tiles [tile][split][rows][16 NT columns]
     int32_t B, M, N, K, group_k, out_dtype, n_strips;
-    // tile kernel: M groups of 16 MT rows, wavefronts that share K, chunks of the longest share, scale groups, log2 of
-    // the workgroups (per M group) of an XCD unit
-    int32_t m_groups, parts, per_part, groups, unit_shift;
-    uint32_t gmul, gone;  // chunk c's scale group is (c gmul >> 32) + c gone
-    uint32_t mgmul;       // x / m_groups is x mgmul >> 31
+    TileGrid grid;                   // tile kernel: M groups of 16 MT rows, columns of a workgroup's column tiles
+    int32_t parts, per_part, groups;  // wavefronts that share K, chunks of the longest share, scale groups
+    Divisor group;                   // chunk c's scale group is c over the chunks of a group
     int32_t out_vec;  // large-M kernel: the output takes 8-byte (16-byte for fp32) stores of 4 adjacent columns
 };
 
@@ -271,7 +270,7 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t tile_rsrc(uint64_t base, int b
 template <int NT, bool PACKED, bool FAR>
 __device__ __forceinline__ void tile_load_w(const Args& p, const TileSrc& src, int c, TileW<NT, PACKED>& s) {
     constexpr int kAll = 0x7FFFFFFF;
-    const int g = (int)(__umulhi((uint32_t)c, p.gmul) + (uint32_t)c * p.gone);  // the chunk's scale group
+    const uint32_t g = quotient((uint32_t)c, p.group);  // the chunk's scale group
     if constexpr (PACKED) {
         const __amdgpu_buffer_rsrc_t lo = tile_rsrc(src.lo + (uint64_t)c * kPackBytes, kAll),
                                      hi = tile_rsrc(src.hi + (uint64_t)c * kPackBytes, kAll),
@@ -463,12 +462,9 @@ __global__ __launch_bounds__(64 * MAXW) void w6a16_tile_kernel(const Args p) {
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int W = (blockDim.x >> 6) / CW, ks = gridDim.z, split = blockIdx.z;  // W: K parts in the workgroup
     const int cw = CW == 1 ? 0 : wv & 1, kp = CW == 1 ? wv : wv >> 1;
-    // A unit of 4 or 8 adjacent column tiles and all its M groups go to one XCD (workgroups are dealt to the XCDs in
-    // turn): neighbouring tiles share cache lines of the weights, the M groups all of them.
-    const int u = blockIdx.x >> 3, v = (int)(((uint64_t)u * p.mgmul) >> 31);  // v = u / m_groups
-    const int us = p.unit_shift, unit = (v >> us) * 8 + (blockIdx.x & 7);
-    const int wtile = ((unit << us) + (v & ((1 << us) - 1))) * NT * CW, tile = wtile + cw * NT;
-    const int mg = u - v * p.m_groups, m0 = mg * 16 * MT, b = blockIdx.y;
+    const TilePos pos = tile_pos(p.grid, blockIdx.x);
+    const int wtile = (int)pos.column * NT * CW, tile = wtile + cw * NT;
+    const int mg = (int)pos.mg, m0 = mg * 16 * MT, b = blockIdx.y;
     if (16 * wtile >= p.N) return;  // uniform over the workgroup
     // this wavefront's chunks g, g + parts, ..
     const int g = split * W + kp, nchunks = p.K / 64;
@@ -586,7 +582,7 @@ __global__ __launch_bounds__(64 * MAXW) void w6a16_tile_kernel(const Args p) {
     // acquire fence: a fence writes back or invalidates the XCD's whole L2, and nothing here is cached there (with one
     // fence per workgroup a call of 256 workgroups took 1 us longer, one of 512 4 us).
     constexpr int kTileFloats = 16 * MT * NC;
-    const int64_t id = ((int64_t)b * p.m_groups + mg) * ((p.N / 16 + NT * CW - 1) / (NT * CW)) + wtile / (NT * CW);
+    const int64_t id = ((int64_t)b * p.grid.m_groups + mg) * ((p.N / 16 + NT * CW - 1) / (NT * CW)) + wtile / (NT * CW);
     float* const part0 = p.part + id * ks * kTileFloats;
     for (int e = threadIdx.x; e < items; e += blockDim.x)
         coherent_store(part0 + split * kTileFloats + e,
@@ -1251,19 +1247,13 @@ int validate(const w6a16_args* a) {
 
 template <class A, int MT, int NA, int NT, int CW, int D, int DA, int MAXW, bool PACKED, bool FAR = false>
 void launch_tile(Args& p, const TilePlan& t, hipStream_t s) {
-    const int tiles = p.N / 16, chunks = p.K / 64, gc = p.group_k / 64;
-    p.m_groups = (p.M + 16 * MT - 1) / (16 * MT);
-    p.mgmul = (uint32_t)(((uint64_t(1) << 31) + p.m_groups - 1) / p.m_groups);
-    p.gone = gc == 1;
-    p.gmul = gc == 1 ? 0 : (uint32_t)(((uint64_t(1) << 32) + gc - 1) / gc);
+    const int chunks = p.K / 64;
+    const uint64_t wgs = tile_grid(p.N / 16, (p.M + 16 * MT - 1) / (16 * MT), NT * CW, p.grid);
+    p.group = divisor(p.group_k / 64);
     p.parts = t.parts;
     p.per_part = (chunks + t.parts - 1) / t.parts;
     p.groups = p.K / p.group_k;
-    // units of eight tiles (a whole line of the planes, a whole block of the packed layout) where they divide evenly
-    // among the XCDs or a workgroup takes eight, else of four
-    const int unit = CW * NT == 8 || ((tiles + 7) / 8) % 8 == 0 ? 8 : 4, units = (tiles + unit - 1) / unit;
-    p.unit_shift = 31 - __builtin_clz(unit / (NT * CW));
-    const dim3 grid(8 * ((units + 7) / 8) * (unit / (NT * CW)) * p.m_groups, p.B, t.ks);
+    const dim3 grid((unsigned)wgs, p.B, t.ks);
     hipLaunchKernelGGL((w6a16_tile_kernel<A, MT, NA, NT, CW, D, DA, MAXW, PACKED, FAR>), grid,
                        dim3(64 * CW * t.parts / t.ks), 0, s, p);
 }

@@ -246,7 +246,7 @@ __device__ __forceinline__ TileSrc tile_src(const Args& p, int b, int m0, int ti
         s.vlo = s.vhi = 16 * lane;
         s.vsc = 16 * i;
     } else {
-        const uint32_t n = min(16 * tile + 4 * i, p.N - 4);
+        const uint32_t n = min(16u * tile + 4u * i, (uint32_t)p.N - 4);  // (unsigned: N up to 2^31 - 16)
         const int hrow = 8 * (q & 1) + 4 * (q >> 1);
         s.lo = reinterpret_cast<uint64_t>(p.lo + (int64_t)b * p.sl_b);
         s.hi = reinterpret_cast<uint64_t>(p.hi + (int64_t)b * p.sh_b);
@@ -465,7 +465,7 @@ __global__ __launch_bounds__(64 * MAXW) void w6a16_tile_kernel(const Args p) {
     const TilePos pos = tile_pos(p.grid, blockIdx.x);
     const int wtile = (int)pos.column * NT * CW, tile = wtile + cw * NT;
     const int mg = (int)pos.mg, m0 = mg * 16 * MT, b = blockIdx.y;
-    if (16 * wtile >= p.N) return;  // uniform over the workgroup
+    if (wtile >= p.N / 16) return;  // uniform over the workgroup
     // this wavefront's chunks g, g + parts, ..
     const int g = split * W + kp, nchunks = p.K / 64;
     const int n = p.per_part - (g + p.parts * (p.per_part - 1) >= nchunks ? 1 : 0);  // >= 1: parts <= chunks
@@ -566,7 +566,7 @@ __global__ __launch_bounds__(64 * MAXW) void w6a16_tile_kernel(const Args p) {
     const int items = min(16 * MT, p.M - m0) * NC, n0 = 16 * wtile;
     auto store = [&](int e, float x) __attribute__((always_inline)) {
         const int r = e / NC, col = e % NC;
-        if (n0 + col >= p.N) return;
+        if (col >= p.N - n0) return;
         const int64_t o = (int64_t)b * p.so_b + (int64_t)(m0 + r) * p.so_m + n0 + col;
         if (p.out_dtype == W6A16_OUT_F16) put_out<true>(p, o, x);
         else put_out<false>(p, o, x);
@@ -1246,31 +1246,36 @@ int validate(const w6a16_args* a) {
 }
 
 template <class A, int MT, int NA, int NT, int CW, int D, int DA, int MAXW, bool PACKED, bool FAR = false>
-void launch_tile(Args& p, const TilePlan& t, hipStream_t s) {
+int launch_tile(Args& p, const TilePlan& t, hipStream_t s) {
     const int chunks = p.K / 64;
     const uint64_t wgs = tile_grid(p.N / 16, (p.M + 16 * MT - 1) / (16 * MT), NT * CW, p.grid);
+    if (wgs >> 34) return WKV7_ERR_SHAPE;
     p.group = divisor(p.group_k / 64);
     p.parts = t.parts;
     p.per_part = (chunks + t.parts - 1) / t.parts;
     p.groups = p.K / p.group_k;
-    const dim3 grid((unsigned)wgs, p.B, t.ks);
-    hipLaunchKernelGGL((w6a16_tile_kernel<A, MT, NA, NT, CW, D, DA, MAXW, PACKED, FAR>), grid,
-                       dim3(64 * CW * t.parts / t.ks), 0, s, p);
+    const uint32_t block = 64 * CW * t.parts / t.ks, most = launch_limit(block);
+    for (uint64_t x = 0; x < wgs; x += most) {
+        p.grid.first = (uint32_t)(x / 8);
+        hipLaunchKernelGGL((w6a16_tile_kernel<A, MT, NA, NT, CW, D, DA, MAXW, PACKED, FAR>),
+                           dim3((unsigned)std::min<uint64_t>(wgs - x, most), p.B, t.ks), dim3(block), 0, s, p);
+    }
+    return WKV7_OK;
 }
 
 // D chunks of weights and DA of A in flight: as many as the registers of MAXW wavefronts allow.
 template <class A, int NA, bool PACKED>
-void launch_tile_one(Args& p, const TilePlan& t, hipStream_t s) {  // one row tile
+int launch_tile_one(Args& p, const TilePlan& t, hipStream_t s) {  // one row tile
     if constexpr (PACKED) {
         if (t.nt == 1) return launch_tile<A, 1, NA, 1, 1, 4, 4, 16, true>(p, t, s);
         if (t.nt == 2) return launch_tile<A, 1, NA, 2, 1, 4, 4, 16, true>(p, t, s);
     }
     if (t.parts / t.ks > 8) return launch_tile<A, 1, NA, 4, 1, 2, 2, 16, PACKED>(p, t, s);
-    launch_tile<A, 1, NA, 4, 1, 4, 4, 8, PACKED>(p, t, s);
+    return launch_tile<A, 1, NA, 4, 1, 4, 4, 8, PACKED>(p, t, s);
 }
 
 template <class A, bool PACKED>
-void launch_tile_plan(Args& p, const TilePlan& t, hipStream_t s) {
+int launch_tile_plan(Args& p, const TilePlan& t, hipStream_t s) {
     if constexpr (!PACKED)
         if (t.far) return launch_tile<A, 1, 2, 4, 1, 2, 2, 16, false, true>(p, t, s);
     if (t.mt == 1) return p.M <= 8 ? launch_tile_one<A, 1, PACKED>(p, t, s) : launch_tile_one<A, 2, PACKED>(p, t, s);
@@ -1283,24 +1288,21 @@ void launch_tile_plan(Args& p, const TilePlan& t, hipStream_t s) {
     }
     if (t.mt == 3)
         return t.cw == 2 ? launch_tile<A, 3, 6, 4, 2, 2, 1, 8, PACKED>(p, t, s) : launch_tile<A, 3, 6, 4, 1, 2, 1, 8, PACKED>(p, t, s);
-    t.cw == 2 ? launch_tile<A, 4, 8, 4, 2, 2, 1, 8, PACKED>(p, t, s) : launch_tile<A, 4, 8, 4, 1, 2, 1, 8, PACKED>(p, t, s);
+    return t.cw == 2 ? launch_tile<A, 4, 8, 4, 2, 2, 1, 8, PACKED>(p, t, s) : launch_tile<A, 4, 8, 4, 1, 2, 1, 8, PACKED>(p, t, s);
 }
 
 // The kernel for the call's shape and layout, with activations of type A.
 template <class A>
-void launch_matmul(Args& p, const w6a16_args* a, const Layout& l, hipStream_t s) {
+int launch_matmul(Args& p, const w6a16_args* a, const Layout& l, hipStream_t s) {
     const bool packed = a->format == W6A16_FORMAT_PACKED;
     if (l.big) {
         const int tiles = ((p.M + kBigTile - 1) / kBigTile) * ((p.N + kBigTile - 1) / kBigTile);
         hipLaunchKernelGGL(w6a16_big_kernel<A>, dim3(tiles, 1, p.B), dim3(512), 0, s, p);
-        return;
+        return WKV7_OK;
     }
     auto launch = [&](Args& q, const w6a16_args* shape) {
         const TilePlan t = tile_plan(shape, l, packed);
-        if (packed)
-            launch_tile_plan<A, true>(q, t, s);
-        else
-            launch_tile_plan<A, false>(q, t, s);
+        return packed ? launch_tile_plan<A, true>(q, t, s) : launch_tile_plan<A, false>(q, t, s);
     };
     if (p.sa_m < (1 << 24)) return launch(p, a);
     // rows so far apart that a workgroup's 64 do not fit a buffer's 32-bit offsets: row by row
@@ -1317,8 +1319,9 @@ void launch_matmul(Args& p, const w6a16_args* a, const Layout& l, hipStream_t s)
             q.out = static_cast<char*>(p.out) + o * (p.out_dtype == W6A16_OUT_F32 ? 4 : 2);
             q.B = q.M = 1;
             q.sa_m = p.K;
-            launch(q, &row);
+            if (const int rc = launch(q, &row)) return rc;
         }
+    return WKV7_OK;
 }
 
 }  // namespace
@@ -1409,10 +1412,9 @@ int w6a16_matmul(const w6a16_args* a, void* stream) {
     p.n_strips = l.n_strips;
     p.out_vec = w6::aligned16(a->out) && a->out_row_stride % 8 == 0 && a->out_batch_stride % 8 == 0;
     const hipStream_t s = static_cast<hipStream_t>(stream);
-    if (a->a_dtype == W6A16_IN_F16)
-        w6::launch_matmul<w6::ActF16>(p, a, l, s);
-    else
-        w6::launch_matmul<w6::ActBF16>(p, a, l, s);
+    if (const int bad = a->a_dtype == W6A16_IN_F16 ? w6::launch_matmul<w6::ActF16>(p, a, l, s)
+                                                   : w6::launch_matmul<w6::ActBF16>(p, a, l, s))
+        return bad;
     return static_cast<int>(hipGetLastError());
 }
 

@@ -32,6 +32,7 @@ W6_HOST_DEVICE uint32_t quotient(uint32_t x, Divisor d) { return (uint32_t)(((ui
 struct TileGrid {
     Divisor by_m_groups;
     uint32_t m_groups, unit_shift;  // log2 of a unit's workgroups (per M group)
+    uint32_t first;                 // this launch's first workgroup, over 8
 };
 
 struct TilePos {
@@ -39,20 +40,23 @@ struct TilePos {
 };
 
 W6_HOST_DEVICE TilePos tile_pos(const TileGrid& g, uint32_t x) {
-    const uint32_t u = x >> 3, v = quotient(u, g.by_m_groups), mask = (1u << g.unit_shift) - 1;
+    const uint32_t u = g.first + (x >> 3), v = quotient(u, g.by_m_groups), mask = (1u << g.unit_shift) - 1;
     return {u - v * g.m_groups, ((((v >> g.unit_shift) * 8 + (x & 7)) << g.unit_shift) + (v & mask))};
 }
 
-// The grid for `tiles` 16-column tiles, wg of them to a workgroup; returns its workgroups.  Units of eight tiles (a whole
+// The grid for `tiles` 16-column tiles, wg of them to a workgroup; returns its workgroups (below 2^34: u < 2^31).  Units of eight tiles (a whole
 // line of the planes, a whole block of the packed layout) where they divide evenly among the XCDs or a workgroup takes
 // eight, else of four.
 inline uint64_t tile_grid(uint32_t tiles, uint32_t m_groups, uint32_t wg, TileGrid& g) {
     const uint32_t unit = wg == 8 || ((tiles + 7) / 8) % 8 == 0 ? 8 : 4, units = (tiles + unit - 1) / unit;
     g.by_m_groups = divisor(m_groups);
     g.m_groups = m_groups;
-    g.unit_shift = 0;
+    g.unit_shift = g.first = 0;
     while ((wg << g.unit_shift) < unit) ++g.unit_shift;
     return ((uint64_t)((units + 7) / 8) << g.unit_shift) * m_groups * 8;
 }
+
+// Workgroups of `block` threads that one launch may have: the work-items of a grid's x dimension are counted in 32 bits.
+inline uint32_t launch_limit(uint32_t block) { return 0x7FFFFFFFu / block & ~7u; }
 
 }  // namespace w6

@@ -85,3 +85,32 @@ def test_planes_past_2_gb():
         P = I6.int6_matmul(a, *part, g, out_dtype=torch.float32)
         torch.cuda.synchronize()
         assert torch.equal(C[:, n0:n0 + 256], P), n0
+
+
+@pytest.mark.parametrize("packed", [False, True])
+def test_rows_beyond_one_launch(monkeypatch, packed):
+    """2^28 + 40 rows of one column tile: more workgroups than one launch takes.  65536 rows, over and over, and 40 others
+    at the end equal the same rows multiplied alone."""
+    from rwkv_next_amd.kernels import int6_gemm as I6
+    monkeypatch.setattr(I6, "MAX_M", 1 << 30)
+    N, K, g, R = 16, 64, 64, 1 << 16
+    M = (1 << 28) + 40
+    if torch.cuda.mem_get_info()[0] < 60 << 30:
+        pytest.skip("needs 60 GB of device memory")
+    say("w6a16 rows beyond one launch", dict(packed=packed))
+    gen = torch.Generator(device=DEV).manual_seed(13)
+    lo = torch.randint(0, 256, (K // 2, N), device=DEV, dtype=torch.uint8, generator=gen)
+    hi = torch.randint(0, 256, (K // 4, N), device=DEV, dtype=torch.uint8, generator=gen)
+    sc = (torch.rand(K // g, N, device=DEV, generator=gen) * 0.05 + 0.002).half()
+    w = (I6.prepack_int6(lo, hi, sc, g),) if packed else (lo, hi, sc, g)
+    base = torch.randn(R, K, device=DEV, generator=gen).to(torch.bfloat16)
+    end = torch.randn(40, K, device=DEV, generator=gen).to(torch.bfloat16)
+    a = torch.empty(M, K, dtype=torch.bfloat16, device=DEV)
+    a[:M - 40].view(-1, R, K).copy_(base)
+    a[M - 40:] = end
+    C = I6.int6_matmul(a, *w)
+    want, last = I6.int6_matmul(base, lo, hi, sc, g), I6.int6_matmul(end, lo, hi, sc, g)
+    torch.cuda.synchronize()
+    for part in C[:M - 40].view(-1, R, N).split(256):
+        assert bool((part == want).all())
+    assert torch.equal(C[M - 40:], last)

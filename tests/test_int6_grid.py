@@ -36,35 +36,45 @@ static void check_division(uint32_t d, uint32_t last) {
     for (uint64_t n = last - 100; n <= last; ++n) at(n);
 }
 
-static void check_grid(uint32_t tiles, uint32_t m_groups, uint32_t wg) {
+// The tiles of a call, over its launches as the host cuts them: each (M group, column) once, and none else but past the
+// last column; of large grids the edges of every M group's run, of the launches and of the grid.
+static void check_grid(uint32_t tiles, uint32_t m_groups, uint32_t wg, uint32_t block) {
     TileGrid g;
-    const uint64_t n = tile_grid(tiles, m_groups, wg, g), columns = (tiles + wg - 1) / wg;
-    if (n % 8 || n < columns * m_groups || n >> 34) { printf("%llu workgroups\n", (unsigned long long)n); exit(1); }
-    std::vector<bool> seen;
+    const uint64_t n = tile_grid(tiles, m_groups, wg, g), columns = (tiles + wg - 1) / wg, most = launch_limit(block);
+    auto fail = [&](const char* what, uint64_t x) {
+        printf("tiles %u, M groups %u, %u to a workgroup, %u threads: %s (%llu)\n", tiles, m_groups, wg, block, what,
+               (unsigned long long)x);
+        exit(1);
+    };
+    if (n % 8 || n < columns * m_groups || n >> 34) fail("workgroups", n);
+    if (most < 8 || most % 8 || (uint64_t)most * block > 0xFFFFFFFFu || (uint64_t)most * 2 * block < 0x80000000u) fail("a launch", most);
     const bool all = n <= (1u << 24);
-    if (all) seen.assign(columns * m_groups, false);
-    auto at = [&](uint32_t x) {
-        const TilePos p = tile_pos(g, x);
-        const uint32_t u = x / 8, v = u / m_groups, per = 1u << g.unit_shift;
-        if (p.mg >= m_groups || p.mg != u % m_groups || p.column != (v / per * 8 + x % 8) * per + v % per) {
-            printf("tiles %u, M groups %u, %u to a workgroup: workgroup %u is (%u, %u)\n", tiles, m_groups, wg, x, p.mg, p.column);
-            exit(1);
-        }
+    std::vector<bool> seen(all ? columns * m_groups : 0);
+    auto at = [&](uint64_t x) {
+        g.first = (uint32_t)(x / most * most / 8);
+        const TilePos p = tile_pos(g, (uint32_t)(x % most));
+        const uint64_t u = x / 8, v = u / m_groups, per = 1u << g.unit_shift;
+        if (p.mg != u % m_groups || p.column != (v / per * 8 + x % 8) * per + v % per) fail("another place", x);
+        if ((uint64_t)p.column * wg > 0x7FFFFFFF) fail("a column tile past 2^31", x);
         if (all && p.column < columns) {
-            if (seen[p.column * (uint64_t)m_groups + p.mg]) { printf("twice\n"); exit(1); }
+            if (seen[p.column * (uint64_t)m_groups + p.mg]) fail("twice", x);
             seen[p.column * (uint64_t)m_groups + p.mg] = true;
         }
     };
     if (all) {
-        for (uint64_t x = 0; x < n; ++x) at((uint32_t)x);
-        for (bool s : seen)
-            if (!s) { printf("tiles %u, M groups %u, %u to a workgroup: a tile without a workgroup\n", tiles, m_groups, wg); exit(1); }
-    } else if (n <= 0x7FFFFFFF) {  // the edges of every M group's run, and the end
-        for (uint64_t u = 0; u < n / 8; u += m_groups)
-            for (int e = -1; e <= 1; ++e)
-                if (u + e < n / 8) at((uint32_t)(8 * (u + e) + rnd() % 8));
-        for (uint64_t x = n - 4096; x < n; ++x) at((uint32_t)x);
+        for (uint64_t x = 0; x < n; ++x) at(x);
+        for (size_t k = 0; k < seen.size(); ++k)
+            if (!seen[k]) fail("a tile without a workgroup", k);
+        return;
     }
+    const uint64_t step = m_groups * (n / 8 / m_groups / 100000 + 1);
+    for (uint64_t u = 0; u < n / 8; u += step)
+        for (int e = -1; e <= 1; ++e)
+            if (u + e < n / 8) at(8 * (u + e) + rnd() % 8);
+    for (uint64_t x = most; x < n; x += most)
+        for (int e = -9; e <= 9; ++e)
+            if (x + e < n) at(x + e);
+    for (uint64_t x = n - 4096; x < n; ++x) at(x);
 }
 
 int main(int argc, char** argv) {
@@ -78,12 +88,17 @@ int main(int argc, char** argv) {
         const uint32_t sizes[] = {1, 2, 3, 4, 5, 7, 8, 9, 16, 20, 31, 48, 64, 65, 100, 160, 1021, 1024, 4096};
         for (uint32_t tiles : sizes)
             for (uint32_t m : sizes)
-                for (uint32_t wg : {1u, 2u, 4u, 8u}) check_grid(tiles, m, wg);
+                for (uint32_t wg : {1u, 2u, 4u, 8u}) check_grid(tiles, m, wg, 512);
         // rows past which a 31-bit reciprocal of the M groups is off by one
         for (uint32_t wg : {4u, 8u}) {
-            check_grid(4096, 6219, wg), check_grid(1024, 11627, wg), check_grid(1024, 11727, wg);
-            check_grid(256, 23831, wg), check_grid(64, 47240, wg), check_grid(1, 3000017, wg);
+            check_grid(4096, 6219, wg, 512), check_grid(1024, 11627, wg, 512), check_grid(1024, 11727, wg, 512);
+            check_grid(256, 23831, wg, 512), check_grid(64, 47240, wg, 512), check_grid(1, 3000017, wg, 512);
         }
+        // 2^32 work-items and more: M = 67.2 M rows of 512 columns of A (16 columns of weights), 16 and 64 rows of N = 2^30
+        // (K = 320) and of N = 2^31 - 16 (K = 64), which a call on a card of 288 GB can have
+        check_grid(1, 1050001, 4, 512), check_grid(1, 1050001, 8, 512);
+        for (uint32_t m : {1u, 4u, 16u}) check_grid(1u << 26, m, 4, 256), check_grid((1u << 27) - 1, m, 4, 64);
+        check_grid(1u << 22, 16, 4, 256), check_grid(1u << 26, 1, 8, 1024);
     }
     printf("fine\n");
 }

@@ -221,12 +221,12 @@ struct TileW<NT, false> {
 
 // The wavefront's loads: wave-uniform 64-bit bases (moved from chunk to chunk on the scalar unit) and 32-bit per-lane
 // offsets fixed for the call, through raw buffers.  A's buffer ends with its last valid row: rows past M read zeros.
-// (64-bit lane offsets for planes whose 32 rows span 2 GB: FAR.)
+// (64-bit lane offsets, of the planes and of the scales, for planes whose 32 rows span 2 GB: FAR.)
 struct TileSrc {
     uint64_t a, lo, hi, sc;
     int na;  // bytes from the first row's start to the last valid row's end
     uint32_t va, vlo, vhi, vsc;
-    int64_t flo, fhi;
+    int64_t flo, fhi, fsc;
 };
 
 template <int MT, bool PACKED, bool FAR>
@@ -254,11 +254,12 @@ __device__ __forceinline__ TileSrc tile_src(const Args& p, int b, int m0, int ti
         if constexpr (FAR) {
             s.flo = (int64_t)(8 * q) * p.N + n;
             s.fhi = (int64_t)hrow * p.N + n;
+            s.fsc = 2 * (int64_t)n;
         } else {
             s.vlo = (uint32_t)(8 * q) * p.N + n;
             s.vhi = (uint32_t)hrow * p.N + n;
+            s.vsc = 2 * n;
         }
-        s.vsc = 2 * n;
     }
     return s;
 }
@@ -298,13 +299,15 @@ __device__ __forceinline__ void tile_load_w(const Args& p, const TileSrc& src, i
         s.sc[0] = z.x, s.sc[1] = z.y;
     } else {
         const uint64_t lo = src.lo + (uint64_t)c * 32 * (uint64_t)p.N, hi = src.hi + (uint64_t)c * 16 * (uint64_t)p.N;
+        const uint64_t sc = src.sc + (uint64_t)g * 2 * (uint64_t)p.N;
         if constexpr (FAR) {
+            typedef const __attribute__((address_space(1))) uint32_t* Words;
 #pragma unroll
-            for (int e = 0; e < 8; ++e)
-                s.lo[e] = *reinterpret_cast<const __attribute__((address_space(1))) uint32_t*>(lo + (uint64_t)(src.flo + (int64_t)e * p.N));
+            for (int e = 0; e < 8; ++e) s.lo[e] = *reinterpret_cast<Words>(lo + (uint64_t)(src.flo + (int64_t)e * p.N));
 #pragma unroll
-            for (int e = 0; e < 4; ++e)
-                s.hd[e] = *reinterpret_cast<const __attribute__((address_space(1))) uint32_t*>(hi + (uint64_t)(src.fhi + (int64_t)e * p.N));
+            for (int e = 0; e < 4; ++e) s.hd[e] = *reinterpret_cast<Words>(hi + (uint64_t)(src.fhi + (int64_t)e * p.N));
+#pragma unroll
+            for (int d = 0; d < 2; ++d) s.sc[d] = reinterpret_cast<Words>(sc + (uint64_t)src.fsc)[d];  // (4-byte aligned)
         } else {
 #pragma unroll
             for (int e = 0; e < 8; ++e)
@@ -312,10 +315,9 @@ __device__ __forceinline__ void tile_load_w(const Args& p, const TileSrc& src, i
 #pragma unroll
             for (int e = 0; e < 4; ++e)
                 s.hd[e] = __builtin_amdgcn_raw_buffer_load_b32(tile_rsrc(hi, kAll), src.vhi, e * p.N, 0);
+            const uint2 z = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(tile_rsrc(sc, kAll), src.vsc, 0, 0));
+            s.sc[0] = z.x, s.sc[1] = z.y;
         }
-        const uint2 z = __builtin_bit_cast(
-            uint2, __builtin_amdgcn_raw_buffer_load_b64(tile_rsrc(src.sc + (uint64_t)g * 2 * (uint64_t)p.N, kAll), src.vsc, 0, 0));
-        s.sc[0] = z.x, s.sc[1] = z.y;
     }
 }
 

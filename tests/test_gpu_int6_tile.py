@@ -68,23 +68,28 @@ def test_rows_far_apart():
     _check(C, a, lo, hi, sc, g, KERNEL_TOL)
 
 
-def test_planes_past_2_gb():
-    """2^26 + 80 columns: the planes' rows of one chunk span more than 2 GB.  Columns from both ends equal the same
-    columns multiplied alone."""
+@pytest.mark.parametrize("M,N", [
+    (2, (1 << 26) + 80),    # the planes' rows of one chunk span more than 2 GB
+    (17, (1 << 26) + 80),   # more rows than one row tile
+    (2, (1 << 30) + 80),    # and so do the scales of one group
+])
+def test_planes_past_2_gb(M, N):
+    """Columns from both ends and the middle, against the exact product."""
     from rwkv_next_amd.kernels import int6_gemm as I6
-    M, N, K, g = 2, (1 << 26) + 80, 64, 64
-    say("w6a16 planes past 2 GB")
+    K, g = 64, 64
+    if torch.cuda.mem_get_info()[0] < 96 * N:
+        pytest.skip("needs 96 bytes a column of device memory")
+    say("w6a16 planes past 2 GB", dict(M=M, N=N))
     gen = torch.Generator(device=DEV).manual_seed(12)
     lo = torch.randint(0, 256, (K // 2, N), device=DEV, dtype=torch.uint8, generator=gen)
     hi = torch.randint(0, 256, (K // 4, N), device=DEV, dtype=torch.uint8, generator=gen)
-    sc = (torch.rand(K // g, N, device=DEV, generator=gen) * 0.05 + 0.002).half()
+    sc = torch.empty(K // g, N, dtype=torch.float16, device=DEV).uniform_(0.002, 0.05, generator=gen)
     a = torch.randn(M, K, device=DEV, generator=gen).to(torch.bfloat16)
     C = I6.int6_matmul(a, lo, hi, sc, g, out_dtype=torch.float32)
+    torch.cuda.synchronize()
     for n0 in (0, N // 32 * 16, N - 256):
-        part = [x[:, n0:n0 + 256].contiguous() for x in (lo, hi, sc)]
-        P = I6.int6_matmul(a, *part, g, out_dtype=torch.float32)
-        torch.cuda.synchronize()
-        assert torch.equal(C[:, n0:n0 + 256], P), n0
+        part = [x[:, n0:n0 + 256].cpu().numpy()[None] for x in (lo, hi, sc)]
+        _check(C[None, :, n0:n0 + 256], a.cpu()[None], *part, g, KERNEL_TOL)
 
 
 @pytest.mark.parametrize("packed", [False, True])

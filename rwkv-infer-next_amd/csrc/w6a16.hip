@@ -221,21 +221,33 @@ struct TileW<NT, false> {
 
 // The wavefront's loads: wave-uniform 64-bit bases (moved from chunk to chunk on the scalar unit) and 32-bit per-lane
 // offsets fixed for the call, through raw buffers.  A's buffer ends with its last valid row: rows past M read zeros.
-// (64-bit lane offsets, of the planes and of the scales, for planes whose 32 rows span 2 GB: FAR.)
+// FAR, for planes whose 32 rows span 2 GB and for rows of A so far apart that a workgroup's 64 do: 64-bit lane offsets of
+// the planes and their scales, 64-bit addresses of A's rows (rows past M read the last one; they only feed outputs that
+// are not stored).
 struct TileSrc {
     uint64_t a, lo, hi, sc;
     int na;  // bytes from the first row's start to the last valid row's end
     uint32_t va, vlo, vhi, vsc;
     int64_t flo, fhi, fsc;
+    uint64_t fa[2];
 };
 
 template <int MT, bool PACKED, bool FAR>
 __device__ __forceinline__ TileSrc tile_src(const Args& p, int b, int m0, int tile, int row0) {
     const int lane = threadIdx.x & 63, i = lane & 15, q = lane >> 4;
     TileSrc s;
-    s.a = reinterpret_cast<uint64_t>(p.a + (int64_t)b * p.sa_b + (int64_t)m0 * p.sa_m);
-    s.na = (int)(((int64_t)(min(p.M - m0, 16 * MT) - 1) * p.sa_m + p.K) * 2);
-    s.va = (uint32_t)(row0 + (lane >> 3)) * (uint32_t)p.sa_m * 2 + 16 * (lane & 7);
+    if constexpr (FAR) {
+        static_assert(MT == 1, "two groups of eight rows");
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const int m = min(m0 + row0 + 8 * e + (lane >> 3), p.M - 1);
+            s.fa[e] = reinterpret_cast<uint64_t>(p.a + (int64_t)b * p.sa_b + (int64_t)m * p.sa_m) + 16 * (lane & 7);
+        }
+    } else {
+        s.a = reinterpret_cast<uint64_t>(p.a + (int64_t)b * p.sa_b + (int64_t)m0 * p.sa_m);
+        s.na = (int)(((int64_t)(min(p.M - m0, 16 * MT) - 1) * p.sa_m + p.K) * 2);
+        s.va = (uint32_t)(row0 + (lane >> 3)) * (uint32_t)p.sa_m * 2 + 16 * (lane & 7);
+    }
     if constexpr (PACKED) {
         const int strip = tile >> 3, t = tile & 7;
         const uint64_t blk =
@@ -323,11 +335,18 @@ __device__ __forceinline__ void tile_load_w(const Args& p, const TileSrc& src, i
 
 // NA groups of 8 rows of A's chunk (128 bytes per row).  The rows' offsets are lane offsets: those are what a raw buffer's
 // bound covers by its definition, and it is the bound that keeps rows past M from being read.
-template <int NA>
+template <int NA, bool FAR>
 __device__ __forceinline__ void tile_load_a(const Args& p, const TileSrc& src, int c, u4 (&a)[NA]) {
-    const __amdgpu_buffer_rsrc_t r = tile_rsrc(src.a + (uint64_t)c * 128, src.na - c * 128);
+    if constexpr (FAR) {
+        static_assert(NA == 2, "two groups of eight rows");
 #pragma unroll
-    for (int e = 0; e < NA; ++e) a[e] = __builtin_amdgcn_raw_buffer_load_b128(r, src.va + 16 * e * (uint32_t)p.sa_m, 0, 0);
+        for (int e = 0; e < NA; ++e)
+            a[e] = *reinterpret_cast<const __attribute__((address_space(1))) u4*>(src.fa[e] + (uint64_t)c * 128);
+    } else {
+        const __amdgpu_buffer_rsrc_t r = tile_rsrc(src.a + (uint64_t)c * 128, src.na - c * 128);
+#pragma unroll
+        for (int e = 0; e < NA; ++e) a[e] = __builtin_amdgcn_raw_buffer_load_b128(r, src.va + 16 * e * (uint32_t)p.sa_m, 0, 0);
+    }
 }
 
 // 16-byte piece j (k = 8 j ..) of row r of the chunk's rows of A in LDS: the 16 rows of one operand read (one j) fall in
@@ -455,6 +474,7 @@ __device__ __forceinline__ float tile_sum(const float* part, int W, int ks, int 
 template <class A, int MT, int NA, int NT, int CW, int D, int DA, int MAXW, bool PACKED, bool FAR>
 __global__ __launch_bounds__(64 * MAXW) void w6a16_tile_kernel(const Args p) {
     static_assert(PACKED || NT == 4, "planes: four column tiles");
+    static_assert(!FAR || (MT == 1 && NT == 4 && CW == 1), "far: 16 rows, 64 columns to a workgroup");
     static_assert(D % DA == 0, "stage rings");
     static_assert(CW == 1 || (CW == 2 && D == 2 && DA == 1 && NA % 2 == 0), "one or two column wavefronts");
     constexpr int kA = 1024 * NA, kPart = MAXW * MT * NT * 1024, kStage = MAXW * kA;  // (CW = 2: two buffers a K part)
@@ -503,7 +523,7 @@ __global__ __launch_bounds__(64 * MAXW) void w6a16_tile_kernel(const Args p) {
 #pragma unroll
     for (int j = 0; j < D; ++j) {
         tile_load_w<NT, PACKED, FAR>(p, src, chunk(j), w[j]);
-        if (j < DA) tile_load_a<NW>(p, src, chunk(j), a[j]);
+        if (j < DA) tile_load_a<NW, FAR>(p, src, chunk(j), a[j]);
     }
     __builtin_amdgcn_sched_barrier(0);
     int base = 0;
@@ -517,7 +537,7 @@ __global__ __launch_bounds__(64 * MAXW) void w6a16_tile_kernel(const Args p) {
 #pragma unroll
             for (int j = 0; j < D; ++j) {
                 stage(a[j % DA]);
-                tile_load_a<NW>(p, src, chunk(base + j + DA), a[j % DA]);
+                tile_load_a<NW, FAR>(p, src, chunk(base + j + DA), a[j % DA]);
                 __builtin_amdgcn_sched_barrier(0);
                 work(w[j], 0);
                 tile_load_w<NT, PACKED, FAR>(p, src, chunk(base + D + j), w[j]);
@@ -527,21 +547,21 @@ __global__ __launch_bounds__(64 * MAXW) void w6a16_tile_kernel(const Args p) {
         for (int j = 0; j < D; ++j)
             if (base + j < n) {
                 stage(a[j % DA]);
-                if (j + DA < D) tile_load_a<NW>(p, src, chunk(base + j + DA), a[j % DA]);
+                if (j + DA < D) tile_load_a<NW, FAR>(p, src, chunk(base + j + DA), a[j % DA]);
                 __builtin_amdgcn_sched_barrier(0);
                 work(w[j], 0);
             }
     } else {
         // chunk j's rows lie in buffer j & 1; the next chunk's are written beside its work and met at the barrier
         write(a[0], 0);
-        tile_load_a<NW>(p, src, chunk(1), a[0]);
+        tile_load_a<NW, FAR>(p, src, chunk(1), a[0]);
         __syncthreads();
         const int steps = p.per_part;  // uniform over the workgroup; a part with a chunk less skips its last one
         for (; base + D < steps; base += D)
 #pragma unroll
             for (int j = 0; j < D; ++j) {
                 write(a[0], (j + 1) & 1);
-                tile_load_a<NW>(p, src, chunk(base + j + 2), a[0]);
+                tile_load_a<NW, FAR>(p, src, chunk(base + j + 2), a[0]);
                 __builtin_amdgcn_sched_barrier(0);
                 work(w[j], j & 1);
                 tile_load_w<NT, PACKED, FAR>(p, src, chunk(base + D + j), w[j]);
@@ -1208,7 +1228,11 @@ TilePlan tile_plan(const w6a16_args* a, const Layout& l, bool packed) {
         const int64_t cost = rounds(wgs(t.mt, nt * t.cw) * ks) * (2 * nt + 3 * t.mt);
         if (!best || cost < best) best = cost, t.nt = nt, t.ks = ks;
     }
-    t.far = !packed && a->N >= (1 << 26);
+    // Planes whose 32 rows span 2 GB, rows of A of which 64 do: 16 rows and 64 columns to a workgroup, with 64-bit
+    // addresses, and the same parts, so the same bits as for the same rows packed or side by side.  (More than 16 parts
+    // come only with few tiles, whose counters and partial tiles have room.)
+    t.far = (!packed && a->N >= (1 << 26)) || (a->M > 1 ? a->a_row_stride : a->K) >= (1 << 24);
+    if (t.far) t.mt = 1, t.nt = 4, t.cw = 1, t.ks = t.parts > 16 ? 2 : 1;
     return t;
 }
 
@@ -1278,8 +1302,7 @@ int launch_tile_one(Args& p, const TilePlan& t, hipStream_t s) {  // one row til
 
 template <class A, bool PACKED>
 int launch_tile_plan(Args& p, const TilePlan& t, hipStream_t s) {
-    if constexpr (!PACKED)
-        if (t.far) return launch_tile<A, 1, 2, 4, 1, 2, 2, 16, false, true>(p, t, s);
+    if (t.far) return launch_tile<A, 1, 2, 4, 1, 2, 2, 16, PACKED, true>(p, t, s);
     if (t.mt == 1) return p.M <= 8 ? launch_tile_one<A, 1, PACKED>(p, t, s) : launch_tile_one<A, 2, PACKED>(p, t, s);
     if (t.mt == 2) {
         if constexpr (PACKED) {
@@ -1302,28 +1325,8 @@ int launch_matmul(Args& p, const w6a16_args* a, const Layout& l, hipStream_t s) 
         hipLaunchKernelGGL(w6a16_big_kernel<A>, dim3(tiles, 1, p.B), dim3(512), 0, s, p);
         return WKV7_OK;
     }
-    auto launch = [&](Args& q, const w6a16_args* shape) {
-        const TilePlan t = tile_plan(shape, l, packed);
-        return packed ? launch_tile_plan<A, true>(q, t, s) : launch_tile_plan<A, false>(q, t, s);
-    };
-    if (p.sa_m < (1 << 24)) return launch(p, a);
-    // rows so far apart that a workgroup's 64 do not fit a buffer's 32-bit offsets: row by row
-    w6a16_args row = *a;
-    row.M = row.B = row.split_k = 1;
-    for (int b = 0; b < a->B; ++b)
-        for (int m = 0; m < a->M; ++m) {
-            Args q = p;
-            q.a += (int64_t)b * p.sa_b + (int64_t)m * p.sa_m;
-            q.lo += (int64_t)b * p.sl_b;
-            if (q.hi) q.hi += (int64_t)b * p.sh_b;
-            q.sc += (int64_t)b * p.ss_b;
-            const int64_t o = (int64_t)b * p.so_b + (int64_t)m * p.so_m;
-            q.out = static_cast<char*>(p.out) + o * (p.out_dtype == W6A16_OUT_F32 ? 4 : 2);
-            q.B = q.M = 1;
-            q.sa_m = p.K;
-            if (const int rc = launch(q, &row)) return rc;
-        }
-    return WKV7_OK;
+    const TilePlan t = tile_plan(a, l, packed);
+    return packed ? launch_tile_plan<A, true>(p, t, s) : launch_tile_plan<A, false>(p, t, s);
 }
 
 }  // namespace

@@ -9,7 +9,7 @@ from gpu_util import say
 torch = pytest.importorskip("torch")
 pytestmark = pytest.mark.gpu
 
-from test_gpu_int6 import DEV, F16_KERNEL_TOL, KERNEL_TOL, _act, _check, _dev, _weights  # noqa: E402
+from test_gpu_int6 import DEV, F16_KERNEL_TOL, KERNEL_TOL, _act, _check, _dev, _split, _weights  # noqa: E402
 
 
 @pytest.mark.parametrize("B,M,N,K,g,split", [
@@ -49,22 +49,31 @@ def test_tile_shapes(B, M, N, K, g, split, dtype):
     _check(C, a, lo, hi, sc, g, KERNEL_TOL if dtype == "bf16" else F16_KERNEL_TOL)
 
 
-def test_rows_far_apart():
-    """A row stride of 2^24 elements: a workgroup's rows span more than its buffer's 32-bit offsets reach."""
+@pytest.mark.parametrize("B,M,N,K,g,split", [
+    (2, 3, 80, 256, 64, None),      # one row tile, as many parts as chunks
+    (1, 40, 144, 2048, 128, None),  # eight parts, where 16 rows would have 16
+    (1, 3, 64, 16384, 128, 32),     # 32 parts over two workgroups
+    (1, 17, 80, 16384, 128, 32),    # two row tiles, 32 parts
+])
+def test_rows_far_apart(B, M, N, K, g, split):
+    """A row stride of 2^24 elements: a workgroup's rows span more than its buffer's 32-bit offsets reach.  The same bits
+    as the same rows side by side."""
     from rwkv_next_amd.kernels import int6_gemm as I6
-    B, M, N, K, g = 2, 3, 80, 256, 64
-    say("w6a16 rows far apart")
-    rng = np.random.default_rng(11)
+    say("w6a16 rows far apart", dict(B=B, M=M, N=N, K=K))
+    rng = np.random.default_rng(11 + M)
     lo, hi, sc = _weights(rng, B, K, N, g)
     a = _act(rng, B, M, K)
     Ld, Hd, Sd = _dev(lo, hi, sc)
     far = torch.zeros(B * M, 1 << 24, dtype=torch.bfloat16, device=DEV)
     far[:, :K] = a.reshape(B * M, K).to(DEV)
     view = far.view(B, M, 1 << 24)[:, :, :K]
-    C = I6.int6_matmul(view, Ld, Hd, Sd, g, out_dtype=torch.float32)
-    Cp = I6.int6_matmul(view, I6.prepack_int6(Ld, Hd, Sd, g), out_dtype=torch.float32)
+    pk = I6.prepack_int6(Ld, Hd, Sd, g)
+    split = _split(split, B, M, N, K)
+    C = I6.int6_matmul(view, Ld, Hd, Sd, g, split_k=split, out_dtype=torch.float32)
+    Cp = I6.int6_matmul(view, pk, split_k=split, out_dtype=torch.float32)
+    near = I6.int6_matmul(a.to(DEV), pk, split_k=split, out_dtype=torch.float32)
     torch.cuda.synchronize()
-    assert torch.equal(C, Cp)
+    assert torch.equal(C, Cp) and torch.equal(C, near)
     _check(C, a, lo, hi, sc, g, KERNEL_TOL)
 
 

@@ -600,9 +600,17 @@ __global__ __launch_bounds__(64 * MAXW) void w6a16_tile_kernel(const Args p) {
     }
     // K split over ks workgroups.  The partial tile goes out in agent-scope atomic stores (written through to where every
     // XCD sees them), each wavefront waits until its own have completed, and the barrier puts all of them before the
-    // arrival count; the workgroup that counts in last reads the partials by agent-scope atomic loads.  No release or
-    // acquire fence: a fence writes back or invalidates the XCD's whole L2, and nothing here is cached there (with one
-    // fence per workgroup a call of 256 workgroups took 1 us longer, one of 512 4 us).
+    // arrival count; the workgroup that counts in last reads the partials by agent-scope atomic loads, past the caches.
+    // No release or acquire fence at agent scope: a fence writes back or invalidates the XCD's whole L2, and nothing here
+    // is cached there (with one fence per workgroup a call of 256 workgroups took 1 us longer, one of 512 4 us).
+    // The language alone does not order this: relaxed accesses on either side of a relaxed count promise nothing.  What
+    // does is this target: a store counts in vmcnt until it is done, at the place that agent-scope accesses of every XCD go
+    // to, so s_waitcnt 0 and the barrier put the stores before the count, and the loads are issued after it by the
+    // workgroup's second barrier.  A target that counts stores apart, or keeps agent-scope stores in a cache, would need
+    // release and acquire at agent scope around the count.
+#if defined(__HIP_DEVICE_COMPILE__) && !defined(__gfx950__)
+#error "the hand-off of the partial tiles is ordered by gfx950's store counter and write-through stores"
+#endif
     constexpr int kTileFloats = 16 * MT * NC;
     const int64_t id = ((int64_t)b * p.grid.m_groups + mg) * ((p.N / 16 + NT * CW - 1) / (NT * CW)) + wtile / (NT * CW);
     float* const part0 = p.part + id * ks * kTileFloats;

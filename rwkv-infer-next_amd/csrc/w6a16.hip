@@ -451,15 +451,11 @@ __device__ __forceinline__ void tile_work(const TileW<NT, PACKED>& s, const uint
     for (int mt = 0; mt < MT; ++mt) acc[mt][NT - 1] = fma4(tc[(NT - 1) & 1][mt], sv[(NT - 1) & 1], acc[mt][NT - 1]);
 }
 
-// The sum of the W partials of element (r, col) of the workgroup's tile, by the quarters of the parts that it holds
-// (4 / ks).
-template <int MT, int NT, int CW, bool PACKED>
-__device__ __forceinline__ float tile_sum(const float* part, int W, int ks, int r, int wcol) {
-    const int col = wcol % (16 * NT), t = PACKED ? col >> 4 : col & 3, i = PACKED ? col & 15 : col >> 2;
-    const float* const x = part + (((wcol / (16 * NT) * MT + (r >> 4)) * NT + t) * 64 + i + 16 * ((r & 15) >> 2)) * 4 + (r & 3);
+// The sum of the W partials of one element, at x, by the quarters of the parts that the workgroup holds (4 / ks).
+__device__ __forceinline__ float tile_sum(const float* x, int stride, int W, int ks) {
     auto sum = [&](int w0, int w1) __attribute__((always_inline)) {
         float y = 0.f;
-        for (int w = w0; w < min(w1, W); ++w) y += x[w * CW * MT * NT * 256];
+        for (int w = w0; w < min(w1, W); ++w) y += x[w * stride];
         return y;
     };
     if (ks == 4) return sum(0, W);
@@ -467,6 +463,25 @@ __device__ __forceinline__ float tile_sum(const float* part, int W, int ks, int 
     const float s = sum(0, n) + sum(n, 2 * n);
     return ks == 2 ? s : s + (sum(2 * n, 3 * n) + sum(3 * n, 4 * n));
 }
+
+// The same of four rows, whole f4 at x (single rows of them meet in a quarter of the banks), Q = 4 / ks quarters at a time.
+template <int Q>
+__device__ __forceinline__ f4 tile_sum4(const f4* x, int stride, int W) {
+    const int n = (W + Q - 1) / Q;  // parts per quarter
+    f4 s[Q];
+#pragma unroll
+    for (int q = 0; q < Q; ++q) s[q] = f4{0.f, 0.f, 0.f, 0.f};
+    for (int w = 0; w < n; ++w)
+#pragma unroll
+        for (int q = 0; q < Q; ++q)
+            if (q == 0 || q * n + w < W) s[q] += x[(q * n + w) * stride];
+    if constexpr (Q == 4) return (s[0] + s[1]) + (s[2] + s[3]);
+    else if constexpr (Q == 2) return s[0] + s[1];
+    else return s[0];
+}
+
+// LDS of a wavefront: its rows of A, then its partial tile.
+constexpr int tile_lds(int MT, int NA, int NT) { return 1024 * (MT * NT > NA ? MT * NT : NA); }
 
 // NA: groups of 8 rows of A a K part stages (1: M <= 8).  D chunks of weights and DA of A are in flight.  CW: wavefronts
 // side by side in a K part, 16 NT columns each, sharing its rows of A; with two, each loads half of them, the rows are
@@ -477,9 +492,9 @@ __global__ __launch_bounds__(64 * MAXW) void w6a16_tile_kernel(const Args p) {
     static_assert(!FAR || (MT == 1 && NT == 4 && CW == 1), "far: 16 rows, 64 columns to a workgroup");
     static_assert(D % DA == 0, "stage rings");
     static_assert(CW == 1 || (CW == 2 && D == 2 && DA == 1 && NA % 2 == 0), "one or two column wavefronts");
-    constexpr int kA = 1024 * NA, kPart = MAXW * MT * NT * 1024, kStage = MAXW * kA;  // (CW = 2: two buffers a K part)
-    constexpr int NW = NA / CW;  // row groups this wavefront loads
-    __shared__ __attribute__((aligned(16))) uint8_t lds[kPart > kStage ? kPart : kStage];
+    constexpr int kA = 1024 * NA;  // bytes of a chunk's rows of A (CW = 2: two buffers a K part)
+    constexpr int NW = NA / CW;    // row groups this wavefront loads
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];  // tile_lds bytes a wavefront
     __shared__ uint32_t completed;
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int W = (blockDim.x >> 6) / CW, ks = gridDim.z, split = blockIdx.z;  // W: K parts in the workgroup
@@ -577,25 +592,48 @@ __global__ __launch_bounds__(64 * MAXW) void w6a16_tile_kernel(const Args p) {
     }
 
     __syncthreads();  // the staging buffers are dead: the partial tiles reuse the LDS
-    f4* const part = reinterpret_cast<f4*>(lds) + wv * MT * NT * 64 + lane;  // [K part][column wavefront]
+    const int tid = threadIdx.x;
+    f4* const part = reinterpret_cast<f4*>(lds) + tid / 64 * MT * NT * 64 + tid % 64;  // [K part][column wavefront]
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
         for (int t = 0; t < NT; ++t) part[(mt * NT + t) * 64] = acc[mt][t];
     __syncthreads();
-    const float* const sums = reinterpret_cast<const float*>(lds);
+    // A thread takes one column of every step-th row, or, with more than one row to a thread, of every step-th four rows.
     constexpr int NC = 16 * NT * CW;
-    const int items = min(16 * MT, p.M - m0) * NC, n0 = 16 * wtile;
-    auto store = [&](int e, float x) __attribute__((always_inline)) {
-        const int r = e / NC, col = e % NC;
-        if (col >= p.N - n0) return;
-        const int64_t o = (int64_t)b * p.so_b + (int64_t)(m0 + r) * p.so_m + n0 + col;
+    const int rows = min(16 * MT, p.M - m0), n0 = 16 * wtile;
+    const int col = tid % NC, step = blockDim.x / NC;
+    auto each_sum = [&](auto sink) __attribute__((always_inline)) {
+        const int c = col % (16 * NT), t = PACKED ? c >> 4 : c & 3, i = PACKED ? c & 15 : c >> 2;
+        const f4* const sums = reinterpret_cast<const f4*>(lds) + (col / (16 * NT) * MT * NT + t) * 64 + i;
+        constexpr int kPart = CW * MT * NT * 64;
+        auto four = [&](int r4) __attribute__((always_inline)) { return sums + (r4 >> 2) * NT * 64 + 16 * (r4 & 3); };
+        auto fours = [&](auto quarters) __attribute__((always_inline)) {
+            for (int r4 = tid / NC; 4 * r4 < rows; r4 += step) {
+                const f4 y = tile_sum4<decltype(quarters)::value>(four(r4), kPart, W);
+#pragma unroll
+                for (int v = 0; v < 4; ++v)
+                    if (4 * r4 + v < rows) sink(4 * r4 + v, y[v]);
+            }
+        };
+        if (rows < 2 * step) {
+            for (int r = tid / NC; r < rows; r += step)
+                sink(r, tile_sum(reinterpret_cast<const float*>(four(r >> 2)) + (r & 3), 4 * kPart, W, ks));
+        } else if (ks == 1) {
+            fours(std::integral_constant<int, 4>{});
+        } else if (ks == 2) {
+            fours(std::integral_constant<int, 2>{});
+        } else {
+            fours(std::integral_constant<int, 1>{});
+        }
+    };
+    auto store = [&](int r, int c, float x) __attribute__((always_inline)) {
+        const int64_t o = (int64_t)b * p.so_b + (int64_t)(m0 + r) * p.so_m + n0 + c;
         if (p.out_dtype == W6A16_OUT_F16) put_out<true>(p, o, x);
         else put_out<false>(p, o, x);
     };
     if (ks == 1) {
-        for (int e = threadIdx.x; e < items; e += blockDim.x)
-            store(e, tile_sum<MT, NT, CW, PACKED>(sums, W, 1, e / NC, e % NC));
+        if (col < p.N - n0) each_sum([&](int r, float x) __attribute__((always_inline)) { store(r, col, x); });
         return;
     }
     // K split over ks workgroups.  The partial tile goes out in agent-scope atomic stores (written through to where every
@@ -614,9 +652,7 @@ __global__ __launch_bounds__(64 * MAXW) void w6a16_tile_kernel(const Args p) {
     constexpr int kTileFloats = 16 * MT * NC;
     const int64_t id = ((int64_t)b * p.grid.m_groups + mg) * ((p.N / 16 + NT * CW - 1) / (NT * CW)) + wtile / (NT * CW);
     float* const part0 = p.part + id * ks * kTileFloats;
-    for (int e = threadIdx.x; e < items; e += blockDim.x)
-        coherent_store(part0 + split * kTileFloats + e,
-                       tile_sum<MT, NT, CW, PACKED>(sums, W, ks, e / NC, e % NC));
+    each_sum([&](int r, float x) __attribute__((always_inline)) { coherent_store(part0 + split * kTileFloats + r * NC + col, x); });
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
     __builtin_amdgcn_s_waitcnt(0);  // this wavefront's partial stores have completed
     __syncthreads();
@@ -628,14 +664,16 @@ __global__ __launch_bounds__(64 * MAXW) void w6a16_tile_kernel(const Args p) {
     }
     __syncthreads();
     if (!completed) return;
-    for (int e = 2 * threadIdx.x; e < items; e += 2 * blockDim.x) {
+    for (int e = 2 * tid; e < rows * NC; e += 2 * blockDim.x) {
         float2 x[4];
 #pragma unroll
         for (int k = 0; k < 4; ++k) x[k] = coherent_load2(part0 + min(k, ks - 1) * kTileFloats + e);
         float2 sum = float2{x[0].x + x[1].x, x[0].y + x[1].y};
         if (ks == 4) sum = float2{sum.x + (x[2].x + x[3].x), sum.y + (x[2].y + x[3].y)};
-        store(e, sum.x);
-        store(e + 1, sum.y);
+        const int c = e % NC;
+        if (c >= p.N - n0) continue;  // (both columns of a pair, or neither)
+        store(e / NC, c, sum.x);
+        store(e / NC, c + 1, sum.y);
     }
 }
 
@@ -1185,12 +1223,33 @@ TilePlan tile_plan(const w6a16_args* a, const Layout& l, bool packed) {
     auto groups = [&](int mt) { return (int64_t)a->B * ((a->M + 16 * mt - 1) / (16 * mt)); };
     auto wgs = [&](int mt, int nt) { return groups(mt) * ((tiles + nt - 1) / nt); };
     auto rounds = [&](int64_t n) { return (n + cus - 1) / cus; };
+    // Workgroups that may share a tile's K: none without room for their counters and partial tiles (so split_k bounds it;
+    // up to 32 rows a split of at most 8 has no workspace).
+    auto room = [&](int mt, int cw) {
+        int most = a->M <= kSmallM ? (a->split_k > kGemvMaxSplit ? 4 : 1) : a->split_k >= 4 ? 4 : a->split_k >= 2 ? 2 : 1;
+        if ((size_t)(groups(mt) * tiles) * 4 > kCounterRegion) most = 1;
+        while (most > 1 && (size_t)wgs(mt, 4 * cw) * most * 16 * mt * 64 * cw * 4 > l.partial_bytes) most >>= 1;
+        return most;
+    };
+    // Workgroups of `wide` K parts for whose parts a deep K has work where CUs would be left without.
+    auto spread = [&](int mt, int cw, int wide) {
+        const int64_t w4 = wgs(mt, 4 * cw), most = room(mt, cw);
+        int s = 1;
+        while (s < most && chunks >= wide * s * 2 && w4 * s * 2 <= cus &&
+               (chunks > 128 || (mt == 2 && w4 * 4 <= cus && s < 2)) && !(mt == 1 && s == 2))
+            s *= 2;
+        return s;
+    };
     // Rows to a workgroup: one tile up to 16 rows, two up to 32; above, two to four tiles and, from three on, 64 or 128
     // columns, whatever costs least (us, packed: K = N = 4096, M = 64: mt 2 10.3, mt 4 13.3; N = 16384: 25.6 / 22.2;
     // K = N = 2560, M = 203: mt 2, 3, 4 14.9 / 11.4 / 12.8).
     t.cw = 1;
     if (a->M <= 16) {
         t.mt = 1;
+    } else if (chunks <= 2) {
+        // what a workgroup writes costs more than what it reads (us, packed, N = 16384: K = 64, M = 64, mt 1, 2, 4 6.0 / 8.3 /
+        // 12.8; M = 256 11.9 / 11.2 / 17; K = 128, M = 128 9.9 / 7.9 / 10.3)
+        t.mt = wgs(1, 4) <= 4 * cus ? 1 : 2;
     } else {
         t.mt = 2;
         auto cost = [&](int mt, int cw) { return rounds(wgs(mt, 4 * cw)) * (4 * mt + 7 * cw); };
@@ -1201,21 +1260,24 @@ TilePlan tile_plan(const w6a16_args* a, const Layout& l, bool packed) {
                     if (cost(mt, cw) < best) best = cost(mt, cw), t.mt = mt, t.cw = cw;
     }
     const int64_t w4 = wgs(t.mt, 4 * t.cw);
-    // Workgroups that may share K: none without room for their counters and partial tiles (so split_k bounds it; up to
-    // 32 rows a split of at most 8 has no workspace).
-    int most = a->M <= kSmallM ? (a->split_k > kGemvMaxSplit ? 4 : 1) : a->split_k >= 4 ? 4 : a->split_k >= 2 ? 2 : 1;
-    if ((size_t)(groups(t.mt) * tiles) * 4 > kCounterRegion) most = 1;
-    while (most > 1 && (size_t)w4 * most * 16 * t.mt * 64 * t.cw * 4 > l.partial_bytes) most >>= 1;
+    const int most = room(t.mt, t.cw);
     // Wavefronts that share K: eight to a workgroup (with two column wavefronts four), with one row tile 16 where the
-    // workgroups do not fill the chip and 4 where they do (K = 4096, N = 16384, M = 1, packed / planes: 4 12.4 / 16.2, 8
-    // 12.6 / 16.8, 16 13.3 / 17.7), and twice or four times as many where a deep K would otherwise leave CUs without
-    // work (K = 16384, N = 4096, M = 1: 16 parts in one workgroup 16.4, 32 in two 14.1).
-    const int wide = t.mt == 1 ? (w4 < cus ? 16 : 4) : 8 / t.cw;
-    int spread = 1;  // workgroups of `wide` wavefronts
-    while (spread < most && chunks >= wide * spread * 2 && w4 * spread * 2 <= cus &&
-           (chunks > 128 || (t.mt == 2 && w4 * 4 <= cus && spread < 2)) && !(t.mt == 1 && spread == 2))
-        spread *= 2;
-    t.parts = std::min(chunks, wide * spread);
+    // workgroups do not fill the chip and a part of 16 has more than one chunk, else 4 (us, packed / planes: K = 4096, N =
+    // 16384, M = 1: 4 12.4 / 16.2, 8 12.6 / 16.8, 16 13.3 / 17.7; K = N = 1024, M = 16: 4 4.0 / 5.6, 16 5.4 / 6.6; K = N = 2048,
+    // M = 1: 8 4.4 / 7.0, 16 5.2 / 6.4), and twice or four times as many where a deep K would otherwise leave CUs without work
+    // (K = 16384, N = 4096, M = 1: 16 parts in one workgroup 16.4, 32 in two 14.1).
+    int wide = t.mt == 1 ? (w4 < cus && chunks > 16 ? 16 : 4) : 8 / t.cw;
+    // Two row tiles and more, several rounds over the CUs: fewer to a workgroup, several of which then share a CU and fewer
+    // follow each other.  A round costs its chunks a part and about 4/3 of a chunk for its start and end (K = 1024, N = 65536,
+    // us, packed: M = 32, 8, 4, 2, 1 parts 25.5 / 18.8 / 18.7 / 20.5; M = 128, 4, 2, 1 53.9 / 46.3 / 43.8; M = 192 76.7 / 64.4 /
+    // 71.1; K = 4096, N = 16384, M = 128 32.2 / 41.9 / 69).
+    if (t.mt > 1) {
+        const int full = wide;
+        auto cost = [&](int n) { return (w4 * n + cus * full - 1) / (cus * full) * (3 * ((chunks + n - 1) / n) + 4); };
+        for (int n = full / 2; n >= 1 && w4 > cus; n /= 2)
+            if (cost(n) < cost(wide)) wide = n;
+    }
+    t.parts = std::min(chunks, wide * spread(t.mt, t.cw, wide));
     auto fits = [&](int ks, int max_w) { return ks == 1 ? t.parts <= max_w : t.parts % 4 == 0 && t.parts / ks <= max_w; };
     // Columns to a wavefront and workgroups to a K range.  Packed: as few workgroups to a K range as hold the parts, and
     // the columns whose rounds cost least.  Planes: always 64 columns (a lane loads four), K spread over more workgroups
@@ -1292,7 +1354,8 @@ int launch_tile(Args& p, const TilePlan& t, hipStream_t s) {
     for (uint64_t x = 0; x < wgs; x += most) {
         p.grid.first = (uint32_t)(x / 8);
         hipLaunchKernelGGL((w6a16_tile_kernel<A, MT, NA, NT, CW, D, DA, MAXW, PACKED, FAR>),
-                           dim3((unsigned)std::min<uint64_t>(wgs - x, most), p.B, t.ks), dim3(block), 0, s, p);
+                           dim3((unsigned)std::min<uint64_t>(wgs - x, most), p.B, t.ks), dim3(block),
+                           block / 64 * tile_lds(MT, NA, NT), s, p);
     }
     return WKV7_OK;
 }

@@ -30,6 +30,11 @@ from test_gpu_int6 import DEV, F16_KERNEL_TOL, KERNEL_TOL, _act, _check, _dev, _
     (1, 64, 16384, 192, 64, 1),      # four row tiles, 64 columns, three chunks
     (1, 203, 10240, 320, 64, 1),     # three row tiles, 128 columns; five chunks over four parts
     (1, 128, 16336, 576, 64, 1),     # four row tiles, 128 columns, nine chunks, columns that end inside a strip
+    (1, 40, 16336, 64, 64, 1),       # one chunk: one row tile
+    (1, 200, 16336, 128, 64, 1),     # two chunks, many workgroups: two row tiles
+    (1, 20, 33024, 576, 64, 1),      # several rounds: two parts, two row tiles
+    (1, 128, 33024, 320, 64, 1),     # one part, four row tiles, 128 columns
+    (1, 16, 256, 1088, 64, 1),       # 16 parts, 17 chunks
 ])
 @pytest.mark.parametrize("dtype", ["bf16", "f16"])
 def test_tile_shapes(B, M, N, K, g, split, dtype):

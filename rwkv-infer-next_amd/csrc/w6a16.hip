@@ -334,7 +334,9 @@ __device__ __forceinline__ void tile_load_w(const Args& p, const TileSrc& src, i
 }
 
 // NA groups of 8 rows of A's chunk (128 bytes per row).  The rows' offsets are lane offsets: those are what a raw buffer's
-// bound covers by its definition, and it is the bound that keeps rows past M from being read.
+// bound covers by its definition, and it is the bound that keeps rows past M from being read.  Eight groups go through two
+// buffers: eight lane offsets put registers of the loop into scratch memory (planes, four row tiles, K = 4096, N = 16384, M =
+// 64: 30.9 us, 26.1 without).
 template <int NA, bool FAR>
 __device__ __forceinline__ void tile_load_a(const Args& p, const TileSrc& src, int c, u4 (&a)[NA]) {
     if constexpr (FAR) {
@@ -343,9 +345,15 @@ __device__ __forceinline__ void tile_load_a(const Args& p, const TileSrc& src, i
         for (int e = 0; e < NA; ++e)
             a[e] = *reinterpret_cast<const __attribute__((address_space(1))) u4*>(src.fa[e] + (uint64_t)c * 128);
     } else {
-        const __amdgpu_buffer_rsrc_t r = tile_rsrc(src.a + (uint64_t)c * 128, src.na - c * 128);
+        constexpr int kGroup = NA == 8 ? 4 : NA;  // row groups to a buffer
 #pragma unroll
-        for (int e = 0; e < NA; ++e) a[e] = __builtin_amdgcn_raw_buffer_load_b128(r, src.va + 16 * e * (uint32_t)p.sa_m, 0, 0);
+        for (int e0 = 0; e0 < NA; e0 += kGroup) {
+            const int off = 16 * e0 * (int)p.sa_m, left = src.na - c * 128 - off;
+            const __amdgpu_buffer_rsrc_t r = tile_rsrc(src.a + (uint64_t)c * 128 + (uint64_t)off, e0 == 0 ? left : max(left, 0));
+#pragma unroll
+            for (int e = e0; e < e0 + kGroup; ++e)
+                a[e] = __builtin_amdgcn_raw_buffer_load_b128(r, src.va + 16 * (e - e0) * (uint32_t)p.sa_m, 0, 0);
+        }
     }
 }
 
@@ -1298,6 +1306,16 @@ TilePlan tile_plan(const w6a16_args* a, const Layout& l, bool packed) {
         const int64_t cost = rounds(wgs(t.mt, nt * t.cw) * ks) * (2 * nt + 3 * t.mt);
         if (!best || cost < best) best = cost, t.nt = nt, t.ks = ks;
     }
+    // Planes, deep K, a single round of workgroups of two row tiles: half as many groups of rows, of up to twice the rows, and
+    // the same parts over two workgroups, since the planes' loads are what takes the time there (K = 16384, N = 4096, us, two
+    // row tiles / three or four: M = 65 47.7 / 36.6, 128 48.1 / 42.4; K = 8192: 25.9 / 25.7, 26.8 / 29.4).
+    if (!packed && t.mt == 2 && t.ks == 1 && t.parts == 8 && most >= 2 && chunks >= 256)
+        for (int mt = 3; mt <= 4; ++mt)
+            if (wgs(mt, 4) * 2 <= cus && groups(mt) * 2 <= groups(2) + 1 &&
+                (size_t)wgs(mt, 4) * 2 * 16 * mt * 64 * 4 <= l.partial_bytes) {
+                t.mt = mt, t.ks = 2;
+                break;
+            }
     // Planes whose 32 rows span 2 GB, rows of A of which 64 do: 16 rows and 64 columns to a workgroup, with 64-bit
     // addresses, and the same parts, so the same bits as for the same rows packed or side by side.  (More than 16 parts
     // come only with few tiles, whose counters and partial tiles have room.)

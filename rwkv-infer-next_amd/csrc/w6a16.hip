@@ -18,7 +18,7 @@
 //     LDS buffer;
 //   * each chunk's fp32 tile is scaled by s (fp16) and accumulated; the wavefronts' tiles are summed through LDS, and
 //     the tiles of several workgroups, where K is split over them, through the workspace, both in a fixed order.
-// Large-M kernel (packed weights): described where it is defined.
+// Wide kernel (145..256 rows, many columns) and large-M kernel (packed weights): described where they are defined.
 // Rows m >= M read zeros and columns n >= N are clamped on load (they only feed outputs that are not stored).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -37,6 +37,8 @@ namespace {
 typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
 typedef float f4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+typedef int v2i __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(3))) v2i lds_v2i;
 
 constexpr int kTileN = 128;          // columns per strip of the packed layout
 constexpr int kTiles = kTileN / 16;  // 16-column tiles per strip
@@ -61,6 +63,8 @@ struct Args {
     TileGrid grid;                   // tile kernel: M groups of 16 MT rows, columns of a workgroup's column tiles
     int32_t parts, per_part, groups;  // wavefronts that share K, chunks of the longest share, scale groups
     Divisor group;                   // chunk c's scale group is c over the chunks of a group
+    float* rsum;                     // wide kernel: row-sum bias [batch][chain][mpad]
+    int32_t mpad, chain_k, nchains;
     int32_t out_vec;  // large-M kernel: the output takes 8-byte (16-byte for fp32) stores of 4 adjacent columns
 };
 
@@ -69,6 +73,8 @@ __device__ __forceinline__ float h2f(uint16_t h) { return (float)__builtin_bit_c
 __device__ __forceinline__ f4 mfma(bf8 a, bf8 b, f4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
 
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
 
 // Activation element types.  The 6-bit code u becomes an exact MFMA operand 2^e + u with no conversion instruction
 // (the code byte beside a constant high byte), and one MFMA pair per chunk against the constant -(2^e + 32) takes the
@@ -78,13 +84,23 @@ typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 struct ActBF16 {
     static constexpr uint32_t kCodeHi = 0x43434343u;
     static constexpr uint32_t kBias = 0xC320C320u;  // (-160, -160)
+    static constexpr uint32_t kOnes = 0x3F803F80u;  // (1, 1)
+    static constexpr float kOffset = 160.f;
     __device__ static f4 mma(u4 a, u4 b, f4 c) { return mfma(__builtin_bit_cast(bf8, a), __builtin_bit_cast(bf8, b), c); }
+    __device__ static float dot2(uint32_t a, uint32_t b, float c) {
+        return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf2, a), __builtin_bit_cast(bf2, b), c, false);
+    }
 };
 struct ActF16 {
     static constexpr uint32_t kCodeHi = 0x64646464u;
     static constexpr uint32_t kBias = 0xE420E420u;  // (-1056, -1056)
+    static constexpr uint32_t kOnes = 0x3C003C00u;  // (1, 1)
+    static constexpr float kOffset = 1056.f;
     __device__ static f4 mma(u4 a, u4 b, f4 c) {
         return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, a), __builtin_bit_cast(h8, b), c, 0, 0, 0);
+    }
+    __device__ static float dot2(uint32_t a, uint32_t b, float c) {
+        return __builtin_amdgcn_fdot2(__builtin_bit_cast(h2, a), __builtin_bit_cast(h2, b), c, false);
     }
 };
 
@@ -704,8 +720,330 @@ __device__ __forceinline__ void store_row8(OutT* dst, const float (&v)[8], bool 
     }
 }
 
-typedef int v2i __attribute__((ext_vector_type(2)));
-typedef __attribute__((address_space(3))) v2i lds_v2i;
+// ---------------------------------------------------------------------------------------------------------------
+// Wide kernel: 145 to 256 rows over so many columns that 64 x 128 tiles go at least twice around the CUs (wide_call).  A
+// workgroup of four wavefronts covers 128 columns for 64 rows, wavefront cp column tiles 2 cp and 2 cp + 1 for all of them,
+// over all of K: each dequantised weight operand serves four row tiles, and each A operand two column tiles.  The tile
+// kernel waits on its own chains there (64 accumulators a lane against 32, a scaling per chunk, a bias product per chunk
+// and row tile): K = 4096, N = 16384, M = 256, us, planes / packed, 63.0 / 59.2 against 60.4 / 49.7 here; K = 1024, N =
+// 65536, M = 256 91.1 / 79.0 against 76.9 / 66.8.
+//   * A's chunk ([64 rows][64 k]) is staged in LDS, double-buffered, one workgroup barrier a step; piece j of row r lies at
+//     a_slot.  Packed weights go straight to registers, four steps ahead; planes are staged with A (48 rows x 128 columns)
+//     and read back transposed (ds_read_b64_tr_b8).
+//   * Chains: the products of CG chunks (two where the quantisation group holds two) accumulate in one MFMA chain, which
+//     starts at the bias -(2^e + 32) sum_k A[m][k] (row sums of a pass before it), and are scaled once.
+constexpr int kWideMT = 4, kWideRows = 16 * kWideMT;
+constexpr int kPitch = 136;                // LDS row pitch of the planes: the 8 rows of one transposing read differ in bank
+constexpr int kScaleOff = 48 * kPitch;     // the chunk's 128 scales follow 32 lo and 16 hi rows
+constexpr int kWideA = kWideRows * 128;    // bytes of A in a stage; the chain's row sums follow, then the planes
+
+template <bool PACKED>
+constexpr int wide_stage() { return kWideA + kWideRows * 4 + (PACKED ? 0 : kScaleOff + 2 * kTileN); }
+
+// (1, 1) as an activation pair held in a register (an empty asm keeps the compiler from folding the pair into an
+// inline constant, which the packed dot product would read differently).
+template <class A>
+__device__ __forceinline__ uint32_t ones_x2() {
+    uint32_t bits = A::kOnes;
+    asm("" : "+v"(bits));
+    return bits;
+}
+
+template <class A>
+__device__ __forceinline__ float sum8(const u4 v, uint32_t one) {
+    float x = 0.f;
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+        // the element is copied out first: bit-casting a vector element in place (v[d]) compiled to a read of
+        // element 0 for every d
+        const uint32_t word = v[d];
+        x = A::dot2(word, one, x);
+    }
+    return x;
+}
+
+template <int CTRL>
+__device__ __forceinline__ float dpp_add(float x) {  // x + x of the lane DPP control CTRL selects (all lanes active)
+    return x + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xF, 0xF, false));
+}
+
+// Row sums of A per chain of chain_k k: rsum[b][chain][m] = -(2^e + 32) sum A[b][m][chain's k], zero for rows M <= m <
+// mpad.  One wavefront per (row, 512-element segment of K; 8 elements per lane, coalesced); the lanes of a chain add
+// their sums with DPP in a fixed order.
+template <class A>
+__global__ __launch_bounds__(256) void w6a16_rowsum_kernel(const Args p) {
+    const int lane = threadIdx.x & 63;
+    const int m = blockIdx.x * 4 + (threadIdx.x >> 6), k = blockIdx.y * 512 + 8 * lane, b = blockIdx.z;
+    if (m >= p.mpad) return;  // uniform over the wavefront
+    const int lanes_per_chain = p.chain_k / 8;  // 8 or 16
+    const uint16_t* const row = p.a + (int64_t)b * p.sa_b + (int64_t)min(m, p.M - 1) * p.sa_m;
+    // K is a multiple of the chain: a chain's lanes are all inside K or all past it
+    float x = (m < p.M && k < p.K) ? sum8<A>(*reinterpret_cast<const u4*>(row + k), ones_x2<A>()) : 0.f;
+    x = dpp_add<0xB1>(x);   // lanes ^ 1
+    x = dpp_add<0x4E>(x);   // lanes ^ 2: each lane holds its quad's sum
+    x = dpp_add<0x141>(x);  // half-row mirror: lane 7 - l of the 8-lane group, in the other quad
+    if (lanes_per_chain == 16) x = dpp_add<0x140>(x);  // row mirror: lane 15 - l, in the other half
+    if ((lane & (lanes_per_chain - 1)) == 0 && k < p.K)
+        p.rsum[((int64_t)b * p.nchains + k / p.chain_k) * p.mpad + m] = -A::kOffset * x;
+}
+
+// What one thread loads per step into the LDS stage: two pieces of A, four row sums (threads 0..15) and (planes) 16 bytes
+// of a lo-plane row, 16 bytes of a hi-plane row (threads 0..127) or two scales (threads 128..191).
+struct WideLds {
+    u4 a[2], rs, pl[2];
+    uint32_t sc;
+};
+
+// Buffer bases and sizes (wave-uniform) and per-lane offsets of the loads, fixed for the call; the chunk goes into the
+// instructions' scalar offset.  Every range is below 2 GB (wide_call).
+struct WideSrc {
+    uint64_t a, rs, lo, hi, sc;
+    int64_t na, nrs, nlo, nhi, nsc;
+    uint32_t va[2], vrs, vlo, vhi, vsc;
+};
+
+template <bool PACKED>
+__device__ __forceinline__ WideSrc wide_src(const Args& p, int b, int m0, int strip) {
+    const int t = threadIdx.x, lane = t & 63, i = lane & 15, cp = t >> 6, n0 = strip * kTileN;
+    WideSrc x;
+    x.a = reinterpret_cast<uint64_t>(p.a + (int64_t)b * p.sa_b);
+    x.na = ((int64_t)(p.M - 1) * p.sa_m + p.K) * 2;
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+        const int piece = t + 256 * e;
+        x.va[e] = (uint32_t)((min(m0 + (piece >> 3), p.M - 1) * p.sa_m + 8 * (piece & 7)) * 2);
+    }
+    x.rs = reinterpret_cast<uint64_t>(p.rsum + (int64_t)b * p.nchains * p.mpad);
+    x.nrs = (int64_t)p.nchains * p.mpad * 4;
+    x.vrs = (m0 + 4 * min(t, kWideRows / 4 - 1)) * 4;
+    if constexpr (PACKED) {
+        const int nchunks = p.K / 64;
+        x.lo = reinterpret_cast<uint64_t>(p.lo + (int64_t)b * p.sl_b + (int64_t)strip * nchunks * kPackBytes);
+        x.nlo = (int64_t)nchunks * kPackBytes;
+        x.vlo = 16 * lane + 1024 * cp;
+        x.vhi = 4096 + 1024 * (cp >> 1) + 8 * (cp & 1) + 16 * lane;
+        x.sc = reinterpret_cast<uint64_t>(p.sc + (int64_t)b * p.ss_b + (int64_t)strip * p.groups * kTileN);
+        x.nsc = (int64_t)p.groups * kTileN * 2;
+        x.vsc = (8 * i + 2 * cp) * 2;
+    } else {
+        const int row = t >> 3, n = min(n0 + 16 * (t & 7), p.N - 16);  // lo row 0..31; hi row (row & 15)
+        x.lo = reinterpret_cast<uint64_t>(p.lo + (int64_t)b * p.sl_b);
+        x.nlo = (int64_t)(p.K / 2) * p.N;
+        x.vlo = row * p.N + n;
+        x.hi = reinterpret_cast<uint64_t>(p.hi + (int64_t)b * p.sh_b);
+        x.nhi = (int64_t)(p.K / 4) * p.N;
+        x.vhi = (row & 15) * p.N + n;
+        x.sc = reinterpret_cast<uint64_t>(p.sc + (int64_t)b * p.ss_b);
+        x.nsc = (int64_t)p.groups * p.N * 2;
+        x.vsc = min(n0 + 2 * (t & 63), p.N - 2) * 2;
+    }
+    return x;
+}
+
+template <int CG, bool PACKED>
+__device__ __forceinline__ void wide_load_lds(const Args& p, const WideSrc& src, int c, WideLds& x) {
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+        x.a[e] = __builtin_amdgcn_raw_buffer_load_b128(rsrc(src.a, src.na), src.va[e], soff(c * 128), 0);
+    x.rs = __builtin_amdgcn_raw_buffer_load_b128(rsrc(src.rs, src.nrs), src.vrs, soff((c / CG) * p.mpad * 4), 0);
+    if constexpr (!PACKED) {
+        x.pl[0] = __builtin_amdgcn_raw_buffer_load_b128(rsrc(src.lo, src.nlo), src.vlo, soff(c * 32 * p.N), 0);
+        x.pl[1] = __builtin_amdgcn_raw_buffer_load_b128(rsrc(src.hi, src.nhi), src.vhi, soff(c * 16 * p.N), 0);
+        x.sc = __builtin_amdgcn_raw_buffer_load_b32(rsrc(src.sc, src.nsc), src.vsc,
+                                                    soff((int)quotient((uint32_t)c, p.group) * p.N * 2), 0);
+    }
+}
+
+template <bool PACKED>
+__device__ __forceinline__ void wide_store_lds(const WideLds& x, uint8_t* st) {
+    const int t = threadIdx.x;
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+        const int piece = t + 256 * e;
+        *reinterpret_cast<u4*>(st + 16 * a_slot(piece >> 3, piece & 7)) = x.a[e];
+    }
+    if (t < kWideRows / 4) *reinterpret_cast<u4*>(st + kWideA + 16 * t) = x.rs;
+    if constexpr (!PACKED) {
+        uint8_t* const pl = st + kWideA + kWideRows * 4;
+        uint8_t* dst = pl + (t >> 3) * kPitch + 16 * (t & 7);
+        *reinterpret_cast<uint2*>(dst) = uint2{x.pl[0][0], x.pl[0][1]};
+        *reinterpret_cast<uint2*>(dst + 8) = uint2{x.pl[0][2], x.pl[0][3]};
+        if (t < 128) {
+            dst += 32 * kPitch;
+            *reinterpret_cast<uint2*>(dst) = uint2{x.pl[1][0], x.pl[1][1]};
+            *reinterpret_cast<uint2*>(dst + 8) = uint2{x.pl[1][2], x.pl[1][3]};
+        } else if (t < 192) {
+            *reinterpret_cast<uint32_t*>(pl + kScaleOff + 4 * (t & 63)) = x.sc;
+        }
+    }
+}
+
+// The packed weights of one chunk in one lane's registers: the lo dwords of the wavefront's two column tiles, their hi
+// dwords and their scales of column i.
+struct WideW {
+    u4 lo;
+    uint2 hd;
+    uint32_t sc;
+};
+
+__device__ __forceinline__ void wide_load_w(const Args& p, const WideSrc& src, int c, WideW& w) {
+    const __amdgpu_buffer_rsrc_t lo = rsrc(src.lo, src.nlo);
+    const int off = soff(c * kPackBytes);
+    w.lo = __builtin_amdgcn_raw_buffer_load_b128(lo, src.vlo, off, 0);
+    w.hd = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(lo, src.vhi, off, 0));
+    w.sc = __builtin_amdgcn_raw_buffer_load_b32(rsrc(src.sc, src.nsc), src.vsc,
+                                                soff((int)quotient((uint32_t)c, p.group) * kTileN * 2), 0);
+}
+
+// The wavefront's two column tiles of one chunk as B operands w0 (rows 0..31 of the chunk) and w1 (rows 32..63), and their
+// scales.
+template <class A, bool PACKED>
+__device__ __forceinline__ void wide_dequant(const uint8_t* st, const WideW& w, u4 (&w0)[2], u4 (&w1)[2], float (&sv)[2]) {
+    const int lane = threadIdx.x & 63, cp = threadIdx.x >> 6, i = lane & 15, q = lane >> 4;
+    if constexpr (PACKED) {
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int tt = 0; tt < 2; ++tt) {
+            const uint32_t L0 = w.lo[2 * tt], L1 = w.lo[2 * tt + 1], Hd = tt ? w.hd.y : w.hd.x;
+            uint32_t o0[4], o1[4];
+            codes_to_op<A>((L0 & 0x0F0F0F0Fu) | ((Hd & 0x03030303u) << 4), o0[0], o0[1]);         // rows 8 q + 0..3
+            codes_to_op<A>((L1 & 0x0F0F0F0Fu) | (Hd & 0x30303030u), o0[2], o0[3]);                // rows 8 q + 4..7
+            codes_to_op<A>(((L0 >> 4) & 0x0F0F0F0Fu) | ((Hd & 0x0C0C0C0Cu) << 2), o1[0], o1[1]);  // rows 32 + 8 q ..
+            codes_to_op<A>(((L1 >> 4) & 0x0F0F0F0Fu) | ((Hd >> 2) & 0x30303030u), o1[2], o1[3]);
+            w0[tt] = u4{o0[0], o0[1], o0[2], o0[3]};
+            w1[tt] = u4{o1[0], o1[1], o1[2], o1[3]};
+            sv[tt] = h2f((uint16_t)(w.sc >> (16 * tt)));
+        }
+    } else {
+        const uint8_t* const pl = st + kWideA + kWideRows * 4;
+        const int sel = 2 * (q >> 1), off = (i >> 1) * kPitch + 8 * (i & 1);
+        v2i lo_t[2], hi_t[2];
+        uint16_t sh[2];
+#pragma unroll
+        for (int tt = 0; tt < 2; ++tt) {
+            const int t = 2 * cp + tt;
+            lo_t[tt] = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i*)(pl + (8 * q) * kPitch + off + 16 * t));
+            hi_t[tt] = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i*)(pl + (32 + 8 * (q & 1)) * kPitch + off + 16 * t));
+            sh[tt] = *reinterpret_cast<const uint16_t*>(pl + kScaleOff + 2 * (16 * t + i));
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int tt = 0; tt < 2; ++tt) {
+            uint32_t o0[4], o1[4];
+#pragma unroll
+            for (int d = 0; d < 2; ++d) {
+                const uint32_t L = (uint32_t)lo_t[tt][d], Hs = (uint32_t)hi_t[tt][d] >> sel;
+                codes_to_op<A>((L & 0x0F0F0F0Fu) | ((Hs & 0x03030303u) << 4), o0[2 * d], o0[2 * d + 1]);  // rows 8 q + e
+                codes_to_op<A>(((L >> 4) & 0x0F0F0F0Fu) | (Hs & 0x30303030u), o1[2 * d], o1[2 * d + 1]);  // 32 + 8 q + e
+            }
+            w0[tt] = u4{o0[0], o0[1], o0[2], o0[3]};
+            w1[tt] = u4{o1[0], o1[1], o1[2], o1[3]};
+            sv[tt] = h2f(sh[tt]);
+        }
+    }
+}
+
+// One chunk: two MFMAs per (row tile, column tile) into the chain accumulators tc; FIRST starts the chain at the row
+// sums' bias, LAST scales it into acc.  The LDS reads are issued ahead of the dequantisation that hides them (left to
+// itself the compiler reused a few operand registers and waited on the LDS once per row tile).
+template <class A, bool PACKED, bool FIRST, bool LAST>
+__device__ __forceinline__ void wide_compute(const uint8_t* st, const WideW& w, f4 (&tc)[kWideMT][2], f4 (&acc)[kWideMT][2]) {
+    const int lane = threadIdx.x & 63, i = lane & 15, q = lane >> 4;
+    const float* const rsum = reinterpret_cast<const float*>(st + kWideA);
+    u4 a0[kWideMT], a1[kWideMT], w0[2], w1[2];
+    f4 nc[kWideMT];
+    float sv[2];
+#pragma unroll
+    for (int mt = 0; mt < kWideMT; ++mt) {
+        a0[mt] = *reinterpret_cast<const u4*>(st + 16 * a_slot(16 * mt + i, q));
+        a1[mt] = *reinterpret_cast<const u4*>(st + 16 * a_slot(16 * mt + i, 4 + q));
+        if constexpr (FIRST) nc[mt] = *reinterpret_cast<const f4*>(rsum + 16 * mt + 4 * q);  // rows 16 mt + 4 q + v
+    }
+    wide_dequant<A, PACKED>(st, w, w0, w1, sv);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int mt = 0; mt < kWideMT; ++mt)
+#pragma unroll
+        for (int tt = 0; tt < 2; ++tt) {
+            const f4 c = A::mma(a0[mt], w0[tt], FIRST ? nc[mt] : tc[mt][tt]);
+            tc[mt][tt] = A::mma(a1[mt], w1[tt], c);
+        }
+    if constexpr (LAST) {
+#pragma unroll
+        for (int mt = 0; mt < kWideMT; ++mt)
+#pragma unroll
+            for (int tt = 0; tt < 2; ++tt) acc[mt][tt] = fma4(tc[mt][tt], sv[tt], acc[mt][tt]);
+    }
+}
+
+// lane (i, q) of wavefront cp holds C[m0 + 16 mt + 4 q + v][n0 + 16 (2 cp + tt) + i]
+template <bool F16>
+__device__ __forceinline__ void wide_store(const Args& p, int b, int m0, int n0, const f4 (&acc)[kWideMT][2]) {
+    const int lane = threadIdx.x & 63, cp = threadIdx.x >> 6, i = lane & 15, q = lane >> 4;
+#pragma unroll
+    for (int mt = 0; mt < kWideMT; ++mt)
+#pragma unroll
+        for (int tt = 0; tt < 2; ++tt) {
+            const int n = n0 + 16 * (2 * cp + tt) + i;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int m = m0 + 16 * mt + 4 * q + v;
+                if (n >= p.N || m >= p.M) continue;
+                put_out<F16>(p, (int64_t)b * p.so_b + (int64_t)m * p.so_m + n, acc[mt][tt][v]);
+            }
+        }
+}
+
+template <class A, int CG, bool PACKED>
+__global__ __launch_bounds__(256, 2) void w6a16_wide_kernel(const Args p) {
+    constexpr int kStage = wide_stage<PACKED>(), D = 4;  // loads D steps ahead
+    static_assert(D % CG == 0 && D % 2 == 0, "a group of D steps holds whole chains and buffer pairs");
+    __shared__ __attribute__((aligned(16))) uint8_t lds[2 * kStage];
+    const TilePos pos = tile_pos(p.grid, blockIdx.x);
+    const int strip = (int)pos.column, n0 = strip * kTileN, m0 = (int)pos.mg * kWideRows, b = blockIdx.z;
+    if (strip >= p.n_strips) return;  // uniform over the workgroup
+    const int steps = p.K / 64;
+    const WideSrc src = wide_src<PACKED>(p, b, m0, strip);
+    f4 acc[kWideMT][2], tc[kWideMT][2];
+#pragma unroll
+    for (int mt = 0; mt < kWideMT; ++mt) acc[mt][0] = acc[mt][1] = f4{0.f, 0.f, 0.f, 0.f};
+    // The LDS stage of step s is written in step s - 1 (after its reads of the other buffer have passed that step's
+    // barrier) from a ring of D register stages.  Loads past the last chunk take it again (a cache hit), so every load is
+    // unconditional; whole groups of D steps run unconditionally with a scheduling barrier after each step's loads, and
+    // the remainder (already loaded, whole chains) follows.
+    WideLds ls[D];
+    WideW ws[D];
+    auto chunk = [&](int s) __attribute__((always_inline)) { return min(s, steps - 1); };
+#pragma unroll
+    for (int j = 0; j < D; ++j) wide_load_lds<CG, PACKED>(p, src, chunk(j), ls[j]);
+    if constexpr (PACKED) {
+#pragma unroll
+        for (int j = 0; j < D; ++j) wide_load_w(p, src, chunk(j), ws[j]);
+    }
+    wide_store_lds<PACKED>(ls[0], lds);
+    wide_load_lds<CG, PACKED>(p, src, chunk(D), ls[0]);
+    __builtin_amdgcn_sched_barrier(0);
+    __syncthreads();
+    auto step = [&](int base, auto J) __attribute__((always_inline)) {
+        constexpr int j = decltype(J)::value;  // every register index is a constant (else the stages go to scratch memory)
+        // (always so here; as a branch it keeps the step apart from its neighbours' loads: without it the planes' form had
+        // 364 registers)
+        if (base + j < steps)
+            wide_compute<A, PACKED, j % CG == 0, j % CG == CG - 1>(lds + (j & 1) * kStage, ws[j], tc, acc);
+        if constexpr (PACKED) wide_load_w(p, src, chunk(base + j + D), ws[j]);
+        wide_store_lds<PACKED>(ls[(j + 1) % D], lds + ((j + 1) & 1) * kStage);
+        wide_load_lds<CG, PACKED>(p, src, chunk(base + j + 1 + D), ls[(j + 1) % D]);
+        __builtin_amdgcn_sched_barrier(0);
+        __syncthreads();
+    };
+    const int full = steps / D * D;
+    for (int base = 0; base < full; base += D) unroll<D>([&](auto J) __attribute__((always_inline)) { step(base, J); });
+    unroll<D - 1>([&](auto J) __attribute__((always_inline)) {
+        if (full + decltype(J)::value < steps) step(full, J);
+    });
+    if (p.out_dtype == W6A16_OUT_F16) wide_store<true>(p, b, m0, n0, acc);
+    else wide_store<false>(p, b, m0, n0, acc);
+}
 
 // Dequantise the packed layout: one wavefront per (b, strip, chunk).  HBM-bound (0.75 byte read and 2 written per weight
 // for bf16) once the stores are whole lines: the block's codes, one column's rows per lane, are turned in LDS -- by
@@ -1405,6 +1743,38 @@ int launch_tile_plan(Args& p, const TilePlan& t, hipStream_t s) {
     return t.cw == 2 ? launch_tile<A, 4, 8, 4, 2, 2, 1, 8, PACKED>(p, t, s) : launch_tile<A, 4, 8, 4, 1, 2, 1, 8, PACKED>(p, t, s);
 }
 
+// Whether a call runs the wide kernel: the sizes decide, not the format, so that planes and packed weights give the same
+// bits.  145..256 rows (of three groups of 64 the last then has 17 rows or more; K = 4096, N = 32768, us, planes / packed,
+// tile against wide: M = 144 83.4 / 70.8 against 95.3 / 78.9, 145 88.9 / 79.5 against 89.6 / 79.2, 176 92.3 / 83.0 against 93.5
+// / 77.1), eight chunks (with four as fast), two tiles and more to a CU, of which the last two rounds fill a quarter (K =
+// 4096, M = 193, tile against wide: N = 16384 59.2 / 55.3 against 56.7 / 48.0, 17408 78.0 / 65.6 against 87.9 / 73.0, 20480
+// 88.2 / 77.0 against 88.7 / 73.7), and every range that a buffer covers below 2 GB.
+bool wide_call(const w6a16_args* a, const Layout& l) {
+    if (l.big || a->M <= 144 || a->M > 256 || a->K < 512) return false;
+    const int64_t tiles = (int64_t)a->B * l.m_groups * l.n_strips, twice = 2 * cu_count(), last = tiles % twice;
+    if (tiles < twice || (last > 0 && 4 * last < twice)) return false;
+    const int64_t limit = 0x7FFFFFFF;
+    return ((int64_t)(a->M - 1) * a->a_row_stride + a->K) * 2 < limit && (int64_t)(a->K / 2) * a->N < limit &&
+           (int64_t)(a->K / a->group_k) * a->N * 2 < limit;
+}
+
+template <class A, bool PACKED>
+int launch_wide(Args& p, const w6a16_args* a, const Layout& l, hipStream_t s) {
+    const uint64_t wgs = tile_grid(p.N / 16, l.m_groups, kTiles, p.grid);  // (K N < 2^32: within one launch)
+    p.group = divisor(p.group_k / 64);
+    p.groups = p.K / p.group_k;
+    p.chain_k = p.group_k % 128 == 0 ? 128 : 64;
+    p.nchains = l.nchains;
+    p.mpad = l.m_groups * kWideRows;
+    p.rsum = reinterpret_cast<float*>(static_cast<char*>(a->workspace) + kCounterRegion + l.partial_bytes);
+    hipLaunchKernelGGL(w6a16_rowsum_kernel<A>, dim3(p.mpad / 4, (p.K + 511) / 512, p.B), dim3(256), 0, s, p);
+    if (p.chain_k == 128)
+        hipLaunchKernelGGL((w6a16_wide_kernel<A, 2, PACKED>), dim3((unsigned)wgs, 1, p.B), dim3(256), 0, s, p);
+    else
+        hipLaunchKernelGGL((w6a16_wide_kernel<A, 1, PACKED>), dim3((unsigned)wgs, 1, p.B), dim3(256), 0, s, p);
+    return WKV7_OK;
+}
+
 // The kernel for the call's shape and layout, with activations of type A.
 template <class A>
 int launch_matmul(Args& p, const w6a16_args* a, const Layout& l, hipStream_t s) {
@@ -1414,6 +1784,7 @@ int launch_matmul(Args& p, const w6a16_args* a, const Layout& l, hipStream_t s) 
         hipLaunchKernelGGL(w6a16_big_kernel<A>, dim3(tiles, 1, p.B), dim3(512), 0, s, p);
         return WKV7_OK;
     }
+    if (wide_call(a, l)) return packed ? launch_wide<A, true>(p, a, l, s) : launch_wide<A, false>(p, a, l, s);
     const TilePlan t = tile_plan(a, l, packed);
     return packed ? launch_tile_plan<A, true>(p, t, s) : launch_tile_plan<A, false>(p, t, s);
 }

@@ -58,6 +58,32 @@ def test_tile_shapes(B, M, N, K, g, split, dtype):
 
 
 @pytest.mark.parametrize("B,M,N,K,g,split", [
+    (1, 193, 16384, 512, 128, None),   # chains of two chunks, the last rows' group with one row
+    (1, 256, 16336, 576, 64, None),    # chains of one, nine chunks, columns that end inside a strip
+    (2, 150, 10896, 640, 128, None),   # a batch, five chains
+    (1, 200, 16384, 704, 64, 4),       # eleven chunks; a split beside it changes nothing
+])
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
+def test_wide_kernel(B, M, N, K, g, split, dtype):
+    """145..256 rows over so many columns that 64 x 128 tiles go twice around the CUs."""
+    from rwkv_next_amd.kernels import int6_gemm as I6
+    say("w6a16 wide", dict(B=B, M=M, N=N, K=K, g=g, split=split, dtype=dtype))
+    rng = np.random.default_rng(12000 + M + N + K)
+    lo, hi, sc = _weights(rng, B, K, N, g)
+    a = _act(rng, B, M, K)
+    if dtype == "f16":
+        a = a.to(torch.float16)
+    Ld, Hd, Sd = _dev(lo, hi, sc)
+    split = _split(split, B, M, N, K)
+    C = I6.int6_matmul(a.to(DEV), Ld, Hd, Sd, g, split_k=split, out_dtype=torch.float32)
+    Cp = I6.int6_matmul(a.to(DEV), I6.prepack_int6(Ld, Hd, Sd, g), split_k=split, out_dtype=torch.float32)
+    narrow = I6.int6_matmul(a.to(DEV), Ld, Hd, Sd, g, split_k=split)
+    torch.cuda.synchronize()
+    assert torch.equal(C, Cp) and torch.equal(narrow, C.to(a.dtype))
+    _check(C, a, lo, hi, sc, g, KERNEL_TOL if dtype == "bf16" else F16_KERNEL_TOL)
+
+
+@pytest.mark.parametrize("B,M,N,K,g,split", [
     (2, 3, 80, 256, 64, None),      # one row tile, as many parts as chunks
     (1, 40, 144, 2048, 128, None),  # eight parts, where 16 rows would have 16
     (1, 3, 64, 16384, 128, 32),     # 32 parts over two workgroups

@@ -229,10 +229,10 @@ struct TileW {
     uint32_t lo[2 * NT], hd[NT < 2 ? 2 : NT], sc[2];
 };
 // Planes: lane (i, q) holds lo-plane rows 8 q + e (e = 0..7) and hi-plane rows 8 (q & 1) + 4 (q >> 1) + e (e = 0..3) of
-// columns n0 + 4 i .. + 3, which are its columns of tiles 0..3 (tile t: columns n0 + 4 i + t).
+// columns n0 + NT i .. + NT - 1, NT / 4 words a row, which are its columns of tiles 0..NT - 1 (tile t: columns n0 + NT i + t).
 template <int NT>
 struct TileW<NT, false> {
-    uint32_t lo[8], hd[4], sc[2];
+    uint32_t lo[2 * NT], hd[NT], sc[NT / 2];
 };
 
 // The wavefront's loads: wave-uniform 64-bit bases (moved from chunk to chunk on the scalar unit) and 32-bit per-lane
@@ -248,7 +248,7 @@ struct TileSrc {
     uint64_t fa[2];
 };
 
-template <int MT, bool PACKED, bool FAR>
+template <int MT, int NT, bool PACKED, bool FAR>
 __device__ __forceinline__ TileSrc tile_src(const Args& p, int b, int m0, int tile, int row0) {
     const int lane = threadIdx.x & 63, i = lane & 15, q = lane >> 4;
     TileSrc s;
@@ -274,7 +274,7 @@ __device__ __forceinline__ TileSrc tile_src(const Args& p, int b, int m0, int ti
         s.vlo = s.vhi = 16 * lane;
         s.vsc = 16 * i;
     } else {
-        const uint32_t n = min(16u * tile + 4u * i, (uint32_t)p.N - 4);  // (unsigned: N up to 2^31 - 16)
+        const uint32_t n = min(16u * tile + (uint32_t)NT * i, (uint32_t)p.N - NT);  // (unsigned: N up to 2^31 - 16)
         const int hrow = 8 * (q & 1) + 4 * (q >> 1);
         s.lo = reinterpret_cast<uint64_t>(p.lo + (int64_t)b * p.sl_b);
         s.hi = reinterpret_cast<uint64_t>(p.hi + (int64_t)b * p.sh_b);
@@ -329,6 +329,7 @@ __device__ __forceinline__ void tile_load_w(const Args& p, const TileSrc& src, i
         const uint64_t lo = src.lo + (uint64_t)c * 32 * (uint64_t)p.N, hi = src.hi + (uint64_t)c * 16 * (uint64_t)p.N;
         const uint64_t sc = src.sc + (uint64_t)g * 2 * (uint64_t)p.N;
         if constexpr (FAR) {
+            static_assert(NT == 4, "far: 64 columns to a workgroup");
             typedef const __attribute__((address_space(1))) uint32_t* Words;
 #pragma unroll
             for (int e = 0; e < 8; ++e) s.lo[e] = *reinterpret_cast<Words>(lo + (uint64_t)(src.flo + (int64_t)e * p.N));
@@ -336,7 +337,7 @@ __device__ __forceinline__ void tile_load_w(const Args& p, const TileSrc& src, i
             for (int e = 0; e < 4; ++e) s.hd[e] = *reinterpret_cast<Words>(hi + (uint64_t)(src.fhi + (int64_t)e * p.N));
 #pragma unroll
             for (int d = 0; d < 2; ++d) s.sc[d] = reinterpret_cast<Words>(sc + (uint64_t)src.fsc)[d];  // (4-byte aligned)
-        } else {
+        } else if constexpr (NT == 4) {
 #pragma unroll
             for (int e = 0; e < 8; ++e)
                 s.lo[e] = __builtin_amdgcn_raw_buffer_load_b32(tile_rsrc(lo, kAll), src.vlo, e * p.N, 0);
@@ -345,6 +346,22 @@ __device__ __forceinline__ void tile_load_w(const Args& p, const TileSrc& src, i
                 s.hd[e] = __builtin_amdgcn_raw_buffer_load_b32(tile_rsrc(hi, kAll), src.vhi, e * p.N, 0);
             const uint2 z = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(tile_rsrc(sc, kAll), src.vsc, 0, 0));
             s.sc[0] = z.x, s.sc[1] = z.y;
+        } else {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const uint2 x = __builtin_bit_cast(
+                    uint2, __builtin_amdgcn_raw_buffer_load_b64(tile_rsrc(lo, kAll), src.vlo, e * p.N, 0));
+                s.lo[2 * e] = x.x, s.lo[2 * e + 1] = x.y;
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const uint2 x = __builtin_bit_cast(
+                    uint2, __builtin_amdgcn_raw_buffer_load_b64(tile_rsrc(hi, kAll), src.vhi, e * p.N, 0));
+                s.hd[2 * e] = x.x, s.hd[2 * e + 1] = x.y;
+            }
+            const u4 z = __builtin_amdgcn_raw_buffer_load_b128(tile_rsrc(sc, kAll), src.vsc, 0, 0);
+#pragma unroll
+            for (int d = 0; d < 4; ++d) s.sc[d] = z[d];
         }
     }
 }
@@ -378,9 +395,9 @@ __device__ __forceinline__ void tile_load_a(const Args& p, const TileSrc& src, i
 __device__ __forceinline__ int a_slot(int r, int j) { return 8 * r + (j ^ ((r >> 1) & 7)); }
 
 // Column tile t's weight operands (rows 8 q .. and 32 + 8 q .. of the chunk) and scale.  u0, u1: the planes' codes of
-// rows 8 q + e and 32 + 8 q + e, four columns each.
+// rows 8 q + e and 32 + 8 q + e, NT / 4 words of four columns each.
 template <class A, int NT, bool PACKED>
-__device__ __forceinline__ void tile_dequant(const TileW<NT, PACKED>& s, const uint32_t (&u0)[8], const uint32_t (&u1)[8],
+__device__ __forceinline__ void tile_dequant(const TileW<NT, PACKED>& s, const uint32_t (&u0)[2 * NT], const uint32_t (&u1)[2 * NT],
                                              int t, int tsel, u4& w0, u4& w1, float& sv) {
     uint32_t o0[4], o1[4];
     uint32_t sw;
@@ -398,8 +415,10 @@ __device__ __forceinline__ void tile_dequant(const TileW<NT, PACKED>& s, const u
         constexpr uint32_t kPair[2] = {0x05010400u, 0x07030602u};  // columns 0, 1 and 2, 3
 #pragma unroll
         for (int d = 0; d < 4; ++d) {
-            const uint32_t x = __builtin_amdgcn_perm(u0[2 * d + 1], u0[2 * d], kPair[t >> 1]);
-            const uint32_t y = __builtin_amdgcn_perm(u1[2 * d + 1], u1[2 * d], kPair[t >> 1]);
+            constexpr int C = NT / 4;
+            const int r0 = 2 * d * C + (t >> 2), r1 = r0 + C;
+            const uint32_t x = __builtin_amdgcn_perm(u0[r1], u0[r0], kPair[(t >> 1) & 1]);
+            const uint32_t y = __builtin_amdgcn_perm(u1[r1], u1[r0], kPair[(t >> 1) & 1]);
             o0[d] = __builtin_amdgcn_perm(A::kCodeHi, x, t & 1 ? 0x04030402u : 0x04010400u);
             o1[d] = __builtin_amdgcn_perm(A::kCodeHi, y, t & 1 ? 0x04030402u : 0x04010400u);
         }
@@ -425,18 +444,18 @@ __device__ __forceinline__ void tile_work(const TileW<NT, PACKED>& s, const uint
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
         for (int h = 0; h < 2; ++h) a[mt][h] = *reinterpret_cast<const u4*>(ra[h] + 2048 * mt);
-    uint32_t u0[8], u1[8];
+    uint32_t u0[2 * NT], u1[2 * NT];
     if constexpr (!PACKED) {
         const int sel = 2 * (q >> 1);  // the hi plane's field of rows 8 q ..
-        uint32_t hd[8];                // hi-plane rows 8 (q & 1) + e: the lower half-wavefront's four, then the upper's
+        uint32_t hd[2 * NT];           // hi-plane rows 8 (q & 1) + e: the lower half-wavefront's four, then the upper's
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
+        for (int e = 0; e < NT; ++e) {
             const auto x = __builtin_amdgcn_permlane32_swap(s.hd[e], s.hd[e], false, false);
             hd[e] = x[0];
-            hd[4 + e] = x[1];
+            hd[NT + e] = x[1];
         }
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
+        for (int e = 0; e < 2 * NT; ++e) {
             const uint32_t L = s.lo[e], H = hd[e] >> sel;
             u0[e] = (L & 0x0F0F0F0Fu) | ((H & 0x03030303u) << 4);
             u1[e] = ((L >> 4) & 0x0F0F0F0Fu) | (H & 0x30303030u);
@@ -512,7 +531,7 @@ constexpr int tile_lds(int MT, int NA, int NT) { return 1024 * (MT * NT > NA ? M
 // double-buffered and the workgroup meets at one barrier per chunk.
 template <class A, int MT, int NA, int NT, int CW, int D, int DA, int MAXW, bool PACKED, bool FAR>
 __global__ __launch_bounds__(64 * MAXW) void w6a16_tile_kernel(const Args p) {
-    static_assert(PACKED || NT == 4, "planes: four column tiles");
+    static_assert(PACKED ? NT <= 4 : NT == 4 || NT == 8, "packed: up to four column tiles; planes: four or eight");
     static_assert(!FAR || (MT == 1 && NT == 4 && CW == 1), "far: 16 rows, 64 columns to a workgroup");
     static_assert(D % DA == 0, "stage rings");
     static_assert(CW == 1 || (CW == 2 && D == 2 && DA == 1 && NA % 2 == 0), "one or two column wavefronts");
@@ -539,7 +558,7 @@ __global__ __launch_bounds__(64 * MAXW) void w6a16_tile_kernel(const Args p) {
     const int ri = NA == 1 ? lane & 7 : lane & 15;
     const uint8_t* const ra[2] = {abuf + 16 * a_slot(ri, lane >> 4), abuf + 16 * a_slot(ri, 4 + (lane >> 4))};
 
-    const TileSrc src = tile_src<MT, PACKED, FAR>(p, b, m0, tile, 8 * NW * cw);
+    const TileSrc src = tile_src<MT, NT, PACKED, FAR>(p, b, m0, tile, 8 * NW * cw);
     f4 acc[MT][NT];
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
@@ -628,7 +647,7 @@ __global__ __launch_bounds__(64 * MAXW) void w6a16_tile_kernel(const Args p) {
     const int rows = min(16 * MT, p.M - m0), n0 = 16 * wtile;
     const int col = tid % NC, step = blockDim.x / NC;
     auto each_sum = [&](auto sink) __attribute__((always_inline)) {
-        const int c = col % (16 * NT), t = PACKED ? c >> 4 : c & 3, i = PACKED ? c & 15 : c >> 2;
+        const int c = col % (16 * NT), t = PACKED ? c >> 4 : c % NT, i = PACKED ? c & 15 : c / NT;
         const f4* const sums = reinterpret_cast<const f4*>(lds) + (col / (16 * NT) * MT * NT + t) * 64 + i;
         constexpr int kPart = CW * MT * NT * 64;
         auto four = [&](int r4) __attribute__((always_inline)) { return sums + (r4 >> 2) * NT * 64 + 16 * (r4 & 3); };
@@ -1626,7 +1645,7 @@ TilePlan tile_plan(const w6a16_args* a, const Layout& l, bool packed) {
     t.parts = std::min(chunks, wide * spread(t.mt, t.cw, wide));
     auto fits = [&](int ks, int max_w) { return ks == 1 ? t.parts <= max_w : t.parts % 4 == 0 && t.parts / ks <= max_w; };
     // Columns to a wavefront and workgroups to a K range.  Packed: as few workgroups to a K range as hold the parts, and
-    // the columns whose rounds cost least.  Planes: always 64 columns (a lane loads four), K spread over more workgroups
+    // the columns whose rounds cost least.  Planes: 64 columns (a lane loads four), K spread over more workgroups
     // while every one of them still gets a CU and, from two row tiles on, a part has six chunks: their partial tiles then
     // cost more than what a short loop gains (six products of C = 768, M = 33: 69 us spread, 53 not; C = 2560, five chunks
     // a part, M = 48: 90.8 / 85.8; C = 4096, eight, M = 64: 133 / 141; one row tile, C = 2560, M = 1: 59.6 / 64.7).
@@ -1644,6 +1663,10 @@ TilePlan tile_plan(const w6a16_args* a, const Layout& l, bool packed) {
         const int64_t cost = rounds(wgs(t.mt, nt * t.cw) * ks) * (2 * nt + 3 * t.mt);
         if (!best || cost < best) best = cost, t.nt = nt, t.ks = ks;
     }
+    // Planes, one row tile, 128 columns to a workgroup where that leaves every CU one: eight columns a lane, half the load
+    // instructions (us, four / eight columns: K = 4096, M = 16, N = 65536 58.5 / 44.0, 32768 31.7 / 24.4, 16384 19.1 / 21.7).
+    // (Two parts at least: the outputs take a thread a column.)
+    if (!packed && t.mt == 1 && t.ks == 1 && t.parts >= 2 && t.parts <= 8 && wgs(1, 8) >= cus) t.nt = 8;
     // Planes, deep K, a single round of workgroups of two row tiles: half as many groups of rows, of up to twice the rows, and
     // the same parts over two workgroups, since the planes' loads are what takes the time there (K = 16384, N = 4096, us, two
     // row tiles / three or four: M = 65 47.7 / 36.6, 128 48.1 / 42.4; K = 8192: 25.9 / 25.7, 26.8 / 29.4).
@@ -1707,6 +1730,7 @@ int launch_tile(Args& p, const TilePlan& t, hipStream_t s) {
     p.per_part = (chunks + t.parts - 1) / t.parts;
     p.groups = p.K / p.group_k;
     const uint32_t block = 64 * CW * t.parts / t.ks, most = launch_limit(block);
+    if (block < 16 * NT * CW || block > 64 * MAXW) return WKV7_ERR_SHAPE;  // (no plan: the outputs take a thread a column)
     for (uint64_t x = 0; x < wgs; x += most) {
         p.grid.first = (uint32_t)(x / 8);
         hipLaunchKernelGGL((w6a16_tile_kernel<A, MT, NA, NT, CW, D, DA, MAXW, PACKED, FAR>),
@@ -1722,6 +1746,8 @@ int launch_tile_one(Args& p, const TilePlan& t, hipStream_t s) {  // one row til
     if constexpr (PACKED) {
         if (t.nt == 1) return launch_tile<A, 1, NA, 1, 1, 4, 4, 16, true>(p, t, s);
         if (t.nt == 2) return launch_tile<A, 1, NA, 2, 1, 4, 4, 16, true>(p, t, s);
+    } else {
+        if (t.nt == 8) return launch_tile<A, 1, NA, 8, 1, 2, 2, 8, false>(p, t, s);
     }
     if (t.parts / t.ks > 8) return launch_tile<A, 1, NA, 4, 1, 2, 2, 16, PACKED>(p, t, s);
     return launch_tile<A, 1, NA, 4, 1, 4, 4, 8, PACKED>(p, t, s);

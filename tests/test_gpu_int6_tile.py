@@ -35,6 +35,9 @@ from test_gpu_int6 import DEV, F16_KERNEL_TOL, KERNEL_TOL, _act, _check, _dev, _
     (1, 20, 33024, 576, 64, 1),      # several rounds: two parts, two row tiles
     (1, 128, 33024, 320, 64, 1),     # one part, four row tiles, 128 columns
     (1, 16, 256, 1088, 64, 1),       # 16 parts, 17 chunks
+    (1, 3, 32768, 128, 64, 1),       # planes: eight column tiles a wavefront, two parts of one chunk
+    (1, 9, 32784, 320, 64, 1),       # the same, columns that end inside a workgroup's
+    (1, 9, 32784, 64, 64, 1),        # one part: four column tiles
     (1, 70, 2752, 16384, 128, 4),    # deep K, one round: planes three row tiles over two workgroups, packed two in one
     (1, 190, 1408, 16384, 128, 2),   # planes four row tiles
     (1, 190, 1408, 16384, 128, 1),   # no room for partial tiles: two row tiles

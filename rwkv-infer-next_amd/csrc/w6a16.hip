@@ -28,7 +28,7 @@
 #include <utility>
 
 #include "w6a16.h"
-#include "w6a16_grid.h"
+#include "w6a16_plan.h"
 #include "wkv7_launch.h"
 
 namespace w6 {
@@ -39,14 +39,6 @@ typedef float f4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u4 __attribute__((ext_vector_type(4)));
 typedef int v2i __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(3))) v2i lds_v2i;
-
-constexpr int kTileN = 128;          // columns per strip of the packed layout
-constexpr int kTiles = kTileN / 16;  // 16-column tiles per strip
-constexpr int kCounterAlign = 256;   // bytes: workspace alignment
-// The arrival counters occupy a fixed region at the start of the workspace, the partials follow it.  Calls with
-// different tile counts can share one workspace: the partials of one call never overlap the counters of another,
-// and every call leaves the counters it used at zero.
-constexpr size_t kCounterRegion = size_t(1) << 20;
 
 struct Args {
     const uint16_t* a;
@@ -176,8 +168,6 @@ __device__ __forceinline__ float2 coherent_load2(const float* p) {
 //                       32 + 8 q + 4 + e' at bits 0-1, 2-3, 4-5, 6-7
 // Scales: block (b, strip, group) of 128 fp16 at ((b * strips + strip) * groups + group) * 128, ordered [i][t], so
 // lane (i, q) reads its eight columns' scales as one 16-byte load.  Columns past N hold zero codes and scales.
-constexpr int kPackBytes = 6144;
-
 using wkv7::unroll;  // f(integral_constant<0>), .., f(integral_constant<N - 1>)
 
 // A raw buffer over [base, base + bytes) (capped at 2 GB).  The base and size are passed through readfirstlane so that
@@ -1523,168 +1513,6 @@ int cu_count() { return wkv7::device_cu_count(); }
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
-// Large-M kernel: M above this, packed weights (no workspace, no split-K).
-constexpr int kBigMinM = 256;
-// (its loads go through raw buffers: A's batch slice and the packed weight's below 2 GB)
-bool big_rows(const w6a16_args* a) {
-    if (a->M <= kBigMinM || a->format != W6A16_FORMAT_PACKED || a->K < 64) return false;
-    const int64_t a_bytes = ((int64_t)(a->M - 1) * a->a_row_stride + a->K) * 2;
-    const int64_t w_bytes = (int64_t)((a->N + kTileN - 1) / kTileN) * (a->K / 64) * kPackBytes;
-    return a_bytes < 0x7FFFFFFF && w_bytes < 0x7FFFFFFF;
-}
-
-// Rows of A up to which a split of 2..8 needs no workspace (include/w6a16.h, w6a16_workspace_size).
-constexpr int kSmallM = 32;
-constexpr int kGemvMaxSplit = 8;
-
-// The workspace that include/w6a16.h promises for a shape and split: the counter region, partial tiles of split_k ranges
-// and, above 32 rows, one float per row and two chunks of K.  The tile kernel uses what it needs of it (counters and
-// partial tiles where it splits K over workgroups; the last part stays unused).
-struct Layout {
-    bool big;                    // the large-M kernel
-    bool wide, gemv, gemv_half;  // wide: more than 32 rows; gemv: at most 32, no workspace; gemv_half: of those, packed
-                                 // weights with fewer strips than CUs
-    int kp, m_groups, n_strips, nchains;
-    size_t tiles, partial_bytes, total_bytes;
-};
-
-Layout layout(const w6a16_args* a) {
-    Layout l{};
-    l.big = big_rows(a);
-    l.wide = !l.big && a->M > kSmallM;
-    l.n_strips = (a->N + kTileN - 1) / kTileN;
-    if (l.big) return l;  // no workspace
-    const int mt = !l.wide ? 1 : a->M <= 64 ? 2 : 4;
-    l.kp = l.wide && a->M <= 128 ? 2 : 1;
-    l.nchains = a->K / (a->group_k % 128 == 0 ? 128 : 64);
-    const int rows_per_group = 16 * mt;
-    l.m_groups = (a->M + rows_per_group - 1) / rows_per_group;
-    l.gemv = !l.wide && a->split_k >= 2 && a->split_k <= kGemvMaxSplit &&
-             (a->format == W6A16_FORMAT_PACKED || (int64_t)a->B * l.m_groups * l.n_strips >= cu_count());
-    l.gemv_half = l.gemv && a->format == W6A16_FORMAT_PACKED && (int64_t)a->B * l.m_groups * l.n_strips < cu_count();
-    if ((a->split_k > 1 && !l.gemv) || l.wide) {
-        l.tiles = (size_t)a->B * l.m_groups * l.n_strips;
-        l.partial_bytes = a->split_k > 1 ? l.tiles * a->split_k * (size_t)rows_per_group * kTileN * 4 : 0;
-        l.total_bytes = kCounterRegion + l.partial_bytes +
-                        (l.wide ? (size_t)a->B * l.nchains * l.m_groups * rows_per_group * 4 : 0);
-    }
-    return l;
-}
-
-// The tile kernel's shape for a call: MT 16-row tiles, NT 16-column tiles a wavefront and CW wavefronts side by side to a
-// workgroup, K shared by `parts`, in ks workgroups.
-struct TilePlan {
-    int mt, nt, cw, parts, ks;
-    bool far;
-};
-
-// mt, cw and parts depend on the sizes and on split_k only, not on the format, so that planes and packed weights give the
-// same bits.  A CU takes its workgroups one after the other, so a shape costs its rounds over the CUs times what one
-// workgroup costs per chunk: the KB that pass the CU's L1, 2 per row tile and 3.5 per 64 columns.
-TilePlan tile_plan(const w6a16_args* a, const Layout& l, bool packed) {
-    TilePlan t{};
-    const int64_t cus = cu_count();
-    const int chunks = a->K / 64, tiles = a->N / 16;
-    auto groups = [&](int mt) { return (int64_t)a->B * ((a->M + 16 * mt - 1) / (16 * mt)); };
-    auto wgs = [&](int mt, int nt) { return groups(mt) * ((tiles + nt - 1) / nt); };
-    auto rounds = [&](int64_t n) { return (n + cus - 1) / cus; };
-    // Workgroups that may share a tile's K: none without room for their counters and partial tiles (so split_k bounds it;
-    // up to 32 rows a split of at most 8 has no workspace).
-    auto room = [&](int mt, int cw) {
-        int most = a->M <= kSmallM ? (a->split_k > kGemvMaxSplit ? 4 : 1) : a->split_k >= 4 ? 4 : a->split_k >= 2 ? 2 : 1;
-        if ((size_t)(groups(mt) * tiles) * 4 > kCounterRegion) most = 1;
-        while (most > 1 && (size_t)wgs(mt, 4 * cw) * most * 16 * mt * 64 * cw * 4 > l.partial_bytes) most >>= 1;
-        return most;
-    };
-    // Workgroups of `wide` K parts for whose parts a deep K has work where CUs would be left without.
-    auto spread = [&](int mt, int cw, int wide) {
-        const int64_t w4 = wgs(mt, 4 * cw), most = room(mt, cw);
-        int s = 1;
-        while (s < most && chunks >= wide * s * 2 && w4 * s * 2 <= cus &&
-               (chunks > 128 || (mt == 2 && w4 * 4 <= cus && s < 2)) && !(mt == 1 && s == 2))
-            s *= 2;
-        return s;
-    };
-    // Rows to a workgroup: one tile up to 16 rows, two up to 32; above, two to four tiles and, from three on, 64 or 128
-    // columns, whatever costs least (us, packed: K = N = 4096, M = 64: mt 2 10.3, mt 4 13.3; N = 16384: 25.6 / 22.2;
-    // K = N = 2560, M = 203: mt 2, 3, 4 14.9 / 11.4 / 12.8).
-    t.cw = 1;
-    if (a->M <= 16) {
-        t.mt = 1;
-    } else if (chunks <= 2) {
-        // what a workgroup writes costs more than what it reads (us, packed, N = 16384: K = 64, M = 64, mt 1, 2, 4 6.0 / 8.3 /
-        // 12.8; M = 256 11.9 / 11.2 / 17; K = 128, M = 128 9.9 / 7.9 / 10.3)
-        t.mt = wgs(1, 4) <= 4 * cus ? 1 : 2;
-    } else {
-        t.mt = 2;
-        auto cost = [&](int mt, int cw) { return rounds(wgs(mt, 4 * cw)) * (4 * mt + 7 * cw); };
-        int64_t best = cost(2, 1);
-        if (a->M > 32)
-            for (int mt = 3; mt <= 4; ++mt)
-                for (int cw = 1; cw <= 2; ++cw)
-                    if (cost(mt, cw) < best) best = cost(mt, cw), t.mt = mt, t.cw = cw;
-    }
-    const int64_t w4 = wgs(t.mt, 4 * t.cw);
-    const int most = room(t.mt, t.cw);
-    // Wavefronts that share K: eight to a workgroup (with two column wavefronts four), with one row tile 16 where the
-    // workgroups do not fill the chip and a part of 16 has more than one chunk, else 4 (us, packed / planes: K = 4096, N =
-    // 16384, M = 1: 4 12.4 / 16.2, 8 12.6 / 16.8, 16 13.3 / 17.7; K = N = 1024, M = 16: 4 4.0 / 5.6, 16 5.4 / 6.6; K = N = 2048,
-    // M = 1: 8 4.4 / 7.0, 16 5.2 / 6.4), and twice or four times as many where a deep K would otherwise leave CUs without work
-    // (K = 16384, N = 4096, M = 1: 16 parts in one workgroup 16.4, 32 in two 14.1).
-    int wide = t.mt == 1 ? (w4 < cus && chunks > 16 ? 16 : 4) : 8 / t.cw;
-    // Two row tiles and more, several rounds over the CUs: fewer to a workgroup, several of which then share a CU and fewer
-    // follow each other.  A round costs its chunks a part and about 4/3 of a chunk for its start and end (K = 1024, N = 65536,
-    // us, packed: M = 32, 8, 4, 2, 1 parts 25.5 / 18.8 / 18.7 / 20.5; M = 128, 4, 2, 1 53.9 / 46.3 / 43.8; M = 192 76.7 / 64.4 /
-    // 71.1; K = 4096, N = 16384, M = 128 32.2 / 41.9 / 69).
-    if (t.mt > 1) {
-        const int full = wide;
-        auto cost = [&](int n) { return (w4 * n + cus * full - 1) / (cus * full) * (3 * ((chunks + n - 1) / n) + 4); };
-        for (int n = full / 2; n >= 1 && w4 > cus; n /= 2)
-            if (cost(n) < cost(wide)) wide = n;
-    }
-    t.parts = std::min(chunks, wide * spread(t.mt, t.cw, wide));
-    auto fits = [&](int ks, int max_w) { return ks == 1 ? t.parts <= max_w : t.parts % 4 == 0 && t.parts / ks <= max_w; };
-    // Columns to a wavefront and workgroups to a K range.  Packed: as few workgroups to a K range as hold the parts, and
-    // the columns whose rounds cost least.  Planes: 64 columns (a lane loads four), K spread over more workgroups
-    // while every one of them still gets a CU and, from two row tiles on, a part has six chunks: their partial tiles then
-    // cost more than what a short loop gains (six products of C = 768, M = 33: 69 us spread, 53 not; C = 2560, five chunks
-    // a part, M = 48: 90.8 / 85.8; C = 4096, eight, M = 64: 133 / 141; one row tile, C = 2560, M = 1: 59.6 / 64.7).
-    int64_t best = 0;
-    for (int nt = packed ? 1 : 4; nt <= 4; nt *= 2) {
-        if (t.mt > 2 && nt < 4) continue;
-        const int max_w = t.mt == 1 || (t.mt == 2 && nt == 1) ? 16 : 8 / t.cw;
-        int ks = 1;
-        while (ks < most && !fits(ks, max_w)) ks *= 2;
-        if (!fits(ks, max_w)) continue;
-        if (!packed)
-            while (ks * 2 <= most && fits(ks * 2, max_w) && t.parts / (ks * 2) >= 4 && w4 * ks * 2 <= cus &&
-                   (t.mt == 1 || chunks >= 6 * t.parts))
-                ks *= 2;
-        const int64_t cost = rounds(wgs(t.mt, nt * t.cw) * ks) * (2 * nt + 3 * t.mt);
-        if (!best || cost < best) best = cost, t.nt = nt, t.ks = ks;
-    }
-    // Planes, one row tile, 128 columns to a workgroup where that leaves every CU one: eight columns a lane, half the load
-    // instructions (us, four / eight columns: K = 4096, M = 16, N = 65536 58.5 / 44.0, 32768 31.7 / 24.4, 16384 19.1 / 21.7).
-    // (Two parts at least: the outputs take a thread a column.)
-    if (!packed && t.mt == 1 && t.ks == 1 && t.parts >= 2 && t.parts <= 8 && wgs(1, 8) >= cus) t.nt = 8;
-    // Planes, deep K, a single round of workgroups of two row tiles: half as many groups of rows, of up to twice the rows, and
-    // the same parts over two workgroups, since the planes' loads are what takes the time there (K = 16384, N = 4096, us, two
-    // row tiles / three or four: M = 65 47.7 / 36.6, 128 48.1 / 42.4; K = 8192: 25.9 / 25.7, 26.8 / 29.4).
-    if (!packed && t.mt == 2 && t.ks == 1 && t.parts == 8 && most >= 2 && chunks >= 256)
-        for (int mt = 3; mt <= 4; ++mt)
-            if (wgs(mt, 4) * 2 <= cus && groups(mt) * 2 <= groups(2) + 1 &&
-                (size_t)wgs(mt, 4) * 2 * 16 * mt * 64 * 4 <= l.partial_bytes) {
-                t.mt = mt, t.ks = 2;
-                break;
-            }
-    // Planes whose 32 rows span 2 GB, rows of A of which 64 do: 16 rows and 64 columns to a workgroup, with 64-bit
-    // addresses, and the same parts, so the same bits as for the same rows packed or side by side.  (More than 16 parts
-    // come only with few tiles, whose counters and partial tiles have room.)
-    t.far = (!packed && a->N >= (1 << 26)) || (a->M > 1 ? a->a_row_stride : a->K) >= (1 << 24);
-    if (t.far) t.mt = 1, t.nt = 4, t.cw = 1, t.ks = t.parts > 16 ? 2 : 1;
-    return t;
-}
-
 int validate(const w6a16_args* a) {
     if (!a) return WKV7_ERR_NULL;
     if (a->B < 1 || a->M < 0 || a->N < 1 || a->K < 64 || a->K % 64 || a->N % 16) return WKV7_ERR_SHAPE;
@@ -1705,15 +1533,16 @@ int validate(const w6a16_args* a) {
                   a->scales_batch_stride % 2))
         return WKV7_ERR_ALIGN;
     if (a->a_row_stride < a->K || a->out_row_stride < a->N) return WKV7_ERR_SHAPE;
-    const Layout l = layout(a);
+    const Layout l = layout(a, cu_count());
     if (l.big) {  // grid (tiles, 1, B)
         const int64_t tiles = (int64_t)((a->M + kBigTile - 1) / kBigTile) * ((a->N + kBigTile - 1) / kBigTile);
         return (a->B > 65535 || tiles > 0x7FFFFFFF) ? WKV7_ERR_SHAPE : WKV7_OK;
     }
-    if ((int64_t)a->B * (l.wide ? 1 : l.m_groups) > 65535) return WKV7_ERR_SHAPE;  // grid z: batch (x M groups)
-    if (l.wide && (int64_t)l.m_groups * ((l.n_strips + 7) / 8) * 8 > 0x7FFFFFFF) return WKV7_ERR_SHAPE;
-    if (a->split_k > 1 && l.tiles * 4 > kCounterRegion) return WKV7_ERR_SHAPE;  // more tiles than counters (0: gemv)
-    if ((a->split_k > 1 && !l.gemv) || l.wide) {
+    const bool small = a->M <= kSmallM;
+    if ((int64_t)a->B * (small ? l.m_groups : 1) > 65535) return WKV7_ERR_SHAPE;  // (B: grid y, at most 65535)
+    if (!small && (int64_t)l.m_groups * ((l.n_strips + 7) / 8) * 8 > 0x7FFFFFFF) return WKV7_ERR_SHAPE;
+    if (a->split_k > 1 && l.tiles * 4 > kCounterRegion) return WKV7_ERR_SHAPE;  // more tiles than counters
+    if (l.total_bytes) {
         if (!a->workspace || a->workspace_bytes < l.total_bytes) return WKV7_ERR_WORKSPACE;
         if (reinterpret_cast<uintptr_t>(a->workspace) % kCounterAlign) return WKV7_ERR_ALIGN;
     }
@@ -1769,21 +1598,6 @@ int launch_tile_plan(Args& p, const TilePlan& t, hipStream_t s) {
     return t.cw == 2 ? launch_tile<A, 4, 8, 4, 2, 2, 1, 8, PACKED>(p, t, s) : launch_tile<A, 4, 8, 4, 1, 2, 1, 8, PACKED>(p, t, s);
 }
 
-// Whether a call runs the wide kernel: the sizes decide, not the format, so that planes and packed weights give the same
-// bits.  145..256 rows (of three groups of 64 the last then has 17 rows or more; K = 4096, N = 32768, us, planes / packed,
-// tile against wide: M = 144 83.4 / 70.8 against 95.3 / 78.9, 145 88.9 / 79.5 against 89.6 / 79.2, 176 92.3 / 83.0 against 93.5
-// / 77.1), eight chunks (with four as fast), two tiles and more to a CU, of which the last two rounds fill a quarter (K =
-// 4096, M = 193, tile against wide: N = 16384 59.2 / 55.3 against 56.7 / 48.0, 17408 78.0 / 65.6 against 87.9 / 73.0, 20480
-// 88.2 / 77.0 against 88.7 / 73.7), and every range that a buffer covers below 2 GB.
-bool wide_call(const w6a16_args* a, const Layout& l) {
-    if (l.big || a->M <= 144 || a->M > 256 || a->K < 512) return false;
-    const int64_t tiles = (int64_t)a->B * l.m_groups * l.n_strips, twice = 2 * cu_count(), last = tiles % twice;
-    if (tiles < twice || (last > 0 && 4 * last < twice)) return false;
-    const int64_t limit = 0x7FFFFFFF;
-    return ((int64_t)(a->M - 1) * a->a_row_stride + a->K) * 2 < limit && (int64_t)(a->K / 2) * a->N < limit &&
-           (int64_t)(a->K / a->group_k) * a->N * 2 < limit;
-}
-
 template <class A, bool PACKED>
 int launch_wide(Args& p, const w6a16_args* a, const Layout& l, hipStream_t s) {
     const uint64_t wgs = tile_grid(p.N / 16, l.m_groups, kTiles, p.grid);  // (K N < 2^32: within one launch)
@@ -1810,8 +1624,8 @@ int launch_matmul(Args& p, const w6a16_args* a, const Layout& l, hipStream_t s) 
         hipLaunchKernelGGL(w6a16_big_kernel<A>, dim3(tiles, 1, p.B), dim3(512), 0, s, p);
         return WKV7_OK;
     }
-    if (wide_call(a, l)) return packed ? launch_wide<A, true>(p, a, l, s) : launch_wide<A, false>(p, a, l, s);
-    const TilePlan t = tile_plan(a, l, packed);
+    if (wide_call(a, l, cu_count())) return packed ? launch_wide<A, true>(p, a, l, s) : launch_wide<A, false>(p, a, l, s);
+    const TilePlan t = tile_plan(a, l, packed, cu_count());
     return packed ? launch_tile_plan<A, true>(p, t, s) : launch_tile_plan<A, false>(p, t, s);
 }
 
@@ -1824,61 +1638,23 @@ size_t w6a16_args_size(void) { return sizeof(w6a16_args); }
 
 int w6a16_workspace_size(const w6a16_args* a, size_t* bytes) {
     if (!a || !bytes) return WKV7_ERR_NULL;
-    if (a->M <= 0 || a->B < 1 || a->N < 1 || a->K < 64 || a->group_k < 64 ||
-        (a->split_k <= 1 && a->M <= w6::kSmallM) || w6::big_rows(a)) {
-        *bytes = 0;
-        return WKV7_OK;
-    }
-    const w6::Layout l = w6::layout(a);
-    *bytes = l.total_bytes;
+    const bool none = a->M <= 0 || a->B < 1 || a->N < 1 || a->K < 64 || a->group_k < 64;
+    *bytes = none ? 0 : w6::layout(a, w6::cu_count()).total_bytes;
     return WKV7_OK;
 }
 
 int w6a16_plan_split(int32_t B, int32_t M, int32_t N, int32_t K) {
-    if (B < 1 || M < 1 || N < 1 || K < 64) return 1;
-    w6a16_args shape{};
-    shape.B = B;
-    shape.M = M;
-    shape.N = N;
-    shape.K = K;
-    shape.group_k = K % 128 == 0 ? 128 : 64;  // chains of two chunks where K allows them
-    const w6::Layout l = w6::layout(&shape);
-    // The rule's units: for M <= 32 four 128-column strips per 16 rows, with one unit per CU; above, one strip per M group
-    // and eight wavefronts (4 KP a unit) per CU.
-    const int64_t groups = (int64_t)B * l.m_groups * (l.wide ? l.n_strips : (l.n_strips + 3) / 4);
-    const int chunks = l.wide ? l.nchains : K / 64;  // the units a split range holds
-    const int64_t cus = l.wide ? w6::cu_count() * 2 / l.kp : w6::cu_count();
-    // The smallest power of two that gives every CU a unit (every range keeps at least one chunk); then doubled while
-    // ranges keep at least 16 chunks and the launch stays within one unit per CU.
-    int sk = 1;
-    while (groups * sk < cus && sk * 2 <= 64 && chunks / (sk * 2) >= 1) sk *= 2;
-    while (chunks / (sk * 2) >= 16 && groups * sk * 2 <= cus && sk * 2 <= 64) sk *= 2;
-    if (!l.wide && sk >= 2 && (int64_t)B * l.m_groups * l.n_strips >= cus)
-        while (sk * 2 <= w6::kGemvMaxSplit && chunks / (sk * 2) >= 1) sk *= 2;
-    return sk;
+    return B < 1 || M < 1 || N < 1 || K < 64 ? 1 : w6::plan_split(B, M, N, K, w6::cu_count());
 }
 
 int w6a16_plan_split_packed(int32_t B, int32_t M, int32_t N, int32_t K) {
-    const int sk = w6a16_plan_split(B, M, N, K);
-    if (sk != 8) return sk;
-    w6a16_args shape{};
-    shape.B = B;
-    shape.M = M;
-    shape.N = N;
-    shape.K = K;
-    shape.group_k = K % 128 == 0 ? 128 : 64;
-    shape.split_k = sk;
-    shape.format = W6A16_FORMAT_PACKED;
-    const w6::Layout l = w6::layout(&shape);
-    // shallower where a batch's strips are fewer than the CUs and the ranges keep at least 8 chunks
-    if (l.gemv_half && K / 64 / 4 >= 8) return 4;
-    return sk;
+    return B < 1 || M < 1 || N < 1 || K < 64 ? 1 : w6::plan_split_packed(B, M, N, K, w6::cu_count());
 }
 
 int w6a16_matmul(const w6a16_args* a, void* stream) {
     const int rc = w6::validate(a);
     if (rc != WKV7_OK || a->M == 0) return rc;
-    const w6::Layout l = w6::layout(a);
+    const w6::Layout l = w6::layout(a, w6::cu_count());
     w6::Args p{};
     p.a = a->a;
     p.sa_b = a->a_batch_stride;

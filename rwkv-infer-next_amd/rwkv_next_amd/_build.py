@@ -27,7 +27,7 @@ SOURCES = ("wkv7_recurrent.hip", "wkv7_chunked.hip", "wkv7_seg.hip", "wkv7_gener
            "wkv7_timemix.hip", "w6a16.hip", "wkv7_capi.hip")
 NOALLOC_SOURCE = "wkv7_noalloc.hip"
 NOALLOC_LIB_PATH = os.path.join(PKG_DIR, "librwkv7_noalloc.so")
-HEADERS = ("w6a16_grid.h", "wkv7_device.h", "wkv7_launch.h", "wkv7_token.h")
+HEADERS = ("w6a16_grid.h", "w6a16_plan.h", "wkv7_device.h", "wkv7_launch.h", "wkv7_token.h")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"

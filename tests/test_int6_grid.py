@@ -1,13 +1,15 @@
-"""The index arithmetic of the W6A16 tile kernel (rwkv-infer-next_amd/csrc/w6a16_grid.h), the very header that the kernel
-and its launch include, carried through on the CPU up to the largest sizes that a call may have: divisions by
-multiplication against divisions, and the map from workgroups to tiles against the tiles."""
+"""The host arithmetic of the W6A16 kernels (rwkv-infer-next_amd/csrc/w6a16_grid.h and w6a16_plan.h, the very headers that
+they include), carried through on the CPU up to the largest sizes that a call may have: divisions by multiplication
+against divisions, the map from workgroups to tiles against the tiles, and every call's plan against what its kernel
+assumes."""
 import os
 import shutil
 import subprocess
 
 import pytest
 
-CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "rwkv-infer-next_amd", "csrc")
+REPO = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+CSRC, INCLUDE = os.path.join(REPO, "rwkv-infer-next_amd", "csrc"), os.path.join(REPO, "include")
 
 PROGRAM = r"""
 #include <cstdio>
@@ -105,16 +107,99 @@ int main(int argc, char** argv) {
 """
 
 
-@pytest.fixture(scope="module")
-def program(tmp_path_factory):
+PLANS = r"""
+#include <cstdio>
+#include <cstdlib>
+#include "w6a16_plan.h"
+using namespace w6;
+
+static int wide_calls, far_calls, split_calls;
+
+static void check(int B, int M, int N, int K, int g, int split, int64_t stride, int64_t cus) {
+    TilePlan plan[2];
+    bool wide[2], big[2];
+    for (int packed = 0; packed < 2; ++packed) {
+        w6a16_args a{};
+        a.B = B, a.M = M, a.N = N, a.K = K, a.group_k = g, a.split_k = split, a.a_row_stride = stride;
+        a.format = packed ? W6A16_FORMAT_PACKED : W6A16_FORMAT_PLANES;
+        const Layout l = layout(&a, cus);
+        auto fail = [&](const char* what) {
+            printf("B %d M %d N %d K %d g %d split %d stride %lld packed %d: %s\n", B, M, N, K, g, split, (long long)stride, packed, what);
+            exit(1);
+        };
+        if (split > 1 && l.tiles * 4 > kCounterRegion) return;  // refused
+        big[packed] = l.big, wide[packed] = wide_call(&a, l, cus);
+        if (l.big) continue;
+        if (wide[packed]) {  // row sums in their place, ranges that 32-bit offsets reach
+            ++wide_calls;
+            if (l.total_bytes != kCounterRegion + l.partial_bytes + (size_t)B * l.nchains * l.m_groups * 64 * 4) fail("row sums");
+            if (((int64_t)(M - 1) * stride + K) * 2 >= 0x7FFFFFFF || (int64_t)K / 2 * N >= 0x7FFFFFFF) fail("2 GB");
+            if ((int64_t)K / 64 * kPackBytes >= 0x7FFFFFFF || (int64_t)l.nchains * l.m_groups * 64 * 4 >= 0x7FFFFFFF) fail("2 GB");
+        }
+        const TilePlan t = plan[packed] = tile_plan(&a, l, packed, cus);
+        const int chunks = K / 64;
+        if (t.mt < 1 || t.mt > 4 || t.cw < 1 || t.cw > 2 || (t.cw == 2 && t.mt < 3)) fail("rows");
+        if (packed ? t.nt != 1 && t.nt != 2 && t.nt != 4 : t.nt != 4 && t.nt != 8) fail("columns");
+        if (t.nt != 4 && t.mt > (packed ? 2 : 1)) fail("columns of these rows");
+        if (t.parts < 1 || t.parts > chunks || (t.ks != 1 && t.ks != 2 && t.ks != 4) || t.parts % t.ks) fail("parts");
+        if (t.ks > 1 && t.parts % 4) fail("quarters");
+        const int waves = t.cw * t.parts / t.ks;
+        const int most = t.far ? 16 : t.mt == 1 ? (t.nt == 8 ? 8 : 16) : t.mt == 2 && t.nt == 1 ? 16 : 8;
+        if (waves > most) fail("wavefronts");
+        if (64 * waves < 16 * t.nt * t.cw) fail("fewer threads than columns");
+        if (t.far && (t.mt != 1 || t.nt != 4 || t.cw != 1)) fail("far");
+        if (!t.far && ((M > 1 ? stride : K) >= (1 << 24) || (!packed && N >= (1 << 26)))) fail("not far");
+        far_calls += t.far, split_calls += t.ks > 1;
+        if (t.ks > 1) {  // counters and partial tiles inside the workspace
+            const int64_t tiles = (int64_t)B * ((M + 16 * t.mt - 1) / (16 * t.mt)) * ((N / 16 + t.nt * t.cw - 1) / (t.nt * t.cw));
+            if (tiles * 4 > (int64_t)kCounterRegion) fail("counters");
+            if ((size_t)tiles * t.ks * 16 * t.mt * 16 * t.nt * t.cw * 4 > l.partial_bytes) fail("partial tiles");
+        }
+    }
+    if (big[1]) return;  // (the planes have no such kernel)
+    if (wide[0] != wide[1] || plan[0].parts != plan[1].parts) {
+        printf("B %d M %d N %d K %d split %d: planes and packed differ\n", B, M, N, K, split);
+        exit(1);
+    }
+}
+
+int main() {
+    const int Ms[] = {1, 2, 8, 9, 15, 16, 17, 31, 32, 33, 40, 48, 49, 64, 65, 96, 97, 128, 129, 144, 145, 160, 192, 193, 203, 256, 257, 300, 1000, 4097, 100000};
+    const int Ns[] = {16, 32, 64, 80, 128, 144, 256, 768, 1024, 1088, 2048, 2560, 2752, 4096, 4112, 5120, 8192, 10240, 16336, 16384, 16400, 22528, 32768,
+                      32784, 65536, 1 << 22, (1 << 26) - 16, 1 << 26, (1 << 30) + 80, 2147483632};
+    const int Ks[] = {64, 128, 192, 256, 320, 512, 576, 768, 1024, 1088, 2048, 2560, 3072, 4096, 8192, 8256, 10240, 16320, 16384, 65536, 1 << 24};
+    const int splits[] = {1, 2, 3, 4, 8, 9, 16, 32, 64, 256};
+    for (int M : Ms)
+        for (int N : Ns)
+            for (int K : Ks)
+                for (int split : splits)
+                    for (int B : {1, 2, 7})
+                        for (int g : {64, 128})
+                            for (int64_t cus : {256, 304, 64}) {
+                                if (K % g) continue;
+                                check(B, M, N, K, g, split, K, cus);
+                                if (B == 1 && g == 64 && K < (1 << 24)) check(B, M, N, K, g, split, 1 << 24, cus);
+                            }
+    if (!wide_calls || !far_calls || !split_calls) { printf("a form that no call took\n"); return 1; }
+    printf("fine\n");
+}
+"""
+
+
+def _compiled(tmp_path_factory, name, text):
     cxx = shutil.which("g++") or shutil.which("amdclang++") or shutil.which("clang++")
     if cxx is None:
         pytest.skip("no C++ compiler")
-    d = tmp_path_factory.mktemp("grid")
-    (d / "grid.cpp").write_text(PROGRAM)
-    subprocess.run([cxx, "-std=c++17", "-O2", "-Wall", "-Werror", f"-I{CSRC}", "-o", str(d / "grid"), str(d / "grid.cpp")],
+    d = tmp_path_factory.mktemp(name)
+    (d / "p.cpp").write_text(text)
+    subprocess.run([cxx, "-std=c++17", "-O2", "-Wall", "-Werror", f"-I{CSRC}", f"-I{INCLUDE}", "-o", str(d / "p"), str(d / "p.cpp")],
                    check=True)
-    return str(d / "grid")
+    return str(d / "p")
+
+
+@pytest.fixture(scope="module")
+def program(tmp_path_factory):
+    return _compiled(tmp_path_factory, "grid", PROGRAM)
 
 
 def _run(program, what):
@@ -128,3 +213,7 @@ def test_divisions_are_exact_below_2_to_the_31(program):
 
 def test_every_tile_has_one_workgroup(program):
     _run(program, "grids")
+
+
+def test_every_call_has_a_plan_that_its_kernel_takes(tmp_path_factory):
+    _run(_compiled(tmp_path_factory, "plan", PLANS), "")

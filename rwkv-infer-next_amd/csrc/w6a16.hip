@@ -206,11 +206,12 @@ __device__ __forceinline__ f4 fma4(const f4 x, float s, const f4 a) {
 // drift apart and their loads, LDS turns and MFMAs overlap.
 // Measured against the kernels it replaced (a strip-wide split-K kernel with a release fence per workgroup up to 32
 // rows, above them a kernel of 128-column workgroups in lock-step with a row-sum pass before it), us per call, packed /
-// planes: K = N = 4096, M = 1 11.5 / 11.6 -> 6.7 / 8.6, M = 16 26.1 / 26.1 -> 8.3 / 10.6, M = 64 17.6 / 18.4 ->
-// 10.7 / 15.5; K = 4096, N = 16384, M = 64 27.5 / 29.7 -> 24.3 / 27.9; K = 2560, N = 10240, M = 203 52 / 62 -> 36.6 / 42.6;
-// K = 10240, N = 2560, M = 203 57 / 67 -> 28.2 / 34.6; a layer's six products at C = 4096: M = 1 planes 83.7 -> 71.3,
-// M = 64 packed 130 -> 95; at C = 2560, M = 203 planes 281 -> 132.  Slower only where 193..256 rows meet K = 4096 and
-// N = 16384 (52 / 67 -> 63 / 71), and one row of packed weights there (11.9 -> 12.4): the rest of the layer gains more.
+// planes: K = N = 4096, M = 1 11.5 / 11.6 -> 7.0 / 8.6, M = 16 26.1 / 26.1 -> 8.6 / 10.0, M = 64 17.6 / 18.4 -> 10.8 / 13.9; K =
+// 4096, N = 16384, M = 1 12.5 / 17.0 -> 12.6 / 16.9, M = 64 27.0 / 29.9 -> 23.0 / 26.1; K = 2560, N = 10240, M = 203 52 / 62 -> 36
+// / 41; K = 10240, N = 2560, M = 203 57 / 67 -> 28 / 34.  Where the old ones stayed ahead: wide_call (w6a16_plan.h), and 0.2 us
+// of 4.5 at K = 512, N = 16384, 8 and 16 rows packed.
+// Counters at K = 4096, N = 16384 (packed / planes): M = 1 MfmaUtil 5 / 4 %, VALUBusy 16 / 17 %; M = 64 16 / 14 and 23 / 23; M =
+// 128 24 / 21 and 34 / 35, LDS under 13 %: no unit is near its limit; the wavefronts wait for loads.
 
 // The weights of one chunk in one lane's registers.  Packed: the lane's record of its NT tiles (tile t: column
 // n0 + 16 t + i); one tile takes the 8-byte pair its top bits lie in.
@@ -804,23 +805,28 @@ struct WideLds {
 };
 
 // Buffer bases and sizes (wave-uniform) and per-lane offsets of the loads, fixed for the call; the chunk goes into the
-// instructions' scalar offset.  Every range is below 2 GB (wide_call).
+// instructions' scalar offset.  Every range is below 2 GB (wide_call; of A the workgroup's 64 rows, which at row strides of
+// 2^24 elements and more, FAR, have 64-bit addresses instead).
 struct WideSrc {
-    uint64_t a, rs, lo, hi, sc;
+    uint64_t a, rs, lo, hi, sc, fa[2];
     int64_t na, nrs, nlo, nhi, nsc;
     uint32_t va[2], vrs, vlo, vhi, vsc;
 };
 
-template <bool PACKED>
+template <bool PACKED, bool FAR>
 __device__ __forceinline__ WideSrc wide_src(const Args& p, int b, int m0, int strip) {
     const int t = threadIdx.x, lane = t & 63, i = lane & 15, cp = t >> 6, n0 = strip * kTileN;
     WideSrc x;
-    x.a = reinterpret_cast<uint64_t>(p.a + (int64_t)b * p.sa_b);
-    x.na = ((int64_t)(p.M - 1) * p.sa_m + p.K) * 2;
+    const uint16_t* const a = p.a + (int64_t)b * p.sa_b + (int64_t)m0 * p.sa_m;
+    x.a = reinterpret_cast<uint64_t>(a);
+    const int last = min(p.M - m0, kWideRows) - 1;  // of the workgroup's rows; those past it take it again
+    x.na = ((int64_t)last * p.sa_m + p.K) * 2;
 #pragma unroll
     for (int e = 0; e < 2; ++e) {
         const int piece = t + 256 * e;
-        x.va[e] = (uint32_t)((min(m0 + (piece >> 3), p.M - 1) * p.sa_m + 8 * (piece & 7)) * 2);
+        const int64_t off = (min(piece >> 3, last) * p.sa_m + 8 * (piece & 7)) * 2;
+        if constexpr (FAR) x.fa[e] = x.a + (uint64_t)off;
+        else x.va[e] = (uint32_t)off;
     }
     x.rs = reinterpret_cast<uint64_t>(p.rsum + (int64_t)b * p.nchains * p.mpad);
     x.nrs = (int64_t)p.nchains * p.mpad * 4;
@@ -849,11 +855,15 @@ __device__ __forceinline__ WideSrc wide_src(const Args& p, int b, int m0, int st
     return x;
 }
 
-template <int CG, bool PACKED>
+template <int CG, bool PACKED, bool FAR>
 __device__ __forceinline__ void wide_load_lds(const Args& p, const WideSrc& src, int c, WideLds& x) {
 #pragma unroll
-    for (int e = 0; e < 2; ++e)
-        x.a[e] = __builtin_amdgcn_raw_buffer_load_b128(rsrc(src.a, src.na), src.va[e], soff(c * 128), 0);
+    for (int e = 0; e < 2; ++e) {
+        if constexpr (FAR)
+            x.a[e] = *reinterpret_cast<const __attribute__((address_space(1))) u4*>(src.fa[e] + (uint64_t)c * 128);
+        else
+            x.a[e] = __builtin_amdgcn_raw_buffer_load_b128(rsrc(src.a, src.na), src.va[e], soff(c * 128), 0);
+    }
     x.rs = __builtin_amdgcn_raw_buffer_load_b128(rsrc(src.rs, src.nrs), src.vrs, soff((c / CG) * p.mpad * 4), 0);
     if constexpr (!PACKED) {
         x.pl[0] = __builtin_amdgcn_raw_buffer_load_b128(rsrc(src.lo, src.nlo), src.vlo, soff(c * 32 * p.N), 0);
@@ -1003,7 +1013,7 @@ __device__ __forceinline__ void wide_store(const Args& p, int b, int m0, int n0,
         }
 }
 
-template <class A, int CG, bool PACKED>
+template <class A, int CG, bool PACKED, bool FAR>
 __global__ __launch_bounds__(256, 2) void w6a16_wide_kernel(const Args p) {
     constexpr int kStage = wide_stage<PACKED>(), D = 4;  // loads D steps ahead
     static_assert(D % CG == 0 && D % 2 == 0, "a group of D steps holds whole chains and buffer pairs");
@@ -1012,7 +1022,7 @@ __global__ __launch_bounds__(256, 2) void w6a16_wide_kernel(const Args p) {
     const int strip = (int)pos.column, n0 = strip * kTileN, m0 = (int)pos.mg * kWideRows, b = blockIdx.z;
     if (strip >= p.n_strips) return;  // uniform over the workgroup
     const int steps = p.K / 64;
-    const WideSrc src = wide_src<PACKED>(p, b, m0, strip);
+    const WideSrc src = wide_src<PACKED, FAR>(p, b, m0, strip);
     f4 acc[kWideMT][2], tc[kWideMT][2];
 #pragma unroll
     for (int mt = 0; mt < kWideMT; ++mt) acc[mt][0] = acc[mt][1] = f4{0.f, 0.f, 0.f, 0.f};
@@ -1024,13 +1034,13 @@ __global__ __launch_bounds__(256, 2) void w6a16_wide_kernel(const Args p) {
     WideW ws[D];
     auto chunk = [&](int s) __attribute__((always_inline)) { return min(s, steps - 1); };
 #pragma unroll
-    for (int j = 0; j < D; ++j) wide_load_lds<CG, PACKED>(p, src, chunk(j), ls[j]);
+    for (int j = 0; j < D; ++j) wide_load_lds<CG, PACKED, FAR>(p, src, chunk(j), ls[j]);
     if constexpr (PACKED) {
 #pragma unroll
         for (int j = 0; j < D; ++j) wide_load_w(p, src, chunk(j), ws[j]);
     }
     wide_store_lds<PACKED>(ls[0], lds);
-    wide_load_lds<CG, PACKED>(p, src, chunk(D), ls[0]);
+    wide_load_lds<CG, PACKED, FAR>(p, src, chunk(D), ls[0]);
     __builtin_amdgcn_sched_barrier(0);
     __syncthreads();
     auto step = [&](int base, auto J) __attribute__((always_inline)) {
@@ -1041,7 +1051,7 @@ __global__ __launch_bounds__(256, 2) void w6a16_wide_kernel(const Args p) {
             wide_compute<A, PACKED, j % CG == 0, j % CG == CG - 1>(lds + (j & 1) * kStage, ws[j], tc, acc);
         if constexpr (PACKED) wide_load_w(p, src, chunk(base + j + D), ws[j]);
         wide_store_lds<PACKED>(ls[(j + 1) % D], lds + ((j + 1) & 1) * kStage);
-        wide_load_lds<CG, PACKED>(p, src, chunk(base + j + 1 + D), ls[(j + 1) % D]);
+        wide_load_lds<CG, PACKED, FAR>(p, src, chunk(base + j + 1 + D), ls[(j + 1) % D]);
         __builtin_amdgcn_sched_barrier(0);
         __syncthreads();
     };
@@ -1608,10 +1618,13 @@ int launch_wide(Args& p, const w6a16_args* a, const Layout& l, hipStream_t s) {
     p.mpad = l.m_groups * kWideRows;
     p.rsum = reinterpret_cast<float*>(static_cast<char*>(a->workspace) + kCounterRegion + l.partial_bytes);
     hipLaunchKernelGGL(w6a16_rowsum_kernel<A>, dim3(p.mpad / 4, (p.K + 511) / 512, p.B), dim3(256), 0, s, p);
-    if (p.chain_k == 128)
-        hipLaunchKernelGGL((w6a16_wide_kernel<A, 2, PACKED>), dim3((unsigned)wgs, 1, p.B), dim3(256), 0, s, p);
-    else
-        hipLaunchKernelGGL((w6a16_wide_kernel<A, 1, PACKED>), dim3((unsigned)wgs, 1, p.B), dim3(256), 0, s, p);
+    auto run = [&](auto two, auto far) {
+        hipLaunchKernelGGL((w6a16_wide_kernel<A, decltype(two)::value ? 2 : 1, PACKED, decltype(far)::value>),
+                           dim3((unsigned)wgs, 1, p.B), dim3(256), 0, s, p);
+    };
+    const bool two = p.chain_k == 128, far = p.sa_m >= (1 << 24);
+    if (two) far ? run(std::true_type{}, std::true_type{}) : run(std::true_type{}, std::false_type{});
+    else far ? run(std::false_type{}, std::true_type{}) : run(std::false_type{}, std::false_type{});
     return WKV7_OK;
 }
 

@@ -110,7 +110,12 @@ inline TilePlan tile_plan(const w6a16_args* a, const Layout& l, bool packed, int
         while (most > 1 && (size_t)wgs(mt, 4 * cw) * most * 16 * mt * 64 * cw * 4 > l.partial_bytes) most >>= 1;
         return most;
     };
-    // Workgroups of `wide` K parts for whose parts a deep K has work where CUs would be left without.
+    // Workgroups of `wide` K parts, where CUs would be left without work.  Up to 128 chunks one workgroup's parts are short
+    // already (us, packed / planes: K = N = 4096, M = 1, 16 / 32 parts 6.9 / 8.2 and 8.4 / 9.0), but for two row tiles on a
+    // quarter of the CUs, whose planes gain (K = 8192, N = 2048, M = 20, 8 / 16 parts 13.6 / 13.7 and 19.1 / 13.5; K = N = 2560
+    // 6.0 / 6.3 and 9.8 / 9.9).  Deeper K pays (K = 16384, N = 4096, M = 20, 8 / 16 / 32 parts 25.3 / 25.2 / 17.5 and 33.0 / 22.1
+    // / 21.9); one row tile has 16 parts to begin with and takes twice as many, no more (M = 1, 16 / 32 / 64 parts 16.5 / 14.0
+    // / 14.1 and 17.4 / 17.7 / 17.3).
     auto spread = [&](int mt, int cw, int wide) {
         const int64_t w4 = wgs(mt, 4 * cw), most = room(mt, cw);
         int s = 1;
@@ -204,14 +209,13 @@ inline TilePlan tile_plan(const w6a16_args* a, const Layout& l, bool packed, int
 // tile against wide: M = 144 83.4 / 70.8 against 95.3 / 78.9, 145 88.9 / 79.5 against 89.6 / 79.2, 176 92.3 / 83.0 against 93.5
 // / 77.1), eight chunks (with four as fast), two tiles and more to a CU, of which the last two rounds fill a quarter (K =
 // 4096, M = 193, tile against wide: N = 16384 59.2 / 55.3 against 56.7 / 48.0, 17408 78.0 / 65.6 against 87.9 / 73.0, 20480
-// 88.2 / 77.0 against 88.7 / 73.7), and every range that a buffer covers below 2 GB.
+// 88.2 / 77.0 against 88.7 / 73.7), and planes and scales that a buffer covers (below 2 GB).
 inline bool wide_call(const w6a16_args* a, const Layout& l, int64_t cus) {
     if (l.big || a->M <= 144 || a->M > 256 || a->K < 512) return false;
     const int64_t tiles = (int64_t)a->B * l.m_groups * l.n_strips, twice = 2 * cus, last = tiles % twice;
     if (tiles < twice || (last > 0 && 4 * last < twice)) return false;
     const int64_t limit = 0x7FFFFFFF;
-    return ((int64_t)(a->M - 1) * a->a_row_stride + a->K) * 2 < limit && (int64_t)(a->K / 2) * a->N < limit &&
-           (int64_t)(a->K / a->group_k) * a->N * 2 < limit;
+    return (int64_t)(a->K / 2) * a->N < limit && (int64_t)(a->K / a->group_k) * a->N * 2 < limit;
 }
 
 }  // namespace w6

@@ -19,9 +19,9 @@
 // wavefront stays on one head group and strides over tokens, so the per-channel parameters are loaded once into
 // registers; the per-head sums are 8-lane butterflies.  All arithmetic is fp32 with one bf16 rounding per output
 // (the reference rounds after every torch op).  Decode-sized launches are bound by latency: with the work split, the
-// look-ahead and the sums below in their present form, 12 layers of one token with H = 12 (prologue, recurrence and
-// epilogue in one graph) went from 101 to 94 us, 8 layers of 23 tokens with H = 40 from 125 to 117, 4 of 64 with
-// H = 64 from 135.4 to 132.6; T = 4096, H = 64 from 107.6 to 106.3 (5.4 TB/s).
+// look-ahead and the sums below in their present form (measured together), 12 layers of one token with H = 12 (prologue,
+// recurrence and epilogue in one graph) went from 101 to 94 us, 8 layers of 23 tokens with H = 40 from 125 to 117; 4 of 64
+// with H = 64 and T = 4096, H = 64 (106.3 us, 5.4 TB/s) changed by no more than a run differs from the next.
 #include <stdint.h>
 
 #include <algorithm>
@@ -86,7 +86,8 @@ __device__ __forceinline__ float softplus(float x) {
 // longer than its arithmetic).
 struct Split {
     int groups;        // head groups of a token
-    uint32_t inv;      // gw / groups = gw inv >> 32
+    uint32_t inv;      // gw / groups = gw inv >> 32: exact while gw groups < 2^32 (groups <= 8192 by the entry points'
+                       // bound on H, gw at most that or 32 wavefronts a CU)
     int per;           // tokens under way at a time
 };
 

@@ -86,24 +86,26 @@ def test_wide_kernel(B, M, N, K, g, split, dtype):
     _check(C, a, lo, hi, sc, g, KERNEL_TOL if dtype == "bf16" else F16_KERNEL_TOL)
 
 
-@pytest.mark.parametrize("B,M,N,K,g,split", [
-    (2, 3, 80, 256, 64, None),      # one row tile, as many parts as chunks
-    (1, 40, 144, 2048, 128, None),  # eight parts, where 16 rows would have 16
-    (1, 3, 64, 16384, 128, 32),     # 32 parts over two workgroups
-    (1, 17, 80, 16384, 128, 32),    # two row tiles, 32 parts
+@pytest.mark.parametrize("B,M,N,K,g,split,stride", [
+    (2, 3, 80, 256, 64, None, 1 << 24),      # one row tile, as many parts as chunks
+    (1, 40, 144, 2048, 128, None, 1 << 24),  # two row tiles
+    (1, 3, 64, 16384, 128, 32, 1 << 24),     # 32 parts over two workgroups
+    (1, 17, 80, 16384, 128, 32, 1 << 24),    # two row tiles, 32 parts
+    (1, 193, 16384, 512, 128, None, 1 << 24),  # the wide kernel
+    (1, 200, 16384, 576, 64, None, 1 << 23),   # the wide kernel, rows that span 2 GB in groups that do not
 ])
-def test_rows_far_apart(B, M, N, K, g, split):
-    """A row stride of 2^24 elements: a workgroup's rows span more than its buffer's 32-bit offsets reach.  The same bits
+def test_rows_far_apart(B, M, N, K, g, split, stride):
+    """Row strides of 2^24 elements: a workgroup's rows span more than its buffer's 32-bit offsets reach.  The same bits
     as the same rows side by side."""
     from rwkv_next_amd.kernels import int6_gemm as I6
-    say("w6a16 rows far apart", dict(B=B, M=M, N=N, K=K))
+    say("w6a16 rows far apart", dict(B=B, M=M, N=N, K=K, stride=stride))
     rng = np.random.default_rng(11 + M)
     lo, hi, sc = _weights(rng, B, K, N, g)
     a = _act(rng, B, M, K)
     Ld, Hd, Sd = _dev(lo, hi, sc)
-    far = torch.zeros(B * M, 1 << 24, dtype=torch.bfloat16, device=DEV)
+    far = torch.zeros(B * M, stride, dtype=torch.bfloat16, device=DEV)
     far[:, :K] = a.reshape(B * M, K).to(DEV)
-    view = far.view(B, M, 1 << 24)[:, :, :K]
+    view = far.view(B, M, stride)[:, :, :K]
     pk = I6.prepack_int6(Ld, Hd, Sd, g)
     split = _split(split, B, M, N, K)
     C = I6.int6_matmul(view, Ld, Hd, Sd, g, split_k=split, out_dtype=torch.float32)

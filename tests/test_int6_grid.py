@@ -133,7 +133,7 @@ static void check(int B, int M, int N, int K, int g, int split, int64_t stride, 
         if (wide[packed]) {  // row sums in their place, ranges that 32-bit offsets reach
             ++wide_calls;
             if (l.total_bytes != kCounterRegion + l.partial_bytes + (size_t)B * l.nchains * l.m_groups * 64 * 4) fail("row sums");
-            if (((int64_t)(M - 1) * stride + K) * 2 >= 0x7FFFFFFF || (int64_t)K / 2 * N >= 0x7FFFFFFF) fail("2 GB");
+            if ((int64_t)K / 2 * N >= 0x7FFFFFFF || (int64_t)K / g * N * 2 >= 0x7FFFFFFF) fail("2 GB");
             if ((int64_t)K / 64 * kPackBytes >= 0x7FFFFFFF || (int64_t)l.nchains * l.m_groups * 64 * 4 >= 0x7FFFFFFF) fail("2 GB");
         }
         const TilePlan t = plan[packed] = tile_plan(&a, l, packed, cus);

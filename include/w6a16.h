@@ -66,27 +66,30 @@ size_t w6a16_args_size(void);
  * B * ceil(M / 16) * ceil(N / 128) reaches the device's CU count; otherwise a fixed 1 MiB region of u32 arrival counters
  * (a call whose B * ceil(M / rows) * ceil(N / 128), rows 16 up to M = 32, 32 up to 64, 64 above, exceeds 262144 with
  * split_k > 1 is refused with WKV7_ERR_SHAPE), then room for split_k fp32 partial tiles (split_k > 1), then, for M > 32, a
- * float per row and chain of two 64-row chunks.  The kernel uses the counters and as many partial tiles as it splits K
- * over workgroups, the workgroup that completes a tile last sums it.  Contract: the counter region (the first 1 MiB)
- * must be zero before the workspace's first use; every completed call leaves it zero again and never writes partials
- * into it, so one workspace serves any number of calls of any shapes issued one after another (stream order).  Calls
- * that can run at the same time (different streams) need different workspaces. */
+ * float per row and chain of two 64-row chunks (of one where group_k holds one).  A call uses of it what its kernel needs:
+ * counters and up to four partial tiles where it splits K over workgroups (the workgroup that completes a tile last sums
+ * it), or row sums of A (145..256 rows of many columns).  Contract: the counter region (the first 1 MiB) must be zero
+ * before the workspace's first use; every completed call leaves it zero again and writes nothing else into it, so one
+ * workspace serves any number of calls of any shapes issued one after another (stream order).  Calls that can run at the
+ * same time (different streams) need different workspaces. */
 int w6a16_workspace_size(const w6a16_args *args, size_t *bytes);
 
-/* Split-K for a shape: the smallest power of two (<= 64, every range keeping at least one 64-row chunk) that gives
- * every CU at least one workgroup, then doubled while ranges keep at least sixteen 64-row chunks and the launch stays
- * within two workgroups per CU.  Replaces the split-K rule of plan_int6 (rwkv_next/kernels/int6_gemm.py:239-250). */
+/* split_k for a shape: a power of two (<= 64, every range keeping at least one 64-row chunk) that grows with the CUs the
+ * shape would leave without work, then doubled while ranges keep at least sixteen.  It sizes the workspace and so bounds
+ * over how many workgroups the kernel may split K; in how many parts K is shared is the kernel's own choice.  Replaces the
+ * split-K rule of plan_int6 (rwkv_next/kernels/int6_gemm.py:239-250). */
 int w6a16_plan_split(int32_t B, int32_t M, int32_t N, int32_t K);
 
 /* split_k for the packed layout (W6A16_FORMAT_PACKED): 4 instead of 8 where B * ceil(M / 16) * ceil(N / 128) stays below
- * the CU count and a range keeps 8 chunks; otherwise equal to w6a16_plan_split.  No counterpart in the reference (its
- * weights come only as planes); for callers that pass packed weights.  Results may depend on split_k: a packed call is
- * sure to give the planes' bits only at the same split_k. */
+ * the CU count and a range keeps 8 chunks; otherwise equal to w6a16_plan_split.  (Up to 32 rows both bound the kernel to
+ * one workgroup a tile.)  No counterpart in the reference, whose weights come only as planes.  Results may depend on
+ * split_k: a packed call is sure to give the planes' bits only at the same split_k. */
 int w6a16_plan_split_packed(int32_t B, int32_t M, int32_t N, int32_t K);
 
 /* C = A @ dequant(W) on `stream` (hipStream_t).  Replaces `_impl` + `_w6a16` (int6_gemm.py:253-287, 156-215).
- * The summation order (which wavefronts share K, and in how many parts) follows from B, M, N, K and split_k, the same for
- * both formats; equal calls give equal bits.
+ * The summation order (which kernel runs, which wavefronts share K, and in how many parts) follows from B, M, N, K,
+ * group_k and split_k and the device's CU count; up to M = 256 it is the same for both formats and whatever the strides,
+ * and equal calls give equal bits.
  * W6A16_FORMAT_PACKED with M > 256 runs the large-M kernel: A times the weight dequantised to A's type (s q rounded
  * once, the values w6a16_dequantize writes), fp32 accumulation, no workspace; split_k is not used there. */
 int w6a16_matmul(const w6a16_args *args, void *stream);

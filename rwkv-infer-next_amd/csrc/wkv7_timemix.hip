@@ -20,8 +20,9 @@
 // registers; the per-head sums are 8-lane butterflies.  All arithmetic is fp32 with one bf16 rounding per output
 // (the reference rounds after every torch op).  Decode-sized launches are bound by latency: with the work split, the
 // look-ahead and the sums below in their present form (measured together), 12 layers of one token with H = 12 (prologue,
-// recurrence and epilogue in one graph) went from 101 to 94 us, 8 layers of 23 tokens with H = 40 from 125 to 117; 4 of 64
-// with H = 64 and T = 4096, H = 64 (106.3 us, 5.4 TB/s) changed by no more than a run differs from the next.
+// recurrence and epilogue in one graph) went from 101.6 to 94.0 us, 8 layers of 23 tokens with H = 40 from 126.0 to 116.6, 4
+// of 64 with H = 64 from 135.8 to 132.6 (two runs of one side differ by up to 1.1, 0.3 and 0.6 %); T = 4096, H = 64 from 108.0
+// to 106.9 (5.4 TB/s), no more than the 1.2 % that its runs differ.
 #include <stdint.h>
 
 #include <algorithm>

@@ -18,11 +18,12 @@ fp16 scale, w ~ s q; the code u = q + 32 is split into bit planes per 64-row chu
     lo[c*32 + j] = lo4(row j) | lo4(row j + 32) << 4                                        j < 32
     hi[c*16 + j] = hi2(row j) | hi2(row j + 16) << 2 | hi2(row j + 32) << 4 | hi2(row j + 48) << 6   j < 16
 
-Compute: one MFMA kernel for every M up to MAX_M (the reference's reduction form for M = 1 has no counterpart:
+Compute: MFMA kernels for every M up to MAX_M (the reference's reduction form for M = 1 has no counterpart:
 an MFMA with M padded to 16 rows costs the CDNA4 matrix core less than a VALU reduction costs the vector units, and
 the weight bytes, not the arithmetic, bound both).  `use_dot` is accepted for the reference's signature and does
-not change the computation; `split_k` bounds over how many workgroups the kernel may split K.  Above MAX_M the weight is dequantised once to the activations' type and the product
-goes to the library GEMM (hipBLASLt through torch.matmul), which is compute-bound there.  The C ABI has its own kernel
+not change the computation; `split_k` bounds over how many workgroups the kernel may split K.  Above MAX_M the weight
+is dequantised once to the activations' type and the product goes to the library GEMM (hipBLASLt through torch.matmul),
+which is compute-bound there.  The C ABI has its own kernel
 for that range (packed weights, M > 256: dequantisation in LDS fused with the product, the same values); at K = 4096,
 N = 16384 it is level with dequantise + hipBLASLt at M = 1024 and slower from M = 2048 (585 against 465 us at
 M = 4096), so MAX_M (env RWKV_INT6_MAX_M) keeps the library GEMM by default.
@@ -295,7 +296,7 @@ def _impl(a, w: _W, split_k, out_dtype=None):
     lib = _lib.load()
     n = ctypes.c_size_t(0)
     _lib.check(lib.w6a16_workspace_size(args, ctypes.byref(n)))
-    if n.value:  # counters and partial tiles of a K split over workgroups
+    if n.value:  # counters and partial tiles of a K split over workgroups, row sums of A
         ws = _workspace(A.device, int(n.value))
         args.workspace, args.workspace_bytes = ws.data_ptr(), ws.numel()
     _lib.check(lib.w6a16_matmul(args, stream_handle(A.device)))
@@ -307,8 +308,8 @@ _WORKSPACES: dict = {}     # (device index, stream handle) -> [buffer, counters 
 
 
 def _workspace(device, nbytes):
-    """The workspace (a fixed counter region, then split-K partials and row sums) of the current stream on `device`;
-    see `_workspace.stream_workspace`."""
+    """The workspace (a fixed counter region, then room for partial tiles and row sums, include/w6a16.h) of the current
+    stream on `device`; see `_workspace.stream_workspace`."""
     return stream_workspace(_WORKSPACES, device, nbytes, _COUNTER_BYTES)
 
 

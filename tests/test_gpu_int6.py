@@ -107,8 +107,8 @@ def test_matmul_matches_oracle(B, M, N, K, g, split):
     (1, 96, 1024, 2048, 128, True, 3),      # split-K with uneven ranges of chains
 ])
 def test_wide_kernel_matches_oracle(B, M, N, K, g, shared, split):
-    """M > 32 runs the wide kernel (row-sum pre-pass, K parts, chains per quantisation group); planes and packed give
-    the same bits."""
+    """M > 32: several row tiles to a workgroup, K shared by parts and, with a split, by workgroups; planes and packed
+    give the same bits."""
     from rwkv_next_amd.kernels import int6_gemm as I6
     say("int6_matmul wide kernel", dict(B=B, M=M, N=N, K=K, g=g, shared=shared, split=split))
     rng = np.random.default_rng(300 + M + N + K)

@@ -159,9 +159,9 @@ def test_random_shapes_match_oracle(seed):
 
 @pytest.mark.parametrize("split", [2, 4, 8, 16])
 def test_in_workgroup_split_on_planes(split):
-    """B x ceil(M / 16) x N / 128 = 4 x 2 x 32 = 256 workgroups fill the chip, so split 2..8 runs the in-workgroup
-    split-K kernel on the planes as well as on the packed layout (split 16: the cross-workgroup hand-off on both);
-    the two layouts give the same bits, within KERNEL_TOL of the oracle."""
+    """B x ceil(M / 16) x N / 128 = 4 x 2 x 32 = 256 tiles, as many as CUs: split 2..8 has no workspace on the planes as
+    well as on the packed layout, so K's parts share a workgroup (split 16: a workspace on both); the two layouts give
+    the same bits, within KERNEL_TOL of the oracle."""
     from rwkv_next_amd.kernels import int6_gemm as I6
     B, M, N, K, g = 4, 20, 4096, 1024, 128
     say("int6_matmul in-workgroup split", dict(B=B, M=M, N=N, K=K, split=split))
@@ -178,9 +178,8 @@ def test_in_workgroup_split_on_planes(split):
 
 @pytest.mark.parametrize("N,M,split", [(80, 1, 4), (80, 17, 3), (208, 5, 2), (16, 32, 4), (208, 2, 8)])
 def test_half_strips_ragged_n(N, M, split):
-    """Packed layout, few strips: each workgroup takes half a 128-column strip (three chunks in flight at split <= 4,
-    two at 8), so at N = 80 the second half (columns 64..127) holds 16 valid columns, at N = 16 none; split 3 leaves
-    uneven ranges; planes (the cross-workgroup kernel) give the same bits."""
+    """Few strips, N past the last full one: workgroups of 64 columns and less, at N = 80 the second half of the strip
+    (columns 64..127) holds 16 valid columns, at N = 16 none; planes and packed give the same bits."""
     from rwkv_next_amd.kernels import int6_gemm as I6
     K, g = 768, 64
     say("int6_matmul half strips", dict(M=M, N=N, K=K, split=split))
@@ -197,8 +196,8 @@ def test_half_strips_ragged_n(N, M, split):
 
 @pytest.mark.parametrize("shared,split", [(False, 3), (True, 4), (False, 8)])
 def test_half_strips_batched(shared, split):
-    """Half strips over a batch (grid z = batch x M groups; per-batch or shared packed weights and scales): same bits
-    as the planes, within KERNEL_TOL of the oracle."""
+    """Parts of strips over a batch (per-batch or shared packed weights and scales): same bits as the planes, within
+    KERNEL_TOL of the oracle."""
     from rwkv_next_amd.kernels import int6_gemm as I6
     B, M, N, K, g = 3, 21, 208, 768, 64
     say("int6_matmul half strips batched", dict(B=B, M=M, N=N, K=K, shared=shared, split=split))
@@ -273,11 +272,11 @@ def test_split_k_is_deterministic_and_consistent():
 
 @pytest.mark.parametrize("B,M,N,K,g,split,packed", [
     (1, 1, 4096, 4096, 128, None, False),   # GEMV, split-K across workgroups or in the workgroup
-    (1, 1, 4096, 4096, 128, None, True),    # packed: half strips
-    (1, 5, 144, 256, 256, 3, False),        # narrow kernel, uneven split ranges, N past the last full strip
+    (1, 1, 4096, 4096, 128, None, True),    # packed
+    (1, 5, 144, 256, 256, 3, False),        # four chunks, N past the last full strip
     (1, 16, 2048, 1024, 64, None, True),
-    (2, 48, 272, 512, 128, None, False),    # wide kernel (row-sum pre-pass), batched weights
-    (1, 150, 640, 1024, 256, 2, True),      # wide kernel, split-K
+    (2, 48, 272, 512, 128, None, False),    # several row tiles, batched weights
+    (1, 150, 640, 1024, 256, 2, True),      # several row tiles, packed, a split
 ])
 def test_fp16_activations(B, M, N, K, g, split, packed):
     """fp16 activations, as the reference takes them (its dot casts the codes to a.dtype, int6_gemm.py:144-147): the

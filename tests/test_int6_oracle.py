@@ -266,26 +266,25 @@ def test_matmul_empty_and_workspace_size():
     # 16 x 128 fp32 partial tile
     tiles = 2 * 1 * 2
     assert n.value == (1 << 20) + tiles * 8 * 16 * 128 * 4
-    # M > 32 runs the wide kernel: after the counters and partials, the row sums of A per chain of two 64-row chunks
-    # (group_k = 128), [B][K / 128][rows padded to the M groups]
-    # M = 40: two 16-row tiles per wavefront, two M groups of 32 rows, two strips (N = 256): four tiles
+    # M > 32: after the counters and partials, room for row sums of A per chain of two 64-row chunks (group_k = 128),
+    # [B][K / 128][rows padded to the M groups]
+    # M = 40: two M groups of 32 rows, two strips (N = 256): four tiles
     assert lib.w6a16_workspace_size(ctypes.byref(base_args(split_k=2, M=40)), ctypes.byref(n)) == 0
     assert n.value == (1 << 20) + 4 * 2 * 32 * 128 * 4 + 4 * 64 * 4
-    # M = 100: four 16-row tiles per wavefront, two M groups of 64 rows, two strips
+    # M = 100: two M groups of 64 rows, two strips
     assert lib.w6a16_workspace_size(ctypes.byref(base_args(split_k=2, M=100)), ctypes.byref(n)) == 0
     assert n.value == (1 << 20) + 4 * 2 * 64 * 128 * 4 + 4 * 128 * 4
     # M = 200: four M groups of 64 rows
     assert lib.w6a16_workspace_size(ctypes.byref(base_args(split_k=2, M=200)), ctypes.byref(n)) == 0
     assert n.value == (1 << 20) + 8 * 2 * 64 * 128 * 4 + 4 * 256 * 4
-    # without split-K the wide kernel still needs the counter region's place and the row sums
+    # without a split, still the counter region's place and the row sums
     assert lib.w6a16_workspace_size(ctypes.byref(base_args(M=40)), ctypes.byref(n)) == 0
     assert n.value == (1 << 20) + 4 * 64 * 4
     wide = base_args(M=40, a_batch_stride=40 * 512, out_batch_stride=40 * 256)
     assert lib.w6a16_matmul(ctypes.byref(wide), None) == _lib.WKV7_ERR_WORKSPACE
     small = base_args(split_k=8, B=2, M=3, workspace=0x10000, workspace_bytes=(1 << 20) + tiles * 8 * 16 * 128 * 4 - 4)
     assert lib.w6a16_matmul(ctypes.byref(small), None) == _lib.WKV7_ERR_WORKSPACE
-    # the in-workgroup split-K kernel (packed layout, split 2..8; or planes once one workgroup per strip and M group
-    # fills the chip) sums its partials in LDS: no workspace
+    # up to 32 rows a split of 2..8 (packed; or planes once the tiles are as many as the CUs): no workspace
     packed = dict(format=_lib.W6A16_FORMAT_PACKED, split_k=8, B=2, M=3)
     assert lib.w6a16_workspace_size(ctypes.byref(base_args(**packed)), ctypes.byref(n)) == 0 and n.value == 0
     assert lib.w6a16_workspace_size(ctypes.byref(base_args(**dict(packed, split_k=16))), ctypes.byref(n)) == 0
@@ -348,8 +347,7 @@ def test_split_rule():
         assert (K // 64) // sk >= 1
     # without a GPU the CU count is taken as 256: K = 4096, N = 16384 has 32 groups of four 128-column strips
     assert lib.w6a16_plan_split(1, 1, 16384, 4096) == 8
-    # M > 32: the wide kernel, one 128-column strip per workgroup; two M groups of eight wavefronts (M = 64, 128) or
-    # four M groups of four (M = 256) put eight wavefronts on every CU without split-K
+    # M > 32: 128 columns by 32 (M = 64) or 64 rows a unit; one unit a CU up to 128 rows, two above, without a split
     assert lib.w6a16_plan_split(1, 64, 16384, 4096) == 1
     assert lib.w6a16_plan_split(1, 128, 16384, 4096) == 1
     assert lib.w6a16_plan_split(1, 256, 16384, 4096) == 1
@@ -358,17 +356,17 @@ def test_split_rule():
     assert lib.w6a16_plan_split(1, 1, 4096, 16384) == 32
     assert I6.plan_int6(1, 4096, 4096, 1) == (lib.w6a16_plan_split(1, 1, 4096, 4096), False)
     assert I6.plan_int6(8, 4096, 4096, 1)[1] is True
-    # M = 32: two M groups x 128 strips = 256 in-workgroup blocks fill the chip, so the deepest split
+    # M = 32: two M groups x 128 strips = 256 tiles, as many as CUs, so the deepest split without a workspace
     assert lib.w6a16_plan_split(1, 32, 16384, 4096) == 8
 
 
 def test_split_rule_packed():
-    """The packed layout takes split 4 instead of 8 where its kernel runs half strips (fewer strips x M groups than
-    CUs) and the ranges keep at least 8 chunks; everywhere else it takes the planes' split."""
+    """The packed layout takes split 4 instead of 8 where strips x M groups are fewer than CUs and the ranges keep at
+    least 8 chunks; everywhere else it takes the planes' split."""
     lib = _lib.load()
     assert lib.w6a16_plan_split_packed(1, 1, 16384, 4096) == 4
     assert lib.w6a16_plan_split_packed(1, 16, 16384, 4096) == 4
-    assert lib.w6a16_plan_split_packed(1, 32, 16384, 4096) == 8      # 256 blocks: whole strips
+    assert lib.w6a16_plan_split_packed(1, 32, 16384, 4096) == 8      # 256 tiles
     assert lib.w6a16_plan_split_packed(1, 1, 16384, 1024) == 8       # 16 chunks: 4 per range at split 4
     for B, M, N, K in [(1, 64, 16384, 4096), (1, 1, 1024, 16384), (4, 1, 2048, 2048), (1, 1, 256, 128)]:
         assert lib.w6a16_plan_split_packed(B, M, N, K) == lib.w6a16_plan_split(B, M, N, K), (B, M, N, K)
